@@ -51,6 +51,27 @@ template <typename R> __device__ __forceinline__ cplx<R> ld_nt(const cplx<R>* p)
     return mk<R>(x.x, x.y);
 }
 
+// Division of n < 2^31 by a fixed d >= 2 as a 32-bit multiply-high and a shift (Granlund and Montgomery's
+// round-up multiplier: m = ceil(2^(31+s) / d) < 2^32 with s = ceil(log2 d) is exact for 31-bit n).  Element-wise
+// kernels decode a mode's three indices with two of these; the 64-bit remainders they replace cost more than
+// the arithmetic of most of those kernels.
+struct FastDiv {
+    unsigned d, m, s;
+};
+static inline FastDiv fast_div(unsigned d)
+{
+    FastDiv f;
+    f.d = d;
+    f.s = 1;
+    while ((1ull << f.s) < d) f.s++;
+    f.m = (unsigned)(((1ull << (31 + f.s)) + d - 1) / d);
+    return f;
+}
+__host__ __device__ __forceinline__ unsigned fdiv(unsigned n, const FastDiv& f)
+{
+    return (unsigned)(((unsigned long long)n * f.m) >> 32) >> (f.s - 1);
+}
+
 // Wavenumber helpers (trunk/lib/four/four_inline.h:88-138, trunk/lib/scft/scft_inline.h:86)
 __host__ __device__ __forceinline__ int kx_four(int l1, int N1) { return (l1 <= N1 / 2) ? l1 : l1 - N1; }
 __host__ __device__ __forceinline__ int ky_of(int l2, int N2) { return (l2 <= N2 / 2) ? l2 : l2 - N2; }

@@ -16,8 +16,16 @@ namespace th {
 struct GeoR {
     int basis, N1, N2, N3, H;
     double f1, f2, f3;
+    FastDiv dH, dN2, dA2;      // by H, N2 and the mirror groups' y extent N2/2 + 1
+    int A2;                    // N2/2 + 1
+    unsigned nq;               // mirror groups (see Quad)
 };
-static GeoR gr(const Geo& g) { return GeoR{g.basis, g.N1, g.N2, g.N3, g.H, g.kf[0], g.kf[1], g.kf[2]}; }
+static GeoR gr(const Geo& g)
+{
+    const unsigned A1 = g.basis == 0 ? g.N1 / 2 + 1 : g.N1, A2 = g.N2 / 2 + 1;
+    return GeoR{g.basis, g.N1, g.N2, g.N3, g.H, g.kf[0], g.kf[1], g.kf[2], fast_div(g.H), fast_div(g.N2), fast_div(A2),
+                (int)A2, A1 * A2 * (unsigned)g.H};
+}
 
 __device__ __forceinline__ double kmag_r(const GeoR& g, int l1, int l2, int l3)
 {
@@ -56,142 +64,213 @@ template <typename R> __device__ __forceinline__ double rdot(const cplx<R>& a, c
     return (double)a.x * b.x + (double)a.y * b.y;
 }
 
+// Index of a mode in three (a plan's arrays hold at most 512 x 512 x 257 < 2^27 modes)
 __device__ __forceinline__ void decode_r(const GeoR& g, long i, int& l1, int& l2, int& l3)
 {
-    l3 = (int)(i % g.H);
-    long r = i / g.H;
-    l2 = (int)(r % g.N2);
-    l1 = (int)(r / g.N2);
+    const unsigned r = fdiv((unsigned)i, g.dH), x = fdiv(r, g.dN2);
+    l3 = (int)((unsigned)i - r * g.dH.d);
+    l2 = (int)(r - x * g.dN2.d);
+    l1 = (int)x;
 }
 
-constexpr int RBLK = 256;
-constexpr int RSEG = 16;      // consecutive modes handled by one thread (run-length accumulation)
+// ------------------------------------------------------------------------------------------
+// Mirror groups.  The modes (+-kx, +-ky, kz) (FOUR; (kx, +-ky, kz) for SCFT) share |K|, the shell index, the
+// multiplicity and every weight of the sums below, so one thread takes the whole group: one square root, one
+// bin and one pair of LDS atomics per four modes, and four independent loads in flight.  Groups are numbered
+// with kz fastest, so the lanes of a wave read consecutive elements of each of the four rows.
+// What bounds them: the field is read once, 128 MiB at 256^3 FP64; before (one mode per step, 64-bit index
+// remainders, the spectra's threads on 16 consecutive modes each) a spectrum took 64 us, an energy 56 us.
+// ------------------------------------------------------------------------------------------
+struct Quad {
+    int a1, a2, l3;           // the group's member with kx, ky >= 0
+    bool m1, m2;              // whether -kx, -ky are other modes (else their indices repeat the member's)
+    unsigned i[4];            // (+,+), (+,-), (-,+), (-,-)
+};
+__device__ __forceinline__ Quad quad_of(const GeoR& g, unsigned j)
+{
+    Quad q;
+    const unsigned r = fdiv(j, g.dH), x = fdiv(r, g.dA2);
+    q.l3 = (int)(j - r * g.dH.d);
+    q.a2 = (int)(r - x * g.dA2.d);
+    q.a1 = (int)x;
+    q.m1 = g.basis == 0 && q.a1 > 0 && q.a1 < g.N1 / 2;
+    q.m2 = q.a2 > 0 && q.a2 < g.N2 / 2;
+    const unsigned b1 = q.m1 ? g.N1 - q.a1 : q.a1, b2 = q.m2 ? g.N2 - q.a2 : q.a2;
+    q.i[0] = (q.a1 * g.N2 + q.a2) * g.H + q.l3;
+    q.i[1] = (q.a1 * g.N2 + b2) * g.H + q.l3;
+    q.i[2] = (b1 * g.N2 + q.a2) * g.H + q.l3;
+    q.i[3] = (b1 * g.N2 + b2) * g.H + q.l3;
+    return q;
+}
+// v0 + v1 + v2 + v3 over the members that exist
+__device__ __forceinline__ double quad_sum(const Quad& q, double v0, double v1, double v2, double v3)
+{
+    return (v0 + (q.m2 ? v1 : 0.0)) + (q.m1 ? v2 + (q.m2 ? v3 : 0.0) : 0.0);
+}
+template <typename R> __device__ __forceinline__ double quad_sq(const Quad& q, const cplx<R>* __restrict__ A)
+{
+    const cplx<R> a = A[q.i[0]], b = A[q.i[1]], c = A[q.i[2]], d = A[q.i[3]];
+    return quad_sum(q, sq(a), sq(b), sq(c), sq(d));
+}
+template <typename R>
+__device__ __forceinline__ double quad_dot(const Quad& q, const cplx<R>* __restrict__ A, const cplx<R>* __restrict__ B)
+{
+    cplx<R> a[4], b[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) { a[k] = A[q.i[k]]; b[k] = B[q.i[k]]; }
+    return quad_sum(q, rdot(a[0], b[0]), rdot(a[1], b[1]), rdot(a[2], b[2]), rdot(a[3], b[3]));
+}
+
+constexpr int RBLK = 256;     // anisotropic and ring kernels
+constexpr int QBLK = 512;     // mirror-group kernels
+constexpr int QMAXB = 1024;   // at most this many blocks: four of 512 threads fill a CU
+
+// Bins of one block: `ncopy` copies, lane l adding to copy l % ncopy (consecutive kz mostly share a shell, and
+// LDS atomics of one wave to one address take a turn each); sums in doubles, mode counts exactly, in quarters.
+// Four copies while they stay within 48 KiB, else one.
+static int bin_copies(int nsum, int ncnt, int nbins)
+{
+    return 4 * (size_t)nbins * (8 * nsum + 4 * ncnt) <= 48 * 1024 ? 4 : 1;
+}
+static size_t bin_lds(int nsum, int ncnt, int nbins) { return (size_t)bin_copies(nsum, ncnt, nbins) * nbins * (8 * nsum + 4 * ncnt); }
 
 // MODE 0: spectrum (bins = ceil(K) <= kkmax; Sk and count), MODE 1: shell_mult_all (bins by radii,
 // K <= kin, value 2*mult*sum_c Re(A_c conj(B_c)))
 template <typename R, int MODE>
-__global__ __launch_bounds__(RBLK) void k_binned(GeoR g, const cplx<R>* __restrict__ A0, const cplx<R>* __restrict__ A1,
+__global__ __launch_bounds__(QBLK) void k_binned(GeoR g, const cplx<R>* __restrict__ A0, const cplx<R>* __restrict__ A1,
                                                  const cplx<R>* __restrict__ A2, const cplx<R>* __restrict__ B0,
                                                  const cplx<R>* __restrict__ B1, const cplx<R>* __restrict__ B2,
                                                  int npow, int kkmax, const double* __restrict__ radii, int nr,
-                                                 int nbins, double* __restrict__ partial)
+                                                 int nbins, int ncopy, double* __restrict__ partial)
 {
     extern __shared__ double sh[];
-    double* sS = sh;
-    double* sC = sh + nbins;
-    for (int b = threadIdx.x; b < 2 * nbins; b += RBLK) sh[b] = 0.0;
+    unsigned* const cn = (unsigned*)(sh + (size_t)ncopy * nbins);
+    for (int b = threadIdx.x; b < ncopy * nbins; b += QBLK) {
+        sh[b] = 0.0;
+        if (MODE == 0) cn[b] = 0;
+    }
     __syncthreads();
-    const long n = (long)g.N1 * g.N2 * g.H;
-    const long nseg = (n + RSEG - 1) / RSEG;
-    for (long s = (long)blockIdx.x * RBLK + threadIdx.x; s < nseg; s += (long)gridDim.x * RBLK) {
-        int cur = -1;
-        double accS = 0.0, accC = 0.0;
-        const long i0 = s * RSEG, i1 = (i0 + RSEG < n) ? i0 + RSEG : n;
-        for (long i = i0; i < i1; i++) {
-            int l1, l2, l3;
-            decode_r(g, i, l1, l2, l3);
-            double km = kmag_r(g, l1, l2, l3);
-            int idx;
-            double val, cnt = 0.0;
-            if (MODE == 0) {
-                idx = (int)ceil(km);
-                if (idx > kkmax) continue;
-                double f = mult_r(g, l1, l2, l3);
-                double v = B0 ? rdot(A0[i], B0[i]) : sq(A0[i]);
-                val = f * my_pow_r(km, npow) * v;
-                cnt = (g.basis == 0) ? f : f / 2;
-            } else {
-                if (km > (double)kkmax) continue;
-                idx = 0;
-                while (idx < nr && !(km <= radii[idx])) idx++;
-                if (idx >= nbins) continue;
-                double f = mult_r(g, l1, l2, l3);
-                double d = rdot(A0[i], B0[i]);
-                if (A1) d += rdot(A1[i], B1[i]);          // null: one-component (scalar) pair
-                if (A2) d += rdot(A2[i], B2[i]);
-                val = 2 * f * d;
-            }
-            if (idx != cur) {
-                if (cur >= 0) {
-                    atomicAdd(&sS[cur], accS);
-                    if (MODE == 0) atomicAdd(&sC[cur], accC);
-                }
-                cur = idx;
-                accS = 0.0;
-                accC = 0.0;
-            }
-            accS += val;
-            accC += cnt;
-        }
-        if (cur >= 0) {
-            atomicAdd(&sS[cur], accS);
-            if (MODE == 0) atomicAdd(&sC[cur], accC);
+    const int cp = ((int)threadIdx.x & (ncopy - 1)) * nbins;
+    for (unsigned j = blockIdx.x * QBLK + threadIdx.x; j < g.nq; j += gridDim.x * QBLK) {
+        const Quad q = quad_of(g, j);
+        const double km = kmag_r(g, q.a1, q.a2, q.l3);
+        int idx;
+        if (MODE == 0) {
+            idx = (int)ceil(km);
+            if (idx > kkmax) continue;
+            const double f = mult_r(g, q.a1, q.a2, q.l3);
+            const double v = B0 ? quad_dot(q, A0, B0) : quad_sq(q, A0);
+            atomicAdd(&sh[cp + idx], f * my_pow_r(km, npow) * v);
+            const int members = (q.m1 ? 2 : 1) * (q.m2 ? 2 : 1);
+            atomicAdd(&cn[cp + idx], (unsigned)(int)(4 * ((g.basis == 0) ? f : f / 2)) * members);
+        } else {
+            if (km > (double)kkmax) continue;
+            idx = 0;
+            while (idx < nr && !(km <= radii[idx])) idx++;
+            if (idx >= nbins) continue;
+            const double f = mult_r(g, q.a1, q.a2, q.l3);
+            double d = quad_dot(q, A0, B0);
+            if (A1) d += quad_dot(q, A1, B1);             // null: one-component (scalar) pair
+            if (A2) d += quad_dot(q, A2, B2);
+            atomicAdd(&sh[cp + idx], 2 * f * d);
         }
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < 2 * nbins; b += RBLK) partial[(long)blockIdx.x * 2 * nbins + b] = sh[b];
+    constexpr int NV = MODE == 0 ? 2 : 1;
+    for (int b = threadIdx.x; b < nbins; b += QBLK) {
+        double s = 0.0;
+        unsigned n = 0;
+        for (int k = 0; k < ncopy; k++) {
+            s += sh[k * nbins + b];
+            if (MODE == 0) n += cn[k * nbins + b];
+        }
+        partial[(long)blockIdx.x * NV * nbins + b] = s;
+        if (MODE == 0) partial[(long)blockIdx.x * NV * nbins + nbins + b] = 0.25 * n;
+    }
 }
 
-// MODE 0: energy weights (Get_local_energy), MODE 1: Sn, MODE 2: shell_mult_single over 3 comps (or 1)
+// Neumaier's compensated s += v
+__device__ __forceinline__ void add_comp(double& s, double& c, double v)
+{
+    const double t = s + v;
+    c += (fabs(s) >= fabs(v)) ? ((s - t) + v) : ((v - t) + s);
+    s = t;
+}
+// partial[block * NV + v] = the block's sum of val[v]
+template <int NV> __device__ __forceinline__ void block_sums(double (&val)[NV], double* __restrict__ partial)
+{
+    __shared__ double red[NV][QBLK];
+#pragma unroll
+    for (int v = 0; v < NV; v++) red[v][threadIdx.x] = val[v];
+    __syncthreads();
+    for (int w = QBLK / 2; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w)
+#pragma unroll
+            for (int v = 0; v < NV; v++) red[v][threadIdx.x] += red[v][threadIdx.x + w];
+        __syncthreads();
+    }
+    if (threadIdx.x < NV) partial[(long)blockIdx.x * NV + threadIdx.x] = red[threadIdx.x][0];
+}
+
+// Get_local_energy's weight of a mode (kx, ky >= 0)
+__device__ __forceinline__ double energy_weight(const GeoR& g, const Quad& q)
+{
+    double w;
+    if (g.basis == 0) {
+        const double e = 1.0 + ((q.a2 == g.N2 / 2 && g.N2 > 1) ? 1.0 : 0.0) + ((q.a1 == g.N1 / 2) ? 1.0 : 0.0);
+        w = q.l3 == 0 ? 0.5 * e : e;
+    } else {
+        w = 2.0 - (q.l3 == 0 ? 1.0 : 0.0) - (q.a1 == 0 ? 1.0 : 0.0) + ((q.a1 == 0 && q.l3 == 0) ? 0.5 : 0.0);
+        if (q.a2 == g.N2 / 2 && g.N2 > 2) w *= 2.0;
+    }
+    if (q.i[0] == 0) w -= 0.5;
+    return w;
+}
+
+// MODE 0: energy weights (Get_local_energy), MODE 1: Sn, MODE 2: shell_mult_single over 3 comps (or 1);
+// MODE 3: the energies of A0, A1, A2, one value each (A1 == nullptr: 0)
 template <typename R, int MODE>
-__global__ __launch_bounds__(RBLK) void k_scalar(GeoR g, const cplx<R>* __restrict__ A0, const cplx<R>* __restrict__ A1,
+__global__ __launch_bounds__(QBLK) void k_scalar(GeoR g, const cplx<R>* __restrict__ A0, const cplx<R>* __restrict__ A1,
                                                  const cplx<R>* __restrict__ A2, const cplx<R>* __restrict__ B0,
                                                  const cplx<R>* __restrict__ B1, const cplx<R>* __restrict__ B2,
                                                  int npow, int kkmax, double inner, double outer,
                                                  double* __restrict__ partial)
 {
-    __shared__ double red[RBLK];
-    double s = 0.0, c = 0.0;                 // Neumaier
-    const long n = (long)g.N1 * g.N2 * g.H;
-    for (long i = (long)blockIdx.x * RBLK + threadIdx.x; i < n; i += (long)gridDim.x * RBLK) {
-        int l1, l2, l3;
-        decode_r(g, i, l1, l2, l3);
-        double v;
-        if (MODE == 0) {
-            double w;
-            if (g.basis == 0) {
-                double ey = (l2 == g.N2 / 2 && g.N2 > 1) ? 1.0 : 0.0;
-                double ex = (l1 == g.N1 / 2) ? 1.0 : 0.0;
-                w = 1.0 + ey + ex;
-                if (l3 == 0) w -= 0.5 * (1.0 + ey + ex);
-            } else {
-                w = 2.0 - (l3 == 0 ? 1.0 : 0.0) - (l1 == 0 ? 1.0 : 0.0) + ((l1 == 0 && l3 == 0) ? 0.5 : 0.0);
-                if (l2 == g.N2 / 2 && g.N2 > 2) w *= 2.0;
+    constexpr int NV = MODE == 3 ? 3 : 1;
+    double s[NV] = {}, c[NV] = {};
+    for (unsigned j = blockIdx.x * QBLK + threadIdx.x; j < g.nq; j += gridDim.x * QBLK) {
+        const Quad q = quad_of(g, j);
+        if (MODE == 0 || MODE == 3) {
+            const double w = energy_weight(g, q);
+            add_comp(s[0], c[0], w * (B0 ? quad_dot(q, A0, B0) : quad_sq(q, A0)));
+            if (MODE == 3 && A1) {
+                add_comp(s[NV > 1 ? 1 : 0], c[NV > 1 ? 1 : 0], w * quad_sq(q, A1));
+                add_comp(s[NV > 2 ? 2 : 0], c[NV > 2 ? 2 : 0], w * quad_sq(q, A2));
             }
-            if (i == 0) w -= 0.5;
-            v = w * (B0 ? rdot(A0[i], B0[i]) : sq(A0[i]));
         } else if (MODE == 1) {
-            double km = kmag_r(g, l1, l2, l3);
+            const double km = kmag_r(g, q.a1, q.a2, q.l3);
             if (!(km <= (double)kkmax)) continue;
-            v = mult_r(g, l1, l2, l3) * my_pow_r(km, npow) * sq(A0[i]);
-            if (i == 0 && npow == 0) v -= mult_r(g, 0, 0, 0) * sq(A0[0]);
+            if (j == 0 && npow == 0) continue;            // the mean mode does not count
+            add_comp(s[0], c[0], mult_r(g, q.a1, q.a2, q.l3) * my_pow_r(km, npow) * quad_sq(q, A0));
         } else {
-            double km = kmag_r(g, l1, l2, l3);
+            const double km = kmag_r(g, q.a1, q.a2, q.l3);
             if (!((km > inner) && (km <= outer))) continue;
-            double d = rdot(A0[i], B0[i]);
-            if (A1) d += rdot(A1[i], B1[i]);              // null: one-component (scalar) pair
-            if (A2) d += rdot(A2[i], B2[i]);
-            v = 2 * mult_r(g, l1, l2, l3) * d;
+            double d = quad_dot(q, A0, B0);
+            if (A1) d += quad_dot(q, A1, B1);             // null: one-component (scalar) pair
+            if (A2) d += quad_dot(q, A2, B2);
+            add_comp(s[0], c[0], 2 * mult_r(g, q.a1, q.a2, q.l3) * d);
         }
-        double t = s + v;
-        c += (fabs(s) >= fabs(v)) ? ((s - t) + v) : ((v - t) + s);
-        s = t;
     }
-    red[threadIdx.x] = s + c;
-    __syncthreads();
-    for (int w = RBLK / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
+#pragma unroll
+    for (int v = 0; v < NV; v++) s[v] += c[v];
+    block_sums<NV>(s, partial);
 }
 
-// out[b] = compensated sum over blocks of partial[blk * stride + b]
 // Helicity and spectral entropy (FOUR basis; the glob.d / spectrum.d columns).
 //   MODE 0: Compute_local_helicity_FOUR four_energy.cc:453-506 over |K| <= kkmax:
 //           modal = 2 mult K.(Vr x Vi); values {sum modal, sum modal/K^2 (K^2 > 1e-15), sum K^2 modal}
 //   MODE 1: Get_local_entropy_FOUR four_energy.cc:687-732: p = (sum_c |V_c|^2 / 2) / E,
-//           value sum 2 mult (-p log2 p) over p > 1e-15
+//           value sum 2 mult (-p log2 p) over p > 1e-15; E[0] + E[1] + E[2] is the energy, already on the device
 // SCFT boxes hold V1 in the sin basis along x; -i V1 is its Fourier counterpart (scft_energy.cc:470-474)
 template <typename R> __device__ __forceinline__ cplx<R> rot_sin(const GeoR& g, const cplx<R>& a)
 {
@@ -205,75 +284,99 @@ template <typename R> __device__ __forceinline__ void vr_x_vi(const cplx<R>& a, 
     x[1] = (double)c.x * a.y - (double)a.x * c.y;
     x[2] = (double)a.x * b.y - (double)b.x * a.y;
 }
+// The group's sums of K_c (Vr x Vi)_c, c = 0..2
+template <typename R>
+__device__ __forceinline__ void quad_hel(const GeoR& g, const Quad& q, const cplx<R>* __restrict__ A0,
+                                         const cplx<R>* __restrict__ A1, const cplx<R>* __restrict__ A2, double (&h)[3])
+{
+    cplx<R> a[4], b[4], c[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) { a[k] = A0[q.i[k]]; b[k] = A1[q.i[k]]; c[k] = A2[q.i[k]]; }
+    const double kx = kx_r(g, q.a1) * g.f1, ky = q.a2 * g.f2, kz = q.l3 * g.f3;
+    double x[4][3];
+#pragma unroll
+    for (int k = 0; k < 4; k++) vr_x_vi(rot_sin(g, a[k]), b[k], c[k], x[k]);
+    h[0] = quad_sum(q, kx * x[0][0], kx * x[1][0], -kx * x[2][0], -kx * x[3][0]);
+    h[1] = quad_sum(q, ky * x[0][1], -ky * x[1][1], ky * x[2][1], -ky * x[3][1]);
+    h[2] = quad_sum(q, kz * x[0][2], kz * x[1][2], kz * x[2][2], kz * x[3][2]);
+}
 template <typename R, int MODE>
-__global__ __launch_bounds__(RBLK) void k_modal(GeoR g, const cplx<R>* __restrict__ A0, const cplx<R>* __restrict__ A1,
-                                                const cplx<R>* __restrict__ A2, int kkmax, double E,
+__global__ __launch_bounds__(QBLK) void k_modal(GeoR g, const cplx<R>* __restrict__ A0, const cplx<R>* __restrict__ A1,
+                                                const cplx<R>* __restrict__ A2, int kkmax, const double* __restrict__ E3,
                                                 double* __restrict__ partial)
 {
     constexpr int NV = MODE == 0 ? 3 : 1;
-    __shared__ double red[NV][RBLK];
     double acc[NV] = {};
-    const long n = (long)g.N1 * g.N2 * g.H;
-    for (long i = (long)blockIdx.x * RBLK + threadIdx.x; i < n; i += (long)gridDim.x * RBLK) {
-        int l1, l2, l3;
-        decode_r(g, i, l1, l2, l3);
+    const double E = MODE == 1 ? E3[0] + E3[1] + E3[2] : 0.0;
+    for (unsigned j = blockIdx.x * QBLK + threadIdx.x; j < g.nq; j += gridDim.x * QBLK) {
+        const Quad q = quad_of(g, j);
         if (MODE == 0) {
-            double km = kmag_r(g, l1, l2, l3);
+            const double km = kmag_r(g, q.a1, q.a2, q.l3);
             if (km > (double)kkmax) continue;
-            double x[3];
-            vr_x_vi(rot_sin(g, A0[i]), A1[i], A2[i], x);
-            const double kx = kx_r(g, l1) * g.f1, ky = ky_of(l2, g.N2) * g.f2, kz = l3 * g.f3;
+            double h[3];
+            quad_hel(g, q, A0, A1, A2, h);
             const double ksq = km * km;
-            const double modal = 2 * mult_r(g, l1, l2, l3) * (kx * x[0] + ky * x[1] + kz * x[2]);
+            const double modal = 2 * mult_r(g, q.a1, q.a2, q.l3) * (h[0] + h[1] + h[2]);
             acc[0] += modal;
             if (ksq > 1e-15) acc[NV > 1 ? 1 : 0] += modal / ksq;
             acc[NV > 2 ? 2 : 0] += ksq * modal;
         } else {
             // Modal_energy_SCFT (scft_inline.h:347-354) is |A|^2 for kx > 0; SCFT weighs by mult, FOUR by 2 mult
-            const double v2 = sq(A0[i]) + (A1 ? sq(A1[i]) + sq(A2[i]) : 0.0);     // A1 == nullptr: one field
-            const double me = 0.5 * v2 * ((g.basis == 1 && l1 > 0) ? 2.0 : 1.0);
-            const double p = me / E;
-            if (p > 1e-15) acc[0] += (g.basis == 1 ? 1.0 : 2.0) * mult_r(g, l1, l2, l3) * (-p * log(p) / log(2.0));
+            double v2[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                v2[k] = sq(A0[q.i[k]]) + (A1 ? sq(A1[q.i[k]]) + sq(A2[q.i[k]]) : 0.0);   // A1 == nullptr: one field
+            const double half = 0.5 * ((g.basis == 1 && q.a1 > 0) ? 2.0 : 1.0);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const double p = half * v2[k] / E;
+                v2[k] = p > 1e-15 ? -p * log(p) / log(2.0) : 0.0;
+            }
+            acc[0] += (g.basis == 1 ? 1.0 : 2.0) * mult_r(g, q.a1, q.a2, q.l3) * quad_sum(q, v2[0], v2[1], v2[2], v2[3]);
         }
     }
-#pragma unroll
-    for (int v = 0; v < NV; v++) red[v][threadIdx.x] = acc[v];
-    __syncthreads();
-    for (int w = RBLK / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w)
-#pragma unroll
-            for (int v = 0; v < NV; v++) red[v][threadIdx.x] += red[v][threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x < NV) partial[(long)blockIdx.x * NV + threadIdx.x] = red[threadIdx.x][0];
+    block_sums<NV>(acc, partial);
 }
 
 // Compute_local_shell_spectrum_helicity_FOUR four_energy.cc:551-599 (_SCFT scft_energy.cc:546-599): bin ceil(K) <= kkmax,
 // H1k_c += 2 mult K_c (Vr x Vi)_c and count += 2 mult; partial[block][4 nbins]
 template <typename R>
-__global__ __launch_bounds__(RBLK) void k_binned_hel(GeoR g, const cplx<R>* __restrict__ A0, const cplx<R>* __restrict__ A1,
-                                                     const cplx<R>* __restrict__ A2, int kkmax, int nbins,
+__global__ __launch_bounds__(QBLK) void k_binned_hel(GeoR g, const cplx<R>* __restrict__ A0, const cplx<R>* __restrict__ A1,
+                                                     const cplx<R>* __restrict__ A2, int kkmax, int nbins, int ncopy,
                                                      double* __restrict__ partial)
 {
     extern __shared__ double sh[];
-    for (int b = threadIdx.x; b < 4 * nbins; b += RBLK) sh[b] = 0.0;
-    __syncthreads();
-    const long n = (long)g.N1 * g.N2 * g.H;
-    for (long i = (long)blockIdx.x * RBLK + threadIdx.x; i < n; i += (long)gridDim.x * RBLK) {
-        int l1, l2, l3;
-        decode_r(g, i, l1, l2, l3);
-        const int idx = (int)ceil(kmag_r(g, l1, l2, l3));
-        if (idx > kkmax || idx >= nbins) continue;
-        double x[3];
-        vr_x_vi(rot_sin(g, A0[i]), A1[i], A2[i], x);
-        const double f = 2 * mult_r(g, l1, l2, l3);
-        atomicAdd(&sh[idx], f * (kx_r(g, l1) * g.f1 * x[0]));
-        atomicAdd(&sh[nbins + idx], f * (ky_of(l2, g.N2) * g.f2 * x[1]));
-        atomicAdd(&sh[2 * nbins + idx], f * (l3 * g.f3 * x[2]));
-        atomicAdd(&sh[3 * nbins + idx], g.basis == 1 ? f / 2 : f);      // SCFT counts factor/2
+    unsigned* const cn = (unsigned*)(sh + (size_t)3 * ncopy * nbins);
+    for (int b = threadIdx.x; b < ncopy * nbins; b += QBLK) {
+        sh[b] = sh[ncopy * nbins + b] = sh[2 * ncopy * nbins + b] = 0.0;
+        cn[b] = 0;
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < 4 * nbins; b += RBLK) partial[(long)blockIdx.x * 4 * nbins + b] = sh[b];
+    const int cp = ((int)threadIdx.x & (ncopy - 1)) * nbins;
+    for (unsigned j = blockIdx.x * QBLK + threadIdx.x; j < g.nq; j += gridDim.x * QBLK) {
+        const Quad q = quad_of(g, j);
+        const int idx = (int)ceil(kmag_r(g, q.a1, q.a2, q.l3));
+        if (idx > kkmax || idx >= nbins) continue;
+        double h[3];
+        quad_hel(g, q, A0, A1, A2, h);
+        const double f = 2 * mult_r(g, q.a1, q.a2, q.l3);
+#pragma unroll
+        for (int c = 0; c < 3; c++) atomicAdd(&sh[c * ncopy * nbins + cp + idx], f * h[c]);
+        const int members = (q.m1 ? 2 : 1) * (q.m2 ? 2 : 1);
+        atomicAdd(&cn[cp + idx], (unsigned)(int)(4 * (g.basis == 1 ? f / 2 : f)) * members);   // SCFT counts factor/2
+    }
+    __syncthreads();
+    for (int b = threadIdx.x; b < nbins; b += QBLK) {
+        double* out = partial + (long)blockIdx.x * 4 * nbins + b;
+        unsigned n = 0;
+        for (int c = 0; c < 3; c++) {
+            double s = 0.0;
+            for (int k = 0; k < ncopy; k++) s += sh[(c * ncopy + k) * nbins + b];
+            out[c * nbins] = s;
+        }
+        for (int k = 0; k < ncopy; k++) n += cn[k * nbins + b];
+        out[3 * nbins] = 0.25 * n;
+    }
 }
 
 // Anisotropic spectra (FOUR, 3-D) about axis a = globalvar_anisotropy_switch (1, 2, 3), bins
@@ -499,8 +602,12 @@ __global__ __launch_bounds__(RBLK) void k_ring_mult(GeoR g, const cplx<R>* __res
     for (int b = threadIdx.x; b < nb; b += RBLK) partial[(long)blockIdx.x * nb + b] = sh[b];
 }
 
+// At least 8 MB and 4096 host values from the first call on: growing step by step through the calls of one output
+// line (energy, spectrum, helicity, ...) costs a device and a pinned allocation each.
 int RedScratch::ensure(size_t n_dev, size_t n_host)
 {
+    if (n_dev < (1u << 20)) n_dev = 1u << 20;
+    if (n_host < 4096) n_host = 4096;
     if (n_dev > cap) {
         if (d) (void)hipFree(d);
         d = nullptr;
@@ -524,11 +631,27 @@ void RedScratch::release()
     cap = hcap = 0;
 }
 
+// blocks of the anisotropic and ring kernels (64 modes per thread: each block writes its whole bin table)
 static int nblocks_for(size_t n)
 {
-    size_t b = (n + RBLK * RSEG - 1) / (RBLK * RSEG);
+    size_t b = (n / 4 + RBLK * 16) / (RBLK * 16);
     if (b > 1024) b = 1024;
     return (int)(b ? b : 1);
+}
+// blocks of the mirror-group kernels
+static int nblocks_q(const GeoR& g)
+{
+    const unsigned b = (g.nq + QBLK - 1) / QBLK;
+    return (int)(b > (unsigned)QMAXB ? QMAXB : b);
+}
+// Sums finalized straight into the pinned host buffer: the store of a few values over the host link overlaps the
+// stream synchronisation that the caller waits for anyway (a separate device-to-host copy costs its own launch).
+static int finalize_to_host(const double* partial, int nblk, int nval, RedScratch& rs, hipStream_t st)
+{
+    launch_finalize(partial, nblk, nval, nval, rs.h, st);
+    TH_CHECK_HIP(hipGetLastError());
+    TH_CHECK_HIP(hipStreamSynchronize(st));
+    return OK;
 }
 
 int ring_params(const Geo& g, int cyl, int axis, const double* radii, int nr, const double* edges, int nsec, RingP* rp)
@@ -554,7 +677,7 @@ int ring_params(const Geo& g, int cyl, int axis, const double* radii, int nr, co
 template <typename R>
 int fill_ring(const Geo& g, const cplx<R>* F, cplx<R>* G, const RingP& rp, int gs, int gq, hipStream_t st)
 {
-    const int nblk = nblocks_for(g.ncplx() / 4 + 1);
+    const int nblk = nblocks_for(g.ncplx());
     hipLaunchKernelGGL((k_fill_ring<R>), dim3(nblk), dim3(RBLK), 0, st, gr(g), F, G, rp, rp.r[gs - 1], rp.r[gs],
                        rp.e[gq - 1], rp.e[gq]);
     TH_CHECK_HIP(hipGetLastError());
@@ -566,10 +689,9 @@ int reduce_ring_mult(const Geo& g, const cplx<R>* const A[3], const cplx<R>* con
                      RedScratch& rs, hipStream_t st)
 {
     const int nb = (rp.nr + 1) * (rp.nsec + 1);
-    const int nblk = nblocks_for(g.ncplx() / 4 + 1);
-    int r = rs.ensure((size_t)nblk * nb + nb, nb);
+    const int nblk = nblocks_for(g.ncplx());
+    int r = rs.ensure((size_t)nblk * nb, nb);
     if (r) return r;
-    double* dout = rs.d + (size_t)nblk * nb;
     const size_t lds = nb * sizeof(double);
     if (rp.cyl)
         hipLaunchKernelGGL((k_ring_mult<R, true>), dim3(nblk), dim3(RBLK), lds, st, gr(g), A[0], A[1], A[2], B[0], B[1],
@@ -578,10 +700,7 @@ int reduce_ring_mult(const Geo& g, const cplx<R>* const A[3], const cplx<R>* con
         hipLaunchKernelGGL((k_ring_mult<R, false>), dim3(nblk), dim3(RBLK), lds, st, gr(g), A[0], A[1], A[2], B[0], B[1],
                            B[2], rp, rs.d);
     TH_CHECK_HIP(hipGetLastError());
-    launch_finalize(rs.d, nblk, nb, nb, dout, st);
-    TH_CHECK_HIP(hipGetLastError());
-    TH_CHECK_HIP(hipMemcpyAsync(rs.h, dout, nb * sizeof(double), hipMemcpyDeviceToHost, st));
-    TH_CHECK_HIP(hipStreamSynchronize(st));
+    TRY(finalize_to_host(rs.d, nblk, nb, rs, st));
     for (int k = 0; k < nb; k++) out[k] = rs.h[k];
     return OK;
 }
@@ -623,20 +742,17 @@ template <typename R>
 int reduce_shell(const Geo& g, const cplx<R>* A, const cplx<R>* B, double n, int nbins, double* Sk, double* cnt,
                  RedScratch& rs, hipStream_t st, bool rescale)
 {
-    int nb = nblocks_for(g.ncplx());
+    const GeoR gq = gr(g);
+    int nb = nblocks_q(gq);
     int kkmax = min_radius_outside(g);
     if (nbins != kkmax + 1) { set_error("reduce_shell: nbins %d != shell_ek_size %d", nbins, kkmax + 1); return E_ARG; }
-    int r = rs.ensure((size_t)nb * 2 * nbins + 2 * nbins, 2 * nbins);
+    int r = rs.ensure((size_t)nb * 2 * nbins, 2 * nbins);
     if (r) return r;
-    double* out = rs.d + (size_t)nb * 2 * nbins;
-    hipLaunchKernelGGL((k_binned<R, 0>), dim3(nb), dim3(RBLK), 2 * nbins * sizeof(double), st, gr(g), A,
-                       (const cplx<R>*)nullptr, (const cplx<R>*)nullptr, B, (const cplx<R>*)nullptr,
-                       (const cplx<R>*)nullptr, (int)n, kkmax, (const double*)nullptr, 0, nbins, rs.d);
+    hipLaunchKernelGGL((k_binned<R, 0>), dim3(nb), dim3(QBLK), bin_lds(1, 1, nbins), st, gq, A, (const cplx<R>*)nullptr,
+                       (const cplx<R>*)nullptr, B, (const cplx<R>*)nullptr, (const cplx<R>*)nullptr, (int)n, kkmax,
+                       (const double*)nullptr, 0, nbins, bin_copies(1, 1, nbins), rs.d);
     TH_CHECK_HIP(hipGetLastError());
-    launch_finalize(rs.d, nb, 2 * nbins, 2 * nbins, out, st);
-    TH_CHECK_HIP(hipGetLastError());
-    TH_CHECK_HIP(hipMemcpyAsync(rs.h, out, 2 * nbins * sizeof(double), hipMemcpyDeviceToHost, st));
-    TH_CHECK_HIP(hipStreamSynchronize(st));
+    TRY(finalize_to_host(rs.d, nb, 2 * nbins, rs, st));
     int kin = max_radius_inside(g);
     for (int k = 0; k < nbins; k++) {
         double s = rs.h[k], c = rs.h[nbins + k];
@@ -648,13 +764,13 @@ int reduce_shell(const Geo& g, const cplx<R>* A, const cplx<R>* B, double n, int
 }
 
 // ---- th_shell_spectrum_noalloc: the shell spectrum with no device or host allocation ----
-// Its per-block partials (nblocks_for(n) <= 1024 blocks x 2 NOALLOC_BINS values) and finalized sums and
+// Its per-block partials (at most QMAXB blocks x 2 NOALLOC_BINS values) and finalized sums and
 // counts (2 NOALLOC_BINS values) live in this file-scope array, one copy per device for the life of the
 // process (8.4 MB).  Host code never passes the array's name to a kernel: each device's own address comes
 // from hipGetSymbolAddress, looked up once per device with that device current.  Calls that overlap on one
 // device share the array and race.
 constexpr int NOALLOC_BINS = 512;
-constexpr size_t NOALLOC_DOUBLES = (size_t)1024 * 2 * NOALLOC_BINS + 2 * NOALLOC_BINS;
+constexpr size_t NOALLOC_DOUBLES = (size_t)QMAXB * 2 * NOALLOC_BINS + 2 * NOALLOC_BINS;
 static __device__ __align__(256) double scratch[NOALLOC_DOUBLES];
 constexpr int NOALLOC_MAX_DEVICES = 64;
 static std::mutex g_scratch_mu;
@@ -698,7 +814,8 @@ template <typename R>
 int reduce_shell_noalloc(const Geo& g, const cplx<R>* A, const cplx<R>* B, double n, int nbins, double* Sk, double* cnt,
                          hipStream_t st)
 {
-    int nb = nblocks_for(g.ncplx());
+    const GeoR gq = gr(g);
+    int nb = nblocks_q(gq);
     int kkmax = min_radius_outside(g);
     if (nbins != kkmax + 1) { set_error("reduce_shell_noalloc: nbins %d != shell_ek_size %d", nbins, kkmax + 1); return E_ARG; }
     if (nbins > NOALLOC_BINS || (size_t)nb * 2 * nbins + 2 * nbins > NOALLOC_DOUBLES) {
@@ -711,9 +828,9 @@ int reduce_shell_noalloc(const Geo& g, const cplx<R>* A, const cplx<R>* B, doubl
     double* out = scr + (size_t)nb * 2 * nbins;
     // every block writes all 2 nbins of its partial row, and the finalize writes all of `out`: nothing here
     // reads what an earlier call left in the array
-    hipLaunchKernelGGL((k_binned<R, 0>), dim3(nb), dim3(RBLK), 2 * nbins * sizeof(double), st, gr(g), A,
-                       (const cplx<R>*)nullptr, (const cplx<R>*)nullptr, B, (const cplx<R>*)nullptr,
-                       (const cplx<R>*)nullptr, (int)n, kkmax, (const double*)nullptr, 0, nbins, scr);
+    hipLaunchKernelGGL((k_binned<R, 0>), dim3(nb), dim3(QBLK), bin_lds(1, 1, nbins), st, gq, A, (const cplx<R>*)nullptr,
+                       (const cplx<R>*)nullptr, B, (const cplx<R>*)nullptr, (const cplx<R>*)nullptr, (int)n, kkmax,
+                       (const double*)nullptr, 0, nbins, bin_copies(1, 1, nbins), scr);
     TH_CHECK_HIP(hipGetLastError());
     launch_finalize(scr, nb, 2 * nbins, 2 * nbins, out, st);
     TH_CHECK_HIP(hipGetLastError());
@@ -730,22 +847,20 @@ template <typename R>
 static int run_scalar(int mode, const Geo& g, const cplx<R>* const A[3], const cplx<R>* const B[3], int npow,
                       double inner, double outer, double* out, RedScratch& rs, hipStream_t st)
 {
-    int nb = nblocks_for(g.ncplx() / 4 + 1);
-    int r = rs.ensure((size_t)nb + 1, 1);
+    const GeoR gq = gr(g);
+    const int nb = nblocks_q(gq);
+    int r = rs.ensure((size_t)nb, 1);
     if (r) return r;
     int kkmax = min_radius_outside(g);
     auto launch = [&](auto kern) {
-        hipLaunchKernelGGL(kern, dim3(nb), dim3(RBLK), 0, st, gr(g), A[0], A[1], A[2], B[0], B[1], B[2], npow, kkmax,
-                           inner, outer, rs.d);
+        hipLaunchKernelGGL(kern, dim3(nb), dim3(QBLK), 0, st, gq, A[0], A[1], A[2], B[0], B[1], B[2], npow, kkmax, inner,
+                           outer, rs.d);
     };
     if (mode == 0) launch(k_scalar<R, 0>);
     else if (mode == 1) launch(k_scalar<R, 1>);
     else launch(k_scalar<R, 2>);
     TH_CHECK_HIP(hipGetLastError());
-    launch_finalize(rs.d, nb, 1, 1, rs.d + nb, st);
-    TH_CHECK_HIP(hipGetLastError());
-    TH_CHECK_HIP(hipMemcpyAsync(rs.h, rs.d + nb, sizeof(double), hipMemcpyDeviceToHost, st));
-    TH_CHECK_HIP(hipStreamSynchronize(st));
+    TRY(finalize_to_host(rs.d, nb, 1, rs, st));
     *out = rs.h[0];
     return OK;
 }
@@ -775,40 +890,44 @@ template <typename R>
 int reduce_shell_mult_all(const Geo& g, const cplx<R>* const A[3], const cplx<R>* const B[3], const double* radii_dev,
                           int nr, double* out, RedScratch& rs, hipStream_t st)
 {
-    int nb = nblocks_for(g.ncplx());
+    const GeoR gq = gr(g);
+    int nb = nblocks_q(gq);
     int nbins = nr;
-    int r = rs.ensure((size_t)nb * 2 * nbins + 2 * nbins, 2 * nbins);
+    int r = rs.ensure((size_t)nb * nbins, nbins);
     if (r) return r;
-    double* dout = rs.d + (size_t)nb * 2 * nbins;
     int kin = max_radius_inside(g);
-    hipLaunchKernelGGL((k_binned<R, 1>), dim3(nb), dim3(RBLK), 2 * nbins * sizeof(double), st, gr(g), A[0], A[1], A[2],
-                       B[0], B[1], B[2], 0, kin, radii_dev, nr, nbins, rs.d);
+    hipLaunchKernelGGL((k_binned<R, 1>), dim3(nb), dim3(QBLK), bin_lds(1, 0, nbins), st, gq, A[0], A[1], A[2], B[0], B[1],
+                       B[2], 0, kin, radii_dev, nr, nbins, bin_copies(1, 0, nbins), rs.d);
     TH_CHECK_HIP(hipGetLastError());
-    launch_finalize(rs.d, nb, 2 * nbins, nbins, dout, st);
-    TH_CHECK_HIP(hipGetLastError());
-    TH_CHECK_HIP(hipMemcpyAsync(rs.h, dout, nbins * sizeof(double), hipMemcpyDeviceToHost, st));
-    TH_CHECK_HIP(hipStreamSynchronize(st));
+    TRY(finalize_to_host(rs.d, nb, nbins, rs, st));
     for (int k = 0; k < nbins; k++) out[k] = rs.h[k];
     return OK;
 }
 
-template <typename R> static int run_modal(int mode, const Geo& g, const cplx<R>* const V[3], double E, double* out,
-                                           RedScratch& rs, hipStream_t st)
+// mode 0: the three helicity sums; mode 1: the entropy of V (V[1] == nullptr: of one field) against its own
+// energy, which a launch before leaves on the device
+template <typename R> static int run_modal(int mode, const Geo& g, const cplx<R>* const V[3], double* out, RedScratch& rs,
+                                           hipStream_t st)
 {
-    const int nv = mode == 0 ? 3 : 1;
-    int nb = nblocks_for(g.ncplx() / 4 + 1);
-    int r = rs.ensure((size_t)nb * nv + nv, nv);
+    const GeoR gq = gr(g);
+    const int nb = nblocks_q(gq), nv = mode == 0 ? 3 : 1;
+    int r = rs.ensure((size_t)nb * 3 + 3, 3);
     if (r) return r;
     int kkmax = min_radius_outside(g);
-    if (mode == 0)
-        hipLaunchKernelGGL((k_modal<R, 0>), dim3(nb), dim3(RBLK), 0, st, gr(g), V[0], V[1], V[2], kkmax, E, rs.d);
-    else
-        hipLaunchKernelGGL((k_modal<R, 1>), dim3(nb), dim3(RBLK), 0, st, gr(g), V[0], V[1], V[2], kkmax, E, rs.d);
+    double* E3 = rs.d + (size_t)nb * 3;
+    if (mode == 0) {
+        hipLaunchKernelGGL((k_modal<R, 0>), dim3(nb), dim3(QBLK), 0, st, gq, V[0], V[1], V[2], kkmax, (const double*)E3, rs.d);
+    } else {
+        const cplx<R>* none = nullptr;
+        hipLaunchKernelGGL((k_scalar<R, 3>), dim3(nb), dim3(QBLK), 0, st, gq, V[0], V[1], V[2], none, none, none, 0, kkmax,
+                           0.0, 0.0, rs.d);
+        TH_CHECK_HIP(hipGetLastError());
+        launch_finalize(rs.d, nb, 3, 3, E3, st);
+        TH_CHECK_HIP(hipGetLastError());
+        hipLaunchKernelGGL((k_modal<R, 1>), dim3(nb), dim3(QBLK), 0, st, gq, V[0], V[1], V[2], kkmax, (const double*)E3, rs.d);
+    }
     TH_CHECK_HIP(hipGetLastError());
-    launch_finalize(rs.d, nb, nv, nv, rs.d + (size_t)nb * nv, st);
-    TH_CHECK_HIP(hipGetLastError());
-    TH_CHECK_HIP(hipMemcpyAsync(rs.h, rs.d + (size_t)nb * nv, nv * sizeof(double), hipMemcpyDeviceToHost, st));
-    TH_CHECK_HIP(hipStreamSynchronize(st));
+    TRY(finalize_to_host(rs.d, nb, nv, rs, st));
     for (int v = 0; v < nv; v++) out[v] = rs.h[v];
     return OK;
 }
@@ -817,7 +936,7 @@ template <typename R> static int run_modal(int mode, const Geo& g, const cplx<R>
 template <typename R> int reduce_helicity(const Geo& g, const cplx<R>* const V[3], double* out, RedScratch& rs, hipStream_t st)
 {
     double v[3];
-    TRY(run_modal<R>(0, g, V, 0.0, v, rs, st));
+    TRY(run_modal<R>(0, g, V, v, rs, st));
     out[0] = v[0];
     out[1] = v[1];
     out[2] = 2.0 * v[2];
@@ -828,21 +947,14 @@ template <typename R> int reduce_helicity(const Geo& g, const cplx<R>* const V[3
 // Get_entropy_FOUR / _SCFT with E = the three components' Get_total_energy
 template <typename R> int reduce_entropy(const Geo& g, const cplx<R>* const V[3], double* out, RedScratch& rs, hipStream_t st)
 {
-    double E = 0, e;
-    for (int c = 0; c < 3; c++) {
-        TRY(reduce_energy<R>(g, V[c], nullptr, &e, rs, st));
-        E += e;
-    }
-    return run_modal<R>(1, g, V, E, out, rs, st);
+    return run_modal<R>(1, g, V, out, rs, st);
 }
 
 // Get_entropy_scalar_FOUR four_energy.cc:761-826 / _SCFT scft_energy.cc:750-800: one field
 template <typename R> int reduce_entropy_scalar(const Geo& g, const cplx<R>* A, double* out, RedScratch& rs, hipStream_t st)
 {
-    double E;
-    TRY(reduce_energy<R>(g, A, nullptr, &E, rs, st));
     const cplx<R>* V[3] = {A, nullptr, nullptr};
-    return run_modal<R>(1, g, V, E, out, rs, st);
+    return run_modal<R>(1, g, V, out, rs, st);
 }
 
 // Compute_shell_spectrum_helicity_FOUR four_energy.cc:602-671 / _SCFT scft_energy.cc:601-677 (with the
@@ -851,19 +963,16 @@ template <typename R>
 int reduce_shell_helicity(const Geo& g, const cplx<R>* const V[3], int nbins, double* H1, double* H2, double* H3,
                           RedScratch& rs, hipStream_t st)
 {
-    int nb = nblocks_for(g.ncplx() / 4 + 1);
+    const GeoR gq = gr(g);
+    int nb = nblocks_q(gq);
     int kkmax = min_radius_outside(g);
     if (nbins != kkmax + 1) { set_error("reduce_shell_helicity: nbins %d != shell_ek_size %d", nbins, kkmax + 1); return E_ARG; }
-    int r = rs.ensure((size_t)nb * 4 * nbins + 4 * nbins, 4 * nbins);
+    int r = rs.ensure((size_t)nb * 4 * nbins, 4 * nbins);
     if (r) return r;
-    double* out = rs.d + (size_t)nb * 4 * nbins;
-    hipLaunchKernelGGL((k_binned_hel<R>), dim3(nb), dim3(RBLK), 4 * nbins * sizeof(double), st, gr(g), V[0], V[1], V[2],
-                       kkmax, nbins, rs.d);
+    hipLaunchKernelGGL((k_binned_hel<R>), dim3(nb), dim3(QBLK), bin_lds(3, 1, nbins), st, gq, V[0], V[1], V[2], kkmax, nbins,
+                       bin_copies(3, 1, nbins), rs.d);
     TH_CHECK_HIP(hipGetLastError());
-    launch_finalize(rs.d, nb, 4 * nbins, 4 * nbins, out, st);
-    TH_CHECK_HIP(hipGetLastError());
-    TH_CHECK_HIP(hipMemcpyAsync(rs.h, out, 4 * nbins * sizeof(double), hipMemcpyDeviceToHost, st));
-    TH_CHECK_HIP(hipStreamSynchronize(st));
+    TRY(finalize_to_host(rs.d, nb, 4 * nbins, rs, st));
     int kin = max_radius_inside(g);
     for (int k = 0; k < nbins; k++) {
         double c = rs.h[3 * nbins + k], s = 1.0;
@@ -920,10 +1029,9 @@ int reduce_aniso(const Geo& g, const cplx<R>* const V[3], int mode, int nbin, in
         set_error("anisotropic spectra: %d x %d bins exceed one workgroup's 64 KiB of LDS", ap.rows, ap.cols);
         return E_ARG;
     }
-    const int nblk = nblocks_for(g.ncplx() / 4 + 1);
-    int r = rs.ensure((size_t)nblk * nb2 + nb2, nb2);
+    const int nblk = nblocks_for(g.ncplx());
+    int r = rs.ensure((size_t)nblk * nb2, nb2);
     if (r) return r;
-    double* out = rs.d + (size_t)nblk * nb2;
     const size_t lds = nb2 * sizeof(double);
     if (mode == 0 && !hel)
         hipLaunchKernelGGL((k_aniso<R, 0, false>), dim3(nblk), dim3(RBLK), lds, st, gr(g), V[0], V[1], V[2], ap, rs.d);
@@ -934,10 +1042,7 @@ int reduce_aniso(const Geo& g, const cplx<R>* const V[3], int mode, int nbin, in
     else
         hipLaunchKernelGGL((k_aniso<R, 1, true>), dim3(nblk), dim3(RBLK), lds, st, gr(g), V[0], V[1], V[2], ap, rs.d);
     TH_CHECK_HIP(hipGetLastError());
-    launch_finalize(rs.d, nblk, nb2, nb2, out, st);
-    TH_CHECK_HIP(hipGetLastError());
-    TH_CHECK_HIP(hipMemcpyAsync(rs.h, out, nb2 * sizeof(double), hipMemcpyDeviceToHost, st));
-    TH_CHECK_HIP(hipStreamSynchronize(st));
+    TRY(finalize_to_host(rs.d, nblk, nb2, rs, st));
     const int nb = ap.rows * ap.cols;
     for (int k = 0; k < nb; k++) {
         S1[k] = rs.h[k];
