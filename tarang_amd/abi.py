@@ -343,6 +343,11 @@ class Plan:
             return torch.zeros(self.shape, dtype=self.dtype, device=dev)
         return [torch.zeros(self.shape, dtype=self.dtype, device=dev) for _ in range(n)]
 
+    def _uninit(self, n):
+        """n arrays for a call that writes every element of them."""
+        torch = _torch()
+        return [torch.empty(self.shape, dtype=self.dtype, device=f"cuda:{self.ctx.device}") for _ in range(n)]
+
     def to_dev(self, arr):
         torch = _torch()
         t = torch.from_numpy(arr).to(device=f"cuda:{self.ctx.device}", dtype=self.dtype).contiguous()
@@ -394,7 +399,7 @@ class Plan:
         return A
 
     def nlin_ns(self, V):
-        N = self.empty(3)
+        N = self._uninit(3)
         self._pre()
         self._post(lib().th_nlin_ns(self.h, _pp(V), _pp(N)), "th_nlin_ns")
         return N
@@ -745,7 +750,7 @@ class State:
         self.plan._post(0, "")
 
     def download(self):
-        out = self.plan.empty(self.ncomp)
+        out = self.plan._uninit(self.ncomp)
         self.plan._pre()
         for c, f in enumerate(out):
             _check(lib().th_state_download(self.h, c, _ptr(f), 0), "th_state_download")
@@ -754,7 +759,7 @@ class State:
 
     def download_buffer(self, which):
         """Diagnostics: 1 = RK stage field, 2 = RK4 accumulator (reference layout)."""
-        out = self.plan.empty(self.ncomp)
+        out = self.plan._uninit(self.ncomp)
         self.plan._pre()
         for c, f in enumerate(out):
             _check(lib().th_state_download_buffer(self.h, which, c, _ptr(f), 0), "th_state_download_buffer")
@@ -869,7 +874,7 @@ class Ensemble:
 
     def download(self, box):
         p = self.plan(box)
-        out = p.empty(3)
+        out = p._uninit(3)
         p._pre()
         for c, f in enumerate(out):
             _check(lib().th_ensemble_download(self.h, box, c, _ptr(f), 0), "th_ensemble_download")

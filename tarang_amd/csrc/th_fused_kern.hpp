@@ -1060,32 +1060,30 @@ __global__ __launch_bounds__(T * P) void k_fx_fwd_et(FG g, const cplx<R>* __rest
     for (int b = threadIdx.x; b < 2 * nr; b += T * P) partial[(long)blockIdx.x * (2 * nr) + b] = bins[b];
 }
 
-// compact <-> reference layout
+// compact <-> reference layout.  Both are bound by memory (a download writes the whole reference array, non-temporally:
+// at the sizes that matter it exceeds the last-level cache); indices come from 32-bit divisions.
 template <typename R>
-__global__ void k_gather(FG g, const cplx<R>* __restrict__ ref, cplx<R>* __restrict__ S)
+__global__ void k_gather(FG g, FastDiv dz, FastDiv dy, const cplx<R>* __restrict__ ref, cplx<R>* __restrict__ S)
 {
-    long n = (long)g.mx.nk * g.sx;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        int cz = (int)(i % g.KZP);
-        long r = i / g.KZP;
-        int cy = (int)(r % g.my.nk), cx = (int)(r / g.my.nk);
+    const unsigned n = (unsigned)(g.mx.nk * g.sx);
+    const int H = g.N3 / 2 + 1;
+    for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const unsigned r = fdiv(i, dz), cx = fdiv(r, dy);
+        const int cz = (int)(i - r * dz.d), cy = (int)(r - cx * dy.d);
         if (cz >= g.nkz) { S[i] = czero<R>(); continue; }
-        int l1 = ll(g.mx, cx), l2 = ll(g.my, cy);
-        S[i] = ref[((long)l1 * g.N2 + l2) * (g.N3 / 2 + 1) + cz];
+        S[i] = ref[((long)ll(g.mx, cx) * g.N2 + ll(g.my, cy)) * H + cz];
     }
 }
 template <typename R>
-__global__ void k_scatter(FG g, const cplx<R>* __restrict__ S, cplx<R>* __restrict__ ref)
+__global__ void k_scatter(FG g, FastDiv dz, FastDiv dy, const cplx<R>* __restrict__ S, cplx<R>* __restrict__ ref)
 {
-    const int H = g.N3 / 2 + 1;
-    long n = (long)g.N1 * g.N2 * H;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        int l3 = (int)(i % H);
-        long r = i / H;
-        int l2 = (int)(r % g.N2), l1 = (int)(r / g.N2);
+    const unsigned n = (unsigned)g.N1 * g.N2 * (g.N3 / 2 + 1);
+    for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const unsigned r = fdiv(i, dz), x = fdiv(r, dy);
+        const int l3 = (int)(i - r * dz.d), l2 = (int)(r - x * dy.d), l1 = (int)x;
         cplx<R> v = czero<R>();
         if (l3 < g.nkz && lkept(g.mx, l1) && lkept(g.my, l2)) v = S[(long)lq(g.mx, l1) * g.sx + (long)lq(g.my, l2) * g.KZP + l3];
-        ref[i] = v;
+        st_nt(ref + i, v);
     }
 }
 
@@ -1374,13 +1372,15 @@ static dim3 grid_1d(size_t n)
 }
 template <typename R> int d_gather(const FG& g, const cplx<R>* ref, cplx<R>* S, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_gather<R>), grid_1d((size_t)g.mx.nk * g.sx), dim3(256), 0, st, g, ref, S);
+    hipLaunchKernelGGL((k_gather<R>), grid_1d((size_t)g.mx.nk * g.sx), dim3(256), 0, st, g, fast_div(g.KZP),
+                       fast_div(g.my.nk), ref, S);
     TH_CHECK_HIP(hipGetLastError());
     return OK;
 }
 template <typename R> int d_scatter(const FG& g, const cplx<R>* S, cplx<R>* ref, hipStream_t st)
 {
-    hipLaunchKernelGGL((k_scatter<R>), grid_1d((size_t)g.N1 * g.N2 * (g.N3 / 2 + 1)), dim3(256), 0, st, g, S, ref);
+    hipLaunchKernelGGL((k_scatter<R>), grid_1d((size_t)g.N1 * g.N2 * (g.N3 / 2 + 1)), dim3(256), 0, st, g,
+                       fast_div(g.N3 / 2 + 1), fast_div(g.N2), S, ref);
     TH_CHECK_HIP(hipGetLastError());
     return OK;
 }

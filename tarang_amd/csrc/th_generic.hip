@@ -310,15 +310,19 @@ int shift_x(cplx<R>* data, const Geo& g, int dir, hipStream_t st)
 struct GeoK {
     int basis, N1, N2, N3, H, dealias;
     double f1, f2, f3;
+    FastDiv dH, dN2;
 };
-static GeoK gk(const Geo& g) { return GeoK{g.basis, g.N1, g.N2, g.N3, g.H, g.dealias, g.kf[0], g.kf[1], g.kf[2]}; }
+static GeoK gk(const Geo& g)
+{
+    return GeoK{g.basis, g.N1, g.N2, g.N3, g.H, g.dealias, g.kf[0], g.kf[1], g.kf[2], fast_div(g.H), fast_div(g.N2)};
+}
 
 __device__ __forceinline__ void decode(const GeoK& g, long i, int& l1, int& l2, int& l3)
 {
-    l3 = (int)(i % g.H);
-    long r = i / g.H;
-    l2 = (int)(r % g.N2);
-    l1 = (int)(r / g.N2);
+    const unsigned r = fdiv((unsigned)i, g.dH), x = fdiv(r, g.dN2);
+    l3 = (int)((unsigned)i - r * g.dH.d);
+    l2 = (int)(r - x * g.dN2.d);
+    l1 = (int)x;
 }
 __device__ __forceinline__ int kx_g(const GeoK& g, int l1) { return g.basis == 1 ? l1 : kx_four(l1, g.N1); }
 
