@@ -17,10 +17,30 @@ struct Sched {
     int r[16];
 };
 
+// Schedules of the 3 2^a lengths with 12 or 24 points per thread.  Radix 6 and 12 (prime-factor, no inner
+// twiddles) leave one exchange less than radix 4 stages followed by a 2 and a 3, and first and last radix agree
+// wherever a pass needs that.  The z pass of 96 x 192 x 384 FP64 took 142 us with [4, 4, 4, 3] lines.
+constexpr Sched sched3(int L, int E)
+{
+    return E == 12 ? (L == 24   ? Sched{3, {2, 6, 2}}
+                      : L == 48  ? Sched{3, {4, 3, 4}}
+                      : L == 96  ? Sched{3, {4, 6, 4}}
+                      : L == 192 ? Sched{3, {4, 12, 4}}
+                      : L == 384 ? Sched{4, {4, 6, 4, 4}}
+                                 : Sched{0, {}})
+         : E == 24 ? (L == 48    ? Sched{2, {12, 4}}
+                      : L == 96  ? Sched{2, {12, 8}}
+                      : L == 192 ? Sched{3, {8, 3, 8}}
+                      : L == 384 ? Sched{3, {8, 6, 8}}
+                                 : Sched{0, {}})
+                   : Sched{0, {}};
+}
+
 // Greedy radix schedule: each radix must divide the remaining length and the points per thread.
 // Radix 16 only on request (it needs all 16 points of a butterfly live at once).
 constexpr Sched make_sched(int L, int E, bool r16 = false)
 {
+    if (sched3(L, E).n > 0) return sched3(L, E);
     Sched s{0, {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}};
     int m = L;
     while (m > 1) {
@@ -88,14 +108,15 @@ template <int L> struct ZPad {
     static constexpr int code(int s)
     {
         // sh * 16 + k; 0 = identity
-        return L == 16 ? (s == 0 ? 3 * 16 + 1 : 0)
-             : L == 24 ? (s <= 1 ? 2 * 16 + 1 : 0)
+        return L == 12 ? (s == 0 ? 1 * 16 + 1 : 0)
+             : L == 16 ? (s == 0 ? 3 * 16 + 1 : 0)
+             : L == 24 ? (s == 0 ? 1 * 16 + 1 : 0)
              : L == 32 ? (s == 0 ? 3 * 16 + 1 : 0)
-             : L == 48 ? (s <= 1 ? 2 * 16 + 1 : 0)
+             : L == 48 ? (s == 0 ? 2 * 16 + 1 : 0)
              : L == 64 ? (s == 0 ? 3 * 16 + 1 : 0)
-             : L == 96 ? (s <= 2 ? 3 * 16 + 1 : 0)
+             : L == 96 ? (s == 0 ? 3 * 16 + 1 : s == 1 ? 4 * 16 + 2 : 0)
              : L == 128 ? (s <= 1 ? 4 * 16 + 1 : 0)
-             : L == 192 ? (s == 0 || s == 2 ? 4 * 16 + 1 : s == 1 ? 2 * 16 + 1 : 0)
+             : L == 192 ? (s <= 1 ? 4 * 16 + 1 : 0)
              : L == 256 ? (s == 0 ? 5 * 16 + 1 : s == 1 ? 3 * 16 + 2 : 0)
              : 0;
     }
@@ -106,7 +127,7 @@ template <int L> struct ZPad {
         for (int s = 0; s < 8; s++) m = map(s, L - 1) + 1 > m ? map(s, L - 1) + 1 : m;
         return m;
     }
-    static constexpr int line = L == 16 ? 18 : L == 24 ? 30 : L == 32 ? 36 : L == 48 ? 60 : L == 64 ? 72 : L == 96 ? 120 : L == 128 ? 144 : L == 192 ? 240 : L == 256 ? 318 : L + 1;
+    static constexpr int line = L == 12 ? 18 : L == 16 ? 18 : L == 24 ? 38 : L == 32 ? 36 : L == 48 ? 60 : L == 64 ? 72 : L == 96 ? 120 : L == 128 ? 144 : L == 192 ? 208 : L == 256 ? 318 : L + 1;
     static_assert(line >= need(), "ZPad line stride too short");
 };
 
@@ -218,6 +239,47 @@ template <int SIGN, typename R> struct DFT<3, SIGN, R> {
     }
 };
 
+// 6 = 2 x 3 and 12 = 4 x 3 points by the prime-factor map: input n = (3 n1 + (L/3) n2) mod L, output
+// k = (kA k1 + 4 k2) mod L with kA = 3 (L = 6) or 9 (L = 12); nk = (L/M) n1 k1 + (L/3) n2 k2 (mod L), M = L/3, so
+// the two factors need no twiddles between them.
+template <int SIGN, typename R> struct DFT<6, SIGN, R> {
+    static __device__ __forceinline__ void run(cplx<R>* v)
+    {
+        cplx<R> a[2][3];
+#pragma unroll
+        for (int n1 = 0; n1 < 2; n1++) {
+#pragma unroll
+            for (int n2 = 0; n2 < 3; n2++) a[n1][n2] = v[(3 * n1 + 2 * n2) % 6];
+            DFT<3, SIGN, R>::run(a[n1]);
+        }
+#pragma unroll
+        for (int k2 = 0; k2 < 3; k2++) {
+            const cplx<R> p = a[0][k2] + a[1][k2], m = a[0][k2] - a[1][k2];
+            v[(4 * k2) % 6] = p;
+            v[(3 + 4 * k2) % 6] = m;
+        }
+    }
+};
+template <int SIGN, typename R> struct DFT<12, SIGN, R> {
+    static __device__ __forceinline__ void run(cplx<R>* v)
+    {
+        cplx<R> a[4][3];
+#pragma unroll
+        for (int n1 = 0; n1 < 4; n1++) {
+#pragma unroll
+            for (int n2 = 0; n2 < 3; n2++) a[n1][n2] = v[(3 * n1 + 4 * n2) % 12];
+            DFT<3, SIGN, R>::run(a[n1]);
+        }
+#pragma unroll
+        for (int k2 = 0; k2 < 3; k2++) {
+            cplx<R> q[4] = {a[0][k2], a[1][k2], a[2][k2], a[3][k2]};
+            DFT<4, SIGN, R>::run(q);
+#pragma unroll
+            for (int k1 = 0; k1 < 4; k1++) v[(9 * k1 + 4 * k2) % 12] = q[k1];
+        }
+    }
+};
+
 // One line of length L, P cooperating threads, E = L/P points per thread.
 //   before run(): v[i] = x[in_pos(t, i)]       after run(): v[i] = X[out_pos(t, i)]
 // lds points at element 0 of this line; element m lives at lds[m * LS].
@@ -244,18 +306,22 @@ template <typename R, int L, int P, int SIGN, bool R16 = false> struct LineFFT {
     // PRE0 overrides that first barrier: -1 as above (always taken without DBUF), 0 never (the caller
     // guarantees that no thread still reads the first exchange's buffer, e.g. nothing read it before this
     // FFT), 1 always (the caller read buffer 0 after the previous FFT).
-    template <int LS, bool WAVE = false, class Lay = NoPad, bool DBUF = false, int PRE0 = -1>
-    static __device__ __forceinline__ void run(cplx<R> (&v)[E], cplx<R>* lds, int t, const cplx<R>* __restrict__ tw)
+    // GUARD: threads with act == false keep to the barriers but leave LDS alone (a workgroup with more threads
+    // than its lines need).
+    template <int LS, bool WAVE = false, class Lay = NoPad, bool DBUF = false, int PRE0 = -1, bool GUARD = false>
+    static __device__ __forceinline__ void run(cplx<R> (&v)[E], cplx<R>* lds, int t, const cplx<R>* __restrict__ tw,
+                                               bool act = true)
     {
-        stage<0, 1, LS, WAVE, Lay, DBUF, PRE0>(v, lds, t, tw);
+        stage<0, 1, LS, WAVE, Lay, DBUF, PRE0, GUARD>(v, lds, t, tw, act);
     }
     // With DBUF, the buffer (0 or 1) that the last exchange did not use; after run() returns every thread
     // has finished reading it (the barrier after the last exchange's writes ensures that), so a caller may
     // write it at once.  Without exchanges (NST == 1) there is no such barrier and this is buffer 0.
     static constexpr int FREEBUF = (NST >= 2) ? 1 - ((NST - 2) & 1) : 0;
 
-    template <int s, int Ns, int LS, bool WAVE, class Lay, bool DBUF = false, int PRE0 = -1>
-    static __device__ __forceinline__ void stage(cplx<R> (&v)[E], cplx<R>* lds, int t, const cplx<R>* __restrict__ tw)
+    template <int s, int Ns, int LS, bool WAVE, class Lay, bool DBUF = false, int PRE0 = -1, bool GUARD = false>
+    static __device__ __forceinline__ void stage(cplx<R> (&v)[E], cplx<R>* lds, int t, const cplx<R>* __restrict__ tw,
+                                                 bool act = true)
     {
         constexpr int Rr = S.r[s];
         constexpr int B = E / Rr;
@@ -277,18 +343,22 @@ template <typename R, int L, int P, int SIGN, bool R16 = false> struct LineFFT {
             cplx<R>* buf = DBUF ? lds + (s & 1) * (L * LS) : lds;
             constexpr bool pre = (s == 0 && PRE0 >= 0) ? (PRE0 == 1) : (!DBUF || (s == 0 && (NST - 1) % 2 == 1));
             if constexpr (pre) line_sync<WAVE>();
+            if (!GUARD || act) {
 #pragma unroll
-            for (int b = 0; b < B; b++) {
-                const int j = t + P * b;
-                const int base = (j / Ns) * Ns * Rr + (j % Ns);
+                for (int b = 0; b < B; b++) {
+                    const int j = t + P * b;
+                    const int base = (j / Ns) * Ns * Rr + (j % Ns);
 #pragma unroll
-                for (int r = 0; r < Rr; r++) buf[Lay::map(s, base + r * Ns) * LS] = v[b * Rr + r];
+                    for (int r = 0; r < Rr; r++) buf[Lay::map(s, base + r * Ns) * LS] = v[b * Rr + r];
+                }
             }
             line_sync<WAVE>();
             constexpr int Rn = S.r[s + 1];
+            if (!GUARD || act) {
 #pragma unroll
-            for (int i = 0; i < E; i++) v[i] = buf[Lay::map(s, t + P * (i / Rn) + (i % Rn) * (L / Rn)) * LS];
-            stage<s + 1, Ns * Rr, LS, WAVE, Lay, DBUF, PRE0>(v, lds, t, tw);
+                for (int i = 0; i < E; i++) v[i] = buf[Lay::map(s, t + P * (i / Rn) + (i % Rn) * (L / Rn)) * LS];
+            }
+            stage<s + 1, Ns * Rr, LS, WAVE, Lay, DBUF, PRE0, GUARD>(v, lds, t, tw, act);
         }
     }
 };
