@@ -64,6 +64,7 @@ FG make_fg(const Geo& geo, int prec)
     g.norm = 0.5 / ((double)geo.N1 * (double)geo.N2 * (double)geo.N3);
     if (g.scft) g.norm *= 0.5;                                          // Norm_SCFT: transforms scale by 1 / (2 N1 N2 N3)
     g.nbox = 1;
+    g.fp64 = prec ? 0 : 1;
     return g;
 }
 
@@ -95,6 +96,8 @@ struct th_state {
     hipEvent_t cev = nullptr;    // recorded after the last upload from hcoef
     bool cev_live = false;
     int var[NPASS] = {0, 0, 0, 0, 0};   // launch-shape variant per pass (autotuner)
+    bool plane = false;          // passes 2-4 as one launch, X1 -> X3 (th_plane.hpp); the y passes launch nothing
+    bool split = false;          // x-forward with the products side by side (th_plane.hpp)
     // Chained step (NS or MHD, unforced): each stage's x-forward also does the next stage's x-inverse, so a
     // step runs 4 passes per stage; X1 must then hold the x-inverse of S when a step starts (chain_ok), which a
     // single x-inverse launch restores after anything else has used the buffers or changed S.
@@ -129,6 +132,39 @@ static std::string tune_key(const th_state* s)
     snprintf(k, sizeof k, "fused:gfx950:%s:%s:N%dx%dx%d:boxes%d", s->esz == 8 ? "fp32" : "fp64",
              s->physics == TH_MHD ? "mhd" : s->physics == TH_RB ? "rb" : "ns", s->fg.N1, s->fg.N2, s->fg.N3, s->nbox);
     return k;
+}
+
+// Short boxes (th_plane.hpp).  Both rules are on the grid alone, so that a box computes the same bits alone and in an
+// ensemble.
+//
+// Passes 2 to 4 as one launch: N2 and N3 up to 128 with at most 8192 points per plane (74 KB of LDS in FP64), and in
+// FP64 planes past 4608 points only on long boxes, where the three passes wait on memory rather than on launches.
+// us per step, three passes / plane pass: 32^3 FP64 160 / 98, 64^3 FP64 174 / 125, eight 64^3 FP32 306 / 187,
+// 512 x 64 x 64 FP64 465 / 309, 512 x 128 x 64 FP32 564 / 369; past the line 96^3 FP32 213 / 202 to 248,
+// 128^3 FP64 359 / 479 (one 147 KB plane per CU), 64 x 64 x 128 FP64 178 / 185.
+bool th::plane_ok(const FG& g)
+{
+    if (g.N2 > 128 || g.LZ > 64 || g.nkz != g.N3 / 3) return false;
+    const int pts = g.N2 * g.N3;
+    return pts <= (g.fp64 && g.N1 < 256 ? 4608 : 8192);
+}
+// The x-forward with the products side by side, NS and MHD: where one workgroup per tile of columns leaves CUs idle
+// or waiting.  us per step, one after another / side by side: 16 x 64 x 64 FP64 107 / 59, 64 x 128 x 128 FP32
+// 207 / 180, 128 x 64 x 64 FP64 173 / 130; past the line 64 x 256 x 256 FP32 347 / 392, eight 96^3 FP32 561 / 743.
+static bool split_ok(const FG& g, int physics)
+{
+    const long pts = (long)g.N1 * g.my.nk * g.nkz;
+    return physics != TH_RB && ((g.N1 <= 64 && pts <= 250000) || (g.N1 <= 128 && pts <= 120000));
+}
+
+// Products of the pipelines (numbered as ZProd in th_fused_kern.hpp), in an order that hands operands on: each
+// rotation step's last operand is the next one's first (NS, RB) or its first y (MHD)
+static const PlaneTab& plane_tab(int physics)
+{
+    static const PlaneTab ns = {2, {0, 1, 2}, {{0, 1, 0}, {1, 2, 0}, {2, 0, 0}}, {{0, 3, 0}, {1, 4, 0}, {2, 5, 0}}};
+    static const PlaneTab mhd = {3, {0, 1, 2}, {{3, 4, 5}, {5, 4, 3}, {3, 4, 5}}, {{0, 1, 2}, {5, 4, 3}, {6, 7, 8}}};
+    static const PlaneTab rb = {3, {0, 1, 2}, {{0, 3, 1}, {1, 3, 2}, {2, 3, 0}}, {{0, 6, 3}, {1, 7, 4}, {2, 8, 5}}};
+    return physics == TH_NS ? ns : physics == TH_MHD ? mhd : rb;
 }
 
 // Fused state for nbox boxes of the plan's size. Single states (nbox == 1) also keep room for the
@@ -177,6 +213,8 @@ static int state_create(th_plan* p, th_state** out, int physics, int nbox)
         delete s;
         return r;
     }
+    s->plane = plane_ok(g);
+    s->split = split_ok(g, physics);
     std::vector<int> tv;
     if (tune_lookup(p->ctx, tune_key(s), tv) && (int)tv.size() == NPASS)
         for (int k = 0; k < NPASS; k++) s->var[k] = (tv[k] >= 0 && tv[k] < pass_nvar(k)) ? tv[k] : 0;
@@ -327,6 +365,17 @@ static int set_coefs(th_state* s, const double* dt, const double* nu, const doub
     return OK;
 }
 
+// Workgroups per x-plane of the plane pass: one per product while that is at most four small planes per CU, one per
+// rotation step up to 384 planes, and less repeated work beyond.  us per step with 1 / 2 / 3 / 6 groups (NS):
+// 32^3 FP64 139 / 116 / 104 / 99, 256 x 64 x 64 FP32 211 / 188 / 179 / 191, 512 x 48 x 48 FP32 262 / 230 / 253 / 272,
+// 512 x 64 x 64 FP64 309 / 329 / 328 / 391.
+static int plane_groups(const FG& g, int nout)
+{
+    const int n = g.N1 * g.nbox, pts = g.N2 * g.N3;
+    if (n * nout <= 1024 && pts <= 4096) return nout;
+    return n <= 384 ? 3 : n < 1024 ? (nout == 6 ? 2 : 3) : 1;
+}
+
 // Pass `pass` of RK stage `stage` (1..4) for every box of s, launch-shape variant var.  Stage 1
 // reads the state, later stages the stage field; pass 5 writes the stage field / accumulator
 // (and the state in stage 4).
@@ -352,18 +401,24 @@ template <typename R> static int run_pass(th_state* s, int pass, int var, int st
         if (ph == TH_RB) return d_sx_inv<R>(g, src, X1, twx, p->twd<R>(4 * g.N1), st);
         return ph == TH_MHD ? d_xinv<R, 1>(g, src, X1, nin, twx, sel, var, st)
                             : d_xinv<R, 0>(g, src, X1, nin, twx, sel, var, st);
-    case PASS_YINV: return d_yinv<R>(g, X1, X2, nin, twy, var, st);
+    case PASS_YINV: return s->plane ? (int)OK : d_yinv<R>(g, X1, X2, nin, twy, var, st);
     case PASS_Z: {
         const cplx<R>* twz = p->twd<R>(g.LZ);
         const cplx<R>* twn = p->twd<R>(g.N3);
+        if (s->plane) return d_plane<R>(g, plane_tab(ph), plane_groups(g, nout), X1, X3, twy, twz, twn, st);
         if (ph == TH_RB) return d_z<R, 3>(g, X2, X3, twz, twn, var, st);
         return ph == TH_MHD ? d_z<R, 1>(g, X2, X3, twz, twn, var, st) : d_z<R, 0>(g, X2, X3, twz, twn, var, st);
     }
-    case PASS_YFWD: return d_yfwd<R>(g, X3, X1, nout, twy, var, st);
-    default:
-        if (ph == TH_RB) return d_sx_fwd_rb<R>(g, X1, S, Vs, acc, twx, p->twd<R>(4 * g.N1), sc, var, st);
-        return ph == TH_MHD ? d_xfwd<R, 1>(g, X1, S, Vs, acc, twx, sc, var, st, chain)
-                            : d_xfwd<R, 0>(g, X1, S, Vs, acc, twx, sc, var, st, chain);
+    case PASS_YFWD: return s->plane ? (int)OK : d_yfwd<R>(g, X3, X1, nout, twy, var, st);
+    default: {
+        const cplx<R>* D = s->plane ? X3 : X1;
+        if (ph == TH_RB) return d_sx_fwd_rb<R>(g, D, S, Vs, acc, twx, p->twd<R>(4 * g.N1), sc, var, st);
+        if (s->split)
+            return ph == TH_MHD ? d_xsplit<R, 1>(g, D, X1, S, Vs, acc, twx, sc, st, chain)
+                                : d_xsplit<R, 0>(g, D, X1, S, Vs, acc, twx, sc, st, chain);
+        return ph == TH_MHD ? d_xfwd<R, 1>(g, D, X1, S, Vs, acc, twx, sc, var, st, chain)
+                            : d_xfwd<R, 0>(g, D, X1, S, Vs, acc, twx, sc, var, st, chain);
+    }
     }
 }
 
@@ -679,7 +734,7 @@ static int ensure_twiddles(th_plan* p, const FG& g, hipStream_t st)
 static bool step_chained(const th_state* s)
 {
     return (s->physics == TH_NS || s->physics == TH_MHD) &&
-           (s->plan->prec ? d_xfwd_chainable<float>(s->fg) : d_xfwd_chainable<double>(s->fg));
+           (s->split || (s->plan->prec ? d_xfwd_chainable<float>(s->fg) : d_xfwd_chainable<double>(s->fg)));
 }
 
 extern "C" int th_step(th_plan* p, th_state* s, double dt, const th_phys* ph, int nsteps)
@@ -898,7 +953,8 @@ extern "C" int th_flux_shell_tr(th_plan* p, th_state* s, const double* radii, in
 // ------------------------------------------------------------------------------------------
 // Per-pass timing of one fused RK stage with HIP events on the plan's stream, and each pass's
 // algorithmic HBM bytes (compulsory reads + writes of kept data; padding excluded).  A chained state is timed as
-// th_step runs it: the x-inverse once beforehand (not timed: 0 ms, 0 bytes) and the chained x-forward.
+// th_step runs it: the x-inverse once beforehand (not timed: 0 ms, 0 bytes) and the chained x-forward.  Where passes 2
+// to 4 are one launch, it is reported as the z pass and the y passes read 0 ms, 0 bytes.
 // ------------------------------------------------------------------------------------------
 template <typename R> static int profile_impl(th_state* s, double dt, double nu, double eta, int stage, int nrep,
                                               double* ms, double* bytes)
@@ -953,8 +1009,12 @@ template <typename R> static int profile_impl(th_state* s, double dt, double nu,
         b[PASS_XFWD] = e * (nout * cA + (state_rw - (stage < 4 ? 1 : 0)) * nst * cS + nin * cA);
         b[PASS_XINV] = 0;
     }
+    if (s->plane) {
+        b[PASS_Z] = e * (nin * cA + nout * cA);
+        b[PASS_YINV] = b[PASS_YFWD] = 0;
+    }
     for (int k = 0; k < 5; k++) {
-        ms[k] = (chained && k == PASS_XINV) ? 0.0 : tot[k] / nrep;
+        ms[k] = b[k] == 0 ? 0.0 : tot[k] / nrep;
         bytes[k] = b[k];
     }
     return OK;
@@ -994,6 +1054,8 @@ template <typename R> static int tune_impl(th_state* s, int nrep, hipStream_t st
     // ramp, another queue's work) cannot decide the choice on its own
     constexpr int ROUNDS = 3;
     for (int k = 0; k < NPASS && !r; k++) {
+        // passes without launch shapes to choose from (the plane pass is one shape, the split x-forward too)
+        if ((s->plane && (k == PASS_YINV || k == PASS_Z || k == PASS_YFWD)) || (s->split && k == PASS_XFWD)) continue;
         const bool ch = chained && k == PASS_XFWD;
         double tv[8];
         for (int v = 0; v < 8; v++) tv[v] = 1e300;

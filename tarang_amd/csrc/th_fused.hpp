@@ -61,6 +61,7 @@ struct FG {
     long bS, bA, bB, bC;   // box strides of the state, A/D, B and C buffers (batched boxes of one size)
     int nbox;              // boxes of this size advanced by one launch per pass
     int scft;              // sin/cos along x (SCFT basis), else Fourier
+    int fp64;              // precision of the plan
     double f1, f2, f3;
     double norm; // 1 / (2 N1 N2 N3): the line transforms' 1 / (N1 N2 N3) and the z pass's unpacking 1/2 (SCFT: 1/2 more)
     int keep3 = 0; // chained x-forward of a forced state: write the stage-3 output (the last stage's input field)
@@ -111,10 +112,10 @@ int d_z(const FG& g, const cplx<R>* B, cplx<R>* Cc, const cplx<R>* twL, const cp
 template <typename R>
 int d_yfwd(const FG& g, const cplx<R>* Cc, cplx<R>* D, int nc, const cplx<R>* tw, int var, hipStream_t st);
 template <typename R, int MODE>
-int d_xfwd(const FG& g, const cplx<R>* D, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw, const StageCoef* sc,
-           int var, hipStream_t st, bool chain = false);
-// chain: the x-forward also transforms its stage output back along x and writes the next stage's A lines over
-// D's first components (NS: U in 0-2; MHD: Z+ in 0-2, Z- in 3-5; the stage field is not written);
+int d_xfwd(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw,
+           const StageCoef* sc, int var, hipStream_t st, bool chain = false);
+// chain: the x-forward also transforms its stage output back along x and writes the next stage's A lines to
+// Aout's first components (Aout may be D) (NS: U in 0-2; MHD: Z+ in 0-2, Z- in 3-5; the stage field is not written);
 // d_xfwd_chainable says whether N1 has that kernel
 template <typename R>
 bool d_xfwd_chainable(const FG& g);
@@ -128,6 +129,26 @@ int d_sx_fwd_rb(const FG& g, const cplx<R>* D, cplx<R>* S, cplx<R>* Vs, cplx<R>*
                 const cplx<R>* tw4, const StageCoef* sc, int var, hipStream_t st);
 template <typename R> int d_gather(const FG& g, const cplx<R>* ref, cplx<R>* S, hipStream_t st);
 template <typename R> int d_scatter(const FG& g, const cplx<R>* S, cplx<R>* ref, hipStream_t st);
+
+// ---- short boxes (th_plane.hpp) ----
+// Passes 2 to 4 in one launch, A (nin lines) -> D (nout lines), for boxes with plane_ok; ngrp = 3 or nout workgroups
+// per x-plane.  D may not be A.
+struct PlaneTab;
+bool plane_ok(const FG& g);
+template <typename R>
+int d_plane(const FG& g, const PlaneTab& tab, int ngrp, const cplx<R>* A, cplx<R>* D, const cplx<R>* tw2, const cplx<R>* twL,
+            const cplx<R>* twN, hipStream_t st);
+// The x-forward with the products side by side (N1 <= 128), NS (MODE 0) and MHD (MODE 1); chained for every N1
+template <typename R, int MODE>
+int d_xsplit(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw,
+             const StageCoef* sc, hipStream_t st, bool chain);
+
+// Operand and product table of a pipeline (ZProd of th_fused_kern.hpp as plain numbers): product j of rotation step r
+// multiplies input x[r] by input y[r][j] into output o[r][j]; operands are kept from one product to the next where the order allows it.
+struct PlaneTab {
+    signed char npr;
+    signed char x[3], y[3][3], o[3][3];
+};
 
 FG make_fg(const Geo& geo, int prec);
 

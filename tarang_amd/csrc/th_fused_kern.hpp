@@ -440,23 +440,28 @@ __device__ __forceinline__ Dc dadd(const Dc& a, const Dc& b) { return dmk(a.x + 
 // Returns the stage's output, the field the next stage transforms: the stage field (stages 1-3) or the new
 // state (stage 4), as stored.  WVS = false leaves the stage field unwritten (its only reader, the next x-inverse,
 // then runs on the returned value in registers).
-template <typename R>
+// NT: the accumulator is written non-temporally.
+template <typename R, bool NT = true>
 __device__ __forceinline__ cplx<R> rk_store(int stage, double dt, double eh, double e1, const Dc& rhs, const cplx<R>& s0,
                                             const cplx<R>& a0, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, bool wvs = true)
 {
     const Dc V0 = dl(s0);
     cplx<R> out;
+    auto put = [](cplx<R>* p, cplx<R> v) {
+        if constexpr (NT) st_nt(p, v);
+        else *p = v;
+    };
     if (stage == 1) {
         Dc v = dadd(V0, dsc(rhs, 0.5 * dt));
         out = ds<R>(dsc(v, eh));
-        st_nt(acc, ds<R>(dsc(dsc(rhs, e1), dt / 6)));
+        put(acc, ds<R>(dsc(dsc(rhs, e1), dt / 6)));
     } else if (stage == 2) {
         out = ds<R>(dadd(dsc(V0, eh), dsc(rhs, 0.5 * dt)));
-        st_nt(acc, ds<R>(dadd(dl(a0), dsc(dsc(rhs, eh), dt / 3))));
+        put(acc, ds<R>(dadd(dl(a0), dsc(dsc(rhs, eh), dt / 3))));
     } else if (stage == 3) {
         Dc v = dadd(dsc(V0, eh), dsc(rhs, 1.0 * dt));
         out = ds<R>(dsc(v, eh));
-        st_nt(acc, ds<R>(dadd(dl(a0), dsc(dsc(rhs, eh), dt / 3))));
+        put(acc, ds<R>(dadd(dl(a0), dsc(dsc(rhs, eh), dt / 3))));
     } else {
         Dc a = dadd(dl(a0), dsc(rhs, dt / 6));
         out = ds<R>(dadd(dsc(V0, e1), a));
@@ -485,12 +490,12 @@ template <int L, int P, int E, int RL> constexpr int xnext(int i)
 
 // CHAIN: the epilogue also performs the next stage's x-inverse: the stage output (stage field, or the new
 // state in stage 4) stays in the accumulator registers in place of N and is transformed back along x, and the
-// A lines are written over this tile's columns of D (every product of the tile has been read by then, and no
-// other workgroup reads these columns); the stage field itself is not written, except the stage-3 output (the
+// A lines are written to this tile's columns of Aout, which may be D itself (every product of the tile has been read
+// by then, and no other workgroup reads these columns); the stage field itself is not written, except the stage-3 output (the
 // last stage's input) of a forced state (FG::keep3), from which the host evaluates the outputs' force.  NS: components 0-2 = U.
 // MHD: the Elsasser lines of k_fx_inv MODE 1, Z+ = U + B into components 0-2 and Z- = U - B into 3-5.
 template <typename R, int L, int P, int T, int MODE, bool CHAIN = false>
-__global__ __launch_bounds__(T * P) __attribute__((amdgpu_waves_per_eu((MODE == 0 && sizeof(R) == 4 && L % 3 != 0) ? 4 : 1))) void k_fx_fwd(FG g, const cplx<R>* D, cplx<R>* S, cplx<R>* Vs,
+__global__ __launch_bounds__(T * P) __attribute__((amdgpu_waves_per_eu((MODE == 0 && sizeof(R) == 4 && L % 3 != 0) ? 4 : 1))) void k_fx_fwd(FG g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs,
                                                   cplx<R>* acc, const cplx<R>* __restrict__ tw,
                                                   const StageCoef* __restrict__ coefs)
 {
@@ -534,6 +539,7 @@ __global__ __launch_bounds__(T * P) __attribute__((amdgpu_waves_per_eu((MODE == 
     }
     __syncthreads();
     D += box * g.bA;
+    Aout += box * g.bA;
     S += box * g.bS;
     Vs += box * g.bS;
     acc += box * g.bS;
@@ -715,7 +721,6 @@ __global__ __launch_bounds__(T * P) __attribute__((amdgpu_waves_per_eu((MODE == 
         // the next stage's x-inverse (k_fx_inv MODE 0 / 1): register i holds row F::out_pos(t, i), which is
         // FI::in_pos(t, i) since the schedule's first and last radix agree
         using FI = LineFFT<R, L, P, +1>;
-        cplx<R>* Aout = const_cast<cplx<R>*>(D);
 #pragma unroll
         for (int a = 0; a < NA; a++) {   // unrolled: Nacc[a] must stay a compile-time register
             FI::template run<T, false, NoPad, true>(Nacc[a], lds + c, t, twl + opaque_zero());
@@ -1157,8 +1162,8 @@ template <typename R, int L, int MODE> constexpr int xfwd_T()
 }
 
 template <typename R, int L, int MODE, int V, bool CHAIN = false>
-static int launch_xfwd(const FG& g, const cplx<R>* D, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw,
-                       const StageCoef* sc, hipStream_t st)
+static int launch_xfwd(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc,
+                       const cplx<R>* tw, const StageCoef* sc, hipStream_t st)
 {
     constexpr int E = xfwd_E(L), P = L / E, T0 = xfwd_T<R, L, MODE>();
     // variant 1: half-width tiles; variant 2: double-width tiles (full 128-byte rows at 512 lines)
@@ -1172,14 +1177,14 @@ static int launch_xfwd(const FG& g, const cplx<R>* D, cplx<R>* S, cplx<R>* Vs, c
     if constexpr (CHAIN) {
         if constexpr (MODE <= 1 && LineFFT<R, L, P, -1>::R0 == LineFFT<R, L, P, -1>::RL) {
             hipLaunchKernelGGL((k_fx_fwd<R, L, P, T, MODE, true>), dim3(g.my.nk * ntz, g.nbox), dim3(T * P), 0, st, g, D,
-                               S, Vs, acc, tw, sc);
+                               Aout, S, Vs, acc, tw, sc);
         } else {
             set_error("chained x-forward: no chained kernel for N1 = %d", L);
             return E_UNSUPPORTED;
         }
     } else {
-        hipLaunchKernelGGL((k_fx_fwd<R, L, P, T, MODE>), dim3(g.my.nk * ntz, g.nbox), dim3(T * P), 0, st, g, D, S, Vs, acc,
-                           tw, sc);
+        hipLaunchKernelGGL((k_fx_fwd<R, L, P, T, MODE>), dim3(g.my.nk * ntz, g.nbox), dim3(T * P), 0, st, g, D, Aout, S, Vs,
+                           acc, tw, sc);
     }
     TH_CHECK_HIP(hipGetLastError());
     return OK;
@@ -1268,22 +1273,22 @@ static int yfwd_v(const FG& g, const cplx<R>* Cc, cplx<R>* D, int nc, const cplx
     return launch_yfwd<R, L, 0>(g, Cc, D, nc, tw, st);
 }
 template <typename R, int MODE, int L>
-static int xfwd_v(const FG& g, const cplx<R>* D, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw, const StageCoef* sc,
+static int xfwd_v(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw, const StageCoef* sc,
                   int var, hipStream_t st, bool chain)
 {
     if (chain) {
         if constexpr (L >= 128)
-            if (var == 1) return launch_xfwd<R, L, MODE, 1, true>(g, D, S, Vs, acc, tw, sc, st);
+            if (var == 1) return launch_xfwd<R, L, MODE, 1, true>(g, D, Aout, S, Vs, acc, tw, sc, st);
         if constexpr (L >= 128 && sizeof(R) == 4 && MODE == 0 && L % 3 != 0 && 2 * xfwd_T<R, L, MODE>() * (L / xfwd_E(L)) <= 1024)
-            if (var == 2) return launch_xfwd<R, L, MODE, 2, true>(g, D, S, Vs, acc, tw, sc, st);
-        return launch_xfwd<R, L, MODE, 0, true>(g, D, S, Vs, acc, tw, sc, st);
+            if (var == 2) return launch_xfwd<R, L, MODE, 2, true>(g, D, Aout, S, Vs, acc, tw, sc, st);
+        return launch_xfwd<R, L, MODE, 0, true>(g, D, Aout, S, Vs, acc, tw, sc, st);
     }
     if constexpr (L >= 128)
-        if (var == 1) return launch_xfwd<R, L, MODE, 1>(g, D, S, Vs, acc, tw, sc, st);
+        if (var == 1) return launch_xfwd<R, L, MODE, 1>(g, D, Aout, S, Vs, acc, tw, sc, st);
     // 1024-thread workgroups hold a wave to 128 VGPRs: only the FP32 NS kernels fit (124)
     if constexpr (L >= 128 && sizeof(R) == 4 && MODE == 0 && L % 3 != 0 && 2 * xfwd_T<R, L, MODE>() * (L / xfwd_E(L)) <= 1024)
-        if (var == 2) return launch_xfwd<R, L, MODE, 2>(g, D, S, Vs, acc, tw, sc, st);
-    return launch_xfwd<R, L, MODE, 0>(g, D, S, Vs, acc, tw, sc, st);
+        if (var == 2) return launch_xfwd<R, L, MODE, 2>(g, D, Aout, S, Vs, acc, tw, sc, st);
+    return launch_xfwd<R, L, MODE, 0>(g, D, Aout, S, Vs, acc, tw, sc, st);
 }
 // whether the chained x-forward exists for this line length and variant (NS or MHD, first radix = last radix)
 template <typename R, int L, int MODE, int V> constexpr bool xfwd_chainable()
@@ -1321,10 +1326,10 @@ int d_yfwd(const FG& g, const cplx<R>* Cc, cplx<R>* D, int nc, const cplx<R>* tw
 #undef C_
 }
 template <typename R, int MODE>
-int d_xfwd(const FG& g, const cplx<R>* D, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw, const StageCoef* sc,
-           int var, hipStream_t st, bool chain)
+int d_xfwd(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw,
+           const StageCoef* sc, int var, hipStream_t st, bool chain)
 {
-#define C_(n) case n: return xfwd_v<R, MODE, n>(g, D, S, Vs, acc, tw, sc, var, st, chain);
+#define C_(n) case n: return xfwd_v<R, MODE, n>(g, D, Aout, S, Vs, acc, tw, sc, var, st, chain);
     switch (g.N1) { TH_FLENS(C_) default: set_error("fused: N1 %d unsupported", g.N1); return E_UNSUPPORTED; }
 #undef C_
 }
@@ -1398,9 +1403,9 @@ template <typename R> int d_scatter(const FG& g, const cplx<R>* S, cplx<R>* ref,
     template int d_sx_fwd_rb<R>(const FG&, const cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, const cplx<R>*,            \
                                 const cplx<R>*, const StageCoef*, int, hipStream_t);                                  \
     template int d_yfwd<R>(const FG&, const cplx<R>*, cplx<R>*, int, const cplx<R>*, int, hipStream_t);              \
-    template int d_xfwd<R, 0>(const FG&, const cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, const cplx<R>*,              \
+    template int d_xfwd<R, 0>(const FG&, const cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, const cplx<R>*,    \
                               const StageCoef*, int, hipStream_t, bool);                                               \
-    template int d_xfwd<R, 1>(const FG&, const cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, const cplx<R>*,              \
+    template int d_xfwd<R, 1>(const FG&, const cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, const cplx<R>*,    \
                               const StageCoef*, int, hipStream_t, bool);                                               \
     template bool d_xfwd_chainable<R>(const FG&);                                                                      \
     template int d_xfwd_et<R>(const FG&, const cplx<R>*, const cplx<R>*, const cplx<R>*, const double*, int, int,    \

@@ -61,3 +61,51 @@ def test_fused_step_of_every_length(ctx, L, axis, prec, tol):
     m = max(np.abs(v).max() for v in V)
     for got, ref in zip(s.download(), V):
         assert np.abs(got.cpu().numpy() - ref).max() <= tol * m
+
+
+# the edges of the short-box rules: smallest planes, one row of every length of the plane pass, the largest planes of
+# each precision, boxes on both sides of the split x-forward's line; boxes = 20 passes the group counts' limits
+@pytest.mark.parametrize("N", [(16, 16, 16), (24, 24, 24), (32, 48, 32), (48, 96, 48), (256, 64, 128), (64, 128, 64),
+                               (128, 16, 128), (96, 64, 64), (128, 96, 64), (256, 128, 64), (64, 128, 128)])
+@pytest.mark.parametrize("physics", ("ns", "mhd", "rb"))
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("fp32", 1e-5)])
+def test_short_boxes(ctx, N, physics, prec, tol):
+    from tarang_amd import Plan, State, abi
+    print(N, physics, prec, flush=True)
+    basis = "SCFT" if physics == "rb" else "FOUR"
+    o = Oracle(N, basis=basis)
+    p = Plan(ctx, N, basis=basis, precision=prec)
+    F = o.ic_random(7, E0=0.5, kp=3.0)
+    F += o.ic_random(8, E0=0.3, kp=3.0) if physics == "mhd" else [o.ic_random_scalar(4, 1e-2)] if physics == "rb" else []
+    s = State(p, {"ns": abi.TH_NS, "mhd": abi.TH_MHD, "rb": abi.TH_RB}[physics])
+    s.upload([p.to_dev(v) for v in F])
+    if physics == "ns":
+        s.step(1e-3, nu=5e-3, steps=2)
+        o.rk4_ns(F, 5e-3, 1e-3, steps=2)
+    elif physics == "mhd":
+        s.step(1e-3, nu=5e-3, eta=4e-3, steps=2)
+        o.rk4_mhd(F[:3], F[3:], 5e-3, 4e-3, 1e-3, steps=2)
+    else:
+        s.step(1e-3, Ra=1e4, Pr=1.0, steps=2)
+        o.rk4_rb(F[:3], F[3], 1e4, 1.0, 1e-3, steps=2)
+    m = max(np.abs(v).max() for v in F)
+    for got, ref in zip(s.download(), F):
+        assert np.abs(got.cpu().numpy() - ref).max() <= tol * m
+
+
+@pytest.mark.parametrize("prec", ("fp64", "fp32"))
+def test_short_boxes_in_an_ensemble_equal_single_boxes(ctx, prec):
+    from tarang_amd import Ensemble, Plan, State
+    shapes = [(64, 64, 64)] * 20 + [(32, 32, 32)] * 3
+    V = {N: Oracle(N).ic_random(3, E0=0.5, kp=3.0) for N in set(shapes)}
+    e = Ensemble(ctx, shapes, precision=prec)
+    for b, N in enumerate(shapes):
+        e.upload(b, [e.plan(b).to_dev(v) for v in V[N]])
+    e.step(np.full(len(shapes), 1e-3), np.full(len(shapes), 5e-3), steps=2)
+    for b in (0, 19, 20, 22):
+        p = Plan(ctx, shapes[b], precision=prec)
+        s = State(p)
+        s.upload([p.to_dev(v) for v in V[shapes[b]]])
+        s.step(1e-3, nu=5e-3, steps=2)
+        for got, ref in zip(e.download(b), s.download()):
+            assert np.array_equal(got.cpu().numpy(), ref.cpu().numpy())
