@@ -151,40 +151,18 @@ __global__ __launch_bounds__(T * P) void k_fy_inv(FG g, const cplx<R>* __restric
 // MODE 1 (MHD): in Z+0..2, Z-0..2,    out P(i,j) = Z+_i Z-_j at 3i+j             (RSprod.cc:117-151)
 // MODE 2 (ET):  in H0..2,  G0..2,     out P(i,j) = G_i H_j at 3i+j               (ET_RSprod.cc:49-85)
 template <int MODE> struct ZProd;
-// Products are also listed as 3 rotation steps r of NPR products each: product j of step r multiplies
-// x = u[G0 + r] by operand yop(j) (-1 - k: u[G0 + (r + k) % 3]; k >= 0: input k) into output pout(r, j).
 template <> struct ZProd<0> {
     static constexpr int NIN = 3, NOUT = 6;
-    static constexpr int a(int p) { return p < 3 ? p : p - 3; }
-    static constexpr int b(int p) { return p < 3 ? p : (p == 5 ? 0 : p - 2); }
-    static constexpr int G0 = 0, NPR = 2;
-    static constexpr int yop(int j) { return j == 0 ? -1 : -2; }
-    static constexpr int pout(int r, int j) { return j == 0 ? r : 3 + r; }
 };
 template <> struct ZProd<1> {
     static constexpr int NIN = 6, NOUT = 9;
-    static constexpr int a(int p) { return p / 3; }
-    static constexpr int b(int p) { return 3 + p % 3; }
-    static constexpr int G0 = 0, NPR = 3;
-    static constexpr int yop(int j) { return 3 + j; }
-    static constexpr int pout(int r, int j) { return 3 * r + j; }
 };
 template <> struct ZProd<2> {
     static constexpr int NIN = 6, NOUT = 9;
-    static constexpr int a(int p) { return 3 + p / 3; }
-    static constexpr int b(int p) { return p % 3; }
-    static constexpr int G0 = 3, NPR = 3;
-    static constexpr int yop(int j) { return j; }
-    static constexpr int pout(int r, int j) { return 3 * r + j; }
 };
 // MODE 3 (RB): in V1 V2 V3 T, out V1V1 V2V2 V3V3 V1V2 V2V3 V3V1 V1T V2T V3T (compute_nlin_SF.cc:80-177)
 template <> struct ZProd<3> {
     static constexpr int NIN = 4, NOUT = 9;
-    static constexpr int a(int p) { return p % 3; }
-    static constexpr int b(int p) { return p < 3 ? p : (p < 6 ? (p - 2) % 3 : 3); }
-    static constexpr int G0 = 0, NPR = 3;
-    static constexpr int yop(int j) { return j == 0 ? -1 : j == 1 ? -2 : 3; }
-    static constexpr int pout(int r, int j) { return 3 * j + r; }
 };
 
 // Lane t of a z line holds the points at positions t + P m, m = 0..E-1, in a register order fixed
@@ -193,6 +171,11 @@ template <int E, int Rr> __device__ __forceinline__ constexpr int zreg(int m)
 {
     return (m % (E / Rr)) * Rr + m / (E / Rr);
 }
+
+// MHD and energy transfer: whether the three second operands stay in registers (96 VGPRs in FP64 with 8 points per
+// thread, which still leaves two waves per SIMD: 256^3 MHD z pass 287 us, 364 transforming them again) or, for
+// the FP64 lines with 12 points per thread, are transformed again for each first operand (held, they would spill)
+template <typename R, int E> constexpr bool ZHELD = sizeof(R) == 4 || E <= 8;
 
 template <typename R, int LZ, int P, int TZ, int MODE>
 __global__ __launch_bounds__(TZ * P) void k_fz(FG g, const cplx<R>* __restrict__ B, cplx<R>* __restrict__ Cout,
@@ -224,9 +207,6 @@ __global__ __launch_bounds__(TZ * P) void k_fz(FG g, const cplx<R>* __restrict__
     // The half-length packing pairs point k = t + P m with LZ - k.  The line's points go to
     // Z[0..LZ) (plain order) with Z[LZ] = the k = N3/2 coefficient (inverse) or point 0 (forward,
     // period LZ), so every lane reads its mirror at Z[LZ - t - P m] with no lane-0 special case.
-    cplx<R> twk[E];   // W_N3^(t + P m)
-#pragma unroll
-    for (int m = 0; m < E; m++) twk[m] = tws[LZ + t + P * m];
     // The state is 2/3-dealiased (th_state_create refuses other plans): a line holds kz < NKZ = N3/3, so
     // register m (points k = t + P m) is zero for every lane when P m >= NKZ, and its mirror LZ - k is
     // zero for every lane when LZ - (P - 1) - P m >= NKZ (LZ itself, the kz = N3/2 coefficient, included).
@@ -235,41 +215,44 @@ __global__ __launch_bounds__(TZ * P) void k_fz(FG g, const cplx<R>* __restrict__
     auto zin = [](int m) constexpr { return P * m >= NKZ; };
     auto zmir = [](int m) constexpr { return LZ - (P - 1) - P * m >= NKZ; };
     static_assert(LZ - (P - 1) >= NKZ, "register 0's mirrors (position LZ included) must be dealiased zeros");
-    cplx<R> u[ZP::NIN][E];
-#pragma unroll
-    for (int a = 0; a < ZP::NIN; a++) {
+    // Input line a: its kept modes (issued early: a load behind a product's stores would wait for them, vector-memory
+    // operations retire through one in-order counter) ...
+    auto load = [&](int a, cplx<R> (&xa)[E]) {
         const cplx<R>* X = B + a * g.cB + off;
-        cplx<R> xa[E];
 #pragma unroll
         for (int m = 0; m < E; m++) {
             const int k = t + P * m;
             xa[m] = (!zin(m) && ok && k < NKZ) ? ld_nt(X + k) : czero<R>();
         }
+    };
+    // ... and the real line: c2r packing and half-length FFT
+    auto inverse = [&](cplx<R> (&xa)[E], cplx<R> (&u)[E]) {
         wave_sync();
         // every position is written (the zeros too): mixed registers read mirrors up to LZ - NKZ + P
 #pragma unroll
         for (int m = 0; m < E; m++) Z[t + P * m] = xa[m];
         wave_sync();
+        const cplx<R>* tw = tws + opaque_zero();   // re-read per line: no registers held between lines
 #pragma unroll
         for (int m = 0; m < E; m++) {
-            cplx<R> w = conjg(twk[m]);
+            cplx<R> w = conjg(tw[LZ + t + P * m]);
             if (zmir(m)) {                    // s = d = x_k
                 cplx<R> xv = xa[m];
                 if (t == 0 && m == 0) xv.y = R(0);
-                u[a][zreg<E, FI::R0>(m)] = add_iwd(xv, w, xv);
+                u[zreg<E, FI::R0>(m)] = add_iwd(xv, w, xv);
             } else if (zin(m)) {              // s = conj(x_{LZ-k}), d = -s
                 cplx<R> xb = conjg(Z[LZ - t - P * m]);
-                u[a][zreg<E, FI::R0>(m)] = add_iwd(xb, mk<R>(-w.x, -w.y), xb);
+                u[zreg<E, FI::R0>(m)] = add_iwd(xb, mk<R>(-w.x, -w.y), xb);
             } else {
                 cplx<R> xb = Z[LZ - t - P * m];
                 cplx<R> xv = xa[m];
                 xb.y = -xb.y;
                 cplx<R> s = xv + xb, d = xv - xb;
-                u[a][zreg<E, FI::R0>(m)] = add_iwd(s, w, d);
+                u[zreg<E, FI::R0>(m)] = add_iwd(s, w, d);
             }
         }
-        FI::template run<1, true, Lay>(u[a], Z, t, tws);
-    }
+        FI::template run<1, true, Lay>(u, Z, t, tw);
+    };
     // One product line: forward half-length FFT, r2c unpacking, store of the kept kz.
     auto product_out = [&](cplx<R> (&w)[E], int p) {
         if constexpr (FI::R0 != FI::RL) {
@@ -301,82 +284,98 @@ __global__ __launch_bounds__(TZ * P) void k_fz(FG g, const cplx<R>* __restrict__
             return add_iwd(zk + zc, mk<R>(-tw.x, -tw.y), zk - zc);
         };
         // registers whose points all lie at kz >= NKZ are neither unpacked nor stored
-        if constexpr (sizeof(R) == 4) {
-            // unpack every point first, then store: no LDS read waits between the stores
-            cplx<R> o[E];
+        // unpack every point first (in place), then store: no LDS read waits between the stores
 #pragma unroll
-            for (int m = 0; m < E; m++)
-                if (!zin(m)) o[m] = unpack(m);
+        for (int m = 0; m < E; m++)
+            if (!zin(m)) w[zreg<E, FF::RL>(m)] = unpack(m);
 #pragma unroll
-            for (int m = 0; m < E; m++) {
-                const int k = t + P * m;
-                if (!zin(m) && ok && k < NKZ) st_nt(X + k, o[m]);
-            }
-        } else {
-            // FP64: holding every unpacked point would cost 4 E VGPRs
-#pragma unroll
-            for (int m = 0; m < E; m++) {
-                if (zin(m)) continue;
-                const int k = t + P * m;
-                const cplx<R> o = unpack(m);
-                if (ok && k < NKZ) st_nt(X + k, o);
-            }
+        for (int m = 0; m < E; m++) {
+            const int k = t + P * m;
+            if (!zin(m) && ok && k < NKZ) st_nt(X + k, w[zreg<E, FF::RL>(m)]);
         }
     };
-    if constexpr (sizeof(R) == 4 && E <= 8) {
-        // FP32, 8 or fewer points per thread: a rolled loop over the 3 rotation steps (fewer live
-        // registers than the unrolled form below: more waves per SIMD); rotating the group's registers
-        // by one between steps puts every operand in a fixed register, so no per-product selects.
-        constexpr int G0 = ZP::G0;
+    // The products in an order that keeps few real lines live; rolled loops, so every operand is a fixed register.
+    // Holding all inputs took 256 VGPRs and the accumulation registers (one wave per SIMD, spills in FP64 MHD) on the
+    // FP64 and the 3 2^a lines, and two waves in FP32 MHD; now two to five waves and no spill.  z pass, us, before /
+    // after: 192^3 FP64 NS 124 / 85, FP64 MHD 239 / 179, 256^3 FP64 MHD 427 / 287, FP32 MHD 190 / 160, FP32 RB
+    // 136 / 132, 192^3 FP32 NS 62 / 52 (the radix-12 schedules among it); 512^3 FP32 NS 0.68 / 0.69 ms.
+    cplx<R> xa[E], x[E], w[E];
+    auto mul = [&](cplx<R> (&o)[E], const cplx<R> (&p)[E], const cplx<R> (&q)[E]) {
+#pragma unroll
+        for (int i = 0; i < E; i++) o[i] = mk<R>(p[i].x * q[i].x, p[i].y * q[i].y);
+    };
+    if constexpr (MODE == 0 || MODE == 3) {
+        // step r: u_r u_r, (u_r T,) u_r u_{r+1}, then u_{r+1} moves on; u_0 is held for the last product (transforming
+        // it again instead costs more than the wave it gains: 512^3 FP32 step 10.33 against 10.02 ms)
+        cplx<R> tl[MODE == 3 ? E : 1];
+        if constexpr (MODE == 3) {
+            load(3, xa);
+            inverse(xa, tl);
+        }
+        load(0, xa);
+        inverse(xa, x);
+        load(1, xa);
+        cplx<R> u0[E];
+#pragma unroll
+        for (int i = 0; i < E; i++) u0[i] = x[i];
 #pragma unroll 1
         for (int r = 0; r < 3; r++) {
-#pragma unroll
-            for (int j = 0; j < ZP::NPR; j++) {
-                const int yo = ZP::yop(j);
-                cplx<R> w[E];
-#pragma unroll
-                for (int i = 0; i < E; i++) {
-                    const cplx<R> x = u[G0][i];
-                    const cplx<R> y = yo < 0 ? u[G0 - 1 - yo][i] : u[yo][i];
-                    w[i] = mk<R>(x.x * y.x, x.y * y.y);
-                }
-                product_out(w, ZP::pout(r, j));
+            mul(w, x, x);
+            product_out(w, r);
+            if constexpr (MODE == 3) {
+                mul(w, x, tl);
+                product_out(w, 6 + r);
             }
+            cplx<R> y[E];
+            if (r < 2) {
+                inverse(xa, y);
+                if (r == 0) load(2, xa);
+            } else {
 #pragma unroll
-            for (int i = 0; i < E; i++) {
-                const cplx<R> t0 = u[G0][i];
-                u[G0][i] = u[G0 + 1][i];
-                u[G0 + 1][i] = u[G0 + 2][i];
-                u[G0 + 2][i] = t0;
+                for (int i = 0; i < E; i++) y[i] = u0[i];
             }
+            mul(w, x, y);
+#pragma unroll
+            for (int i = 0; i < E; i++) x[i] = y[i];
+            product_out(w, 3 + r);
         }
-    } else if constexpr (sizeof(R) == 4) {
-        // FP32: products one after another, each fenced off for the scheduler, so that the compiler
-        // neither interleaves products nor holds two products' lines and twiddles at once (registers,
-        // occupancy); every operand is a compile-time register.
-        constexpr int G0 = ZP::G0;
-#pragma unroll
+    } else if constexpr (ZHELD<R, E>) {
+        // second operands held: 3 + 3 transforms
+        constexpr int X0 = MODE == 1 ? 0 : 3, Y0 = 3 - X0;
+        cplx<R> y0[E], y1[E], y2[E];
+        load(Y0, xa);
+        inverse(xa, y0);
+        load(Y0 + 1, xa);
+        inverse(xa, y1);
+        load(Y0 + 2, xa);
+        inverse(xa, y2);
+        load(X0, xa);
+#pragma unroll 1
         for (int r = 0; r < 3; r++) {
-#pragma unroll
-            for (int j = 0; j < ZP::NPR; j++) {
-                const int yo = ZP::yop(j);
-                const int xi = G0 + r, yi = yo < 0 ? G0 + (r - 1 - yo) % 3 : yo;
-                cplx<R> w[E];
-#pragma unroll
-                for (int i = 0; i < E; i++) w[i] = mk<R>(u[xi][i].x * u[yi][i].x, u[xi][i].y * u[yi][i].y);
-                product_out(w, ZP::pout(r, j));
-                __builtin_amdgcn_sched_barrier(0);
-            }
+            inverse(xa, x);
+            if (r < 2) load(X0 + r + 1, xa);
+            mul(w, x, y0);
+            product_out(w, 3 * r);
+            mul(w, x, y1);
+            product_out(w, 3 * r + 1);
+            mul(w, x, y2);
+            product_out(w, 3 * r + 2);
         }
     } else {
-        // FP64: selects over the arrays would become dynamic indexing (scratch); unroll instead
-#pragma unroll
-        for (int p = 0; p < ZP::NOUT; p++) {
-            const int ia = ZP::a(p), ib = ZP::b(p);
-            cplx<R> w[E];
-#pragma unroll
-            for (int i = 0; i < E; i++) w[i] = mk<R>(u[ia][i].x * u[ib][i].x, u[ia][i].y * u[ib][i].y);
-            product_out(w, p);
+        // second operands transformed again for each first one: 3 + 9 transforms, two lines live
+        constexpr int X0 = MODE == 1 ? 0 : 3, Y0 = 3 - X0;
+        load(X0, xa);
+#pragma unroll 1
+        for (int q = 0; q < 9; q++) {
+            const int r = q / 3, j = q - 3 * r;
+            if (j == 0) {
+                inverse(xa, x);
+                load(Y0, xa);
+            }
+            inverse(xa, w);
+            if (q < 8) load(j == 2 ? X0 + r + 1 : Y0 + j + 1, xa);
+            mul(w, x, w);
+            product_out(w, q);
         }
     }
 }
