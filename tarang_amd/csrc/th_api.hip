@@ -4,6 +4,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 #include <string.h>
+#include <algorithm>
 #include <new>
 #include <vector>
 #include "../../include/tarang_hip.h"
@@ -190,6 +191,7 @@ th_plan::~th_plan()
     tw.release();
     rs.release();
     if (radii_dev) (void)hipFree(radii_dev);
+    plain.release();
     release_fused(this);
 }
 
@@ -826,6 +828,27 @@ extern "C" int th_et_nlin(th_plan* p, void* const H[3], void* const G[3], void* 
     return DISPATCH(p, do_et_nlin, p, H, G, nlin);
 }
 
+// Whether a step runs through the fused passes (th_plain.hpp): a dealiased plan whose lengths those passes have, and a
+// force that lives on kept modes only.  (SCFT N1 = 384 stays refused, as by the array transforms.)  Everything else
+// takes the operation sequence above.
+static bool plain_fast(const th_plan* p, int physics, const ForceBand* b)
+{
+    auto len = [](int n) {
+        for (int v : {16, 24, 32, 48, 64, 96, 128, 192, 256, 384, 512})
+            if (v == n) return true;
+        return false;
+    };
+    const Geo& g = p->g;
+    if (!g.dealias || !len(g.N1) || !len(g.N2) || !len(g.N3)) return false;
+    if ((physics == TH_RB) != (g.basis == TH_SCFT) || (g.basis == TH_SCFT && g.N1 == 384)) return false;
+    if (!b || b->proc == 3 || b->proc == 4) return true;      // their modes are kept ones (force_setup)
+    // every wavevector of the band's ball is kept: |k| below the shortest kept half-range of each axis (the kept ky of
+    // lengths 3 2^a reach less far on the negative side)
+    const int hx = g.N1 / 3 - 1, hy = g.N2 - (2 * g.N2 / 3 + 2), hz = g.N3 / 3 - 1;
+    const int ly = std::min(hy, g.N2 / 3 - 1);
+    return b->outer < (hx + 1) * fabs(g.kf[0]) && b->outer < (ly + 1) * fabs(g.kf[1]) && b->outer < (hz + 1) * fabs(g.kf[2]);
+}
+
 template <typename R> static int do_step_plain(th_plan* p, int physics, int scheme, void* const fields[], double dt,
                                                const th_phys* ph)
 {
@@ -836,6 +859,11 @@ template <typename R> static int do_step_plain(th_plan* p, int physics, int sche
     if (physics == TH_RB && ph->Ra > 0 && ph->Pr > 0) {
         nu = sqrt(ph->Pr / ph->Ra);
         kap = 1 / sqrt(ph->Pr * ph->Ra);
+    }
+    if (plain_fast(p, physics, nullptr)) {
+        cplx<R>* F[6] = {};
+        for (int q = 0; q < o.nc; q++) F[q] = CP(R, fields[q]);
+        return plain_step<R>(p, physics, scheme, F, dt, nu, physics == TH_MHD ? eta : kap, nullptr, nullptr, nullptr);
     }
     for (int q = 0; q < o.nc; q++) {
         o.F[q] = CP(R, fields[q]);
@@ -862,6 +890,10 @@ template <typename R> static int do_step_plain_forced(th_plan* p, int scheme, vo
     o.force = fb;
     if (last)
         for (int c = 0; c < 3; c++) o.keep[c] = CP(R, last[c]);
+    if (plain_fast(p, TH_NS, fb)) {
+        cplx<R>* F[3] = {CP(R, V[0]), CP(R, V[1]), CP(R, V[2])};
+        return plain_step<R>(p, TH_NS, scheme, F, dt, ph->nu, 0.0, fb, nullptr, o.keep);
+    }
     for (int q = 0; q < 3; q++) {
         o.F[q] = CP(R, V[q]);
         o.N[q] = o.S(SC_N0 + q);
@@ -881,6 +913,13 @@ template <typename R> static int do_step_plain_forced_mhd(th_plan* p, int scheme
     o.force_w = fw;
     if (last)
         for (int c = 0; c < 6; c++) o.keep[c] = CP(R, last[c]);
+    if (plain_fast(p, TH_MHD, fu)) {
+        cplx<R>* F[6];
+        for (int q = 0; q < 6; q++) F[q] = CP(R, q < 3 ? U[q] : B[q - 3]);
+        // each part only when its level per mode exceeds MYEPS (compute_rhs above)
+        const bool u = fu->proc == 3 || fu->per_mode > 1e-15, w = fw->proc == 3 || fw->per_mode > 1e-15;
+        return plain_step<R>(p, TH_MHD, scheme, F, dt, ph->nu, ph->eta, u ? fu : nullptr, w ? fw : nullptr, o.keep);
+    }
     for (int q = 0; q < 6; q++) {
         o.F[q] = CP(R, q < 3 ? U[q] : B[q - 3]);
         o.N[q] = o.S(SC_N0 + q);

@@ -72,6 +72,49 @@ FG make_fg(const Geo& geo, int prec)
 
 using namespace th;
 
+int PlainBufs::ensure(size_t esz, size_t nX, size_t nY, size_t nC, size_t nF, hipStream_t st)
+{
+    auto grow = [&](void** q, size_t bytes, bool clear) -> int {
+        if (*q) TH_CHECK_HIP(hipFree(*q));       // (waits for the launches that still read it)
+        *q = nullptr;
+        if (hipMalloc(q, bytes) != hipSuccess) {
+            *q = nullptr;
+            set_error("plain step: workspace allocation of %zu bytes failed", bytes);
+            return E_NOMEM;
+        }
+        if (clear) TH_CHECK_HIP(hipMemsetAsync(*q, 0, bytes, st));
+        return OK;
+    };
+    if (nX * esz > bX) { bX = 0; TRY(grow(&X, nX * esz, true)); bX = nX * esz; }
+    if (nY * esz > bY) { bY = 0; TRY(grow(&Y, nY * esz, true)); bY = nY * esz; }
+    if (nC * esz > bC) {
+        bC = 0;
+        TRY(grow(&rhs, nC * esz, true));
+        TRY(grow(&acc, nC * esz, true));
+        TRY(grow(&zero, nC * esz, true));
+        TRY(grow(&junk, nC * esz, true));
+        bC = nC * esz;
+    }
+    if (nF * esz > bF) { bF = 0; TRY(grow(&Fs, nF * esz, false)); bF = nF * esz; }
+    if (!coef) {
+        StageCoef c;
+        memset(&c, 0, sizeof c);
+        c.stage = 1;
+        c.dt = 2.0;
+        TRY(grow(&coef, sizeof c, false));
+        TH_CHECK_HIP(hipMemcpy(coef, &c, sizeof c, hipMemcpyHostToDevice));
+    }
+    return OK;
+}
+void PlainBufs::release()
+{
+    for (void** q : {&X, &Y, &rhs, &acc, &zero, &junk, &Fs, &coef}) {
+        if (*q) (void)hipFree(*q);
+        *q = nullptr;
+    }
+    bX = bY = bC = bF = 0;
+}
+
 struct th_state {
     th_plan* plan = nullptr;
     int physics = TH_NS;

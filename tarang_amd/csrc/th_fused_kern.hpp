@@ -177,7 +177,9 @@ template <int E, int Rr> __device__ __forceinline__ constexpr int zreg(int m)
 // the FP64 lines with 12 points per thread, are transformed again for each first operand (held, they would spill)
 template <typename R, int E> constexpr bool ZHELD = sizeof(R) == 4 || E <= 8;
 
-template <typename R, int LZ, int P, int TZ, int MODE>
+// FULL (the plain steppers): input lines hold every kz <= N3/2 (component and line strides g.cBi, g.KZPi) instead of the
+// dealiased ones.
+template <typename R, int LZ, int P, int TZ, int MODE, bool FULL = false>
 __global__ __launch_bounds__(TZ * P) void k_fz(FG g, const cplx<R>* __restrict__ B, cplx<R>* __restrict__ Cout,
                                                const cplx<R>* __restrict__ twL, const cplx<R>* __restrict__ twN)
 {
@@ -214,38 +216,48 @@ __global__ __launch_bounds__(TZ * P) void k_fz(FG g, const cplx<R>* __restrict__
     constexpr int NKZ = (2 * LZ) / 3;
     auto zin = [](int m) constexpr { return P * m >= NKZ; };
     auto zmir = [](int m) constexpr { return LZ - (P - 1) - P * m >= NKZ; };
-    static_assert(LZ - (P - 1) >= NKZ, "register 0's mirrors (position LZ included) must be dealiased zeros");
+    static_assert(FULL || LZ - (P - 1) >= NKZ, "register 0's mirrors (position LZ included) must be dealiased zeros");
+    constexpr int XE = E + (FULL ? 1 : 0);   // FULL: the line's kz = N3/2 coefficient too (lane 0)
     // Input line a: its kept modes (issued early: a load behind a product's stores would wait for them, vector-memory
     // operations retire through one in-order counter) ...
-    auto load = [&](int a, cplx<R> (&xa)[E]) {
-        const cplx<R>* X = B + a * g.cB + off;
+    auto load = [&](int a, cplx<R> (&xa)[XE]) {
+        if constexpr (FULL) {
+            const cplx<R>* X = B + a * g.cBi + q * g.KZPi;
 #pragma unroll
-        for (int m = 0; m < E; m++) {
-            const int k = t + P * m;
-            xa[m] = (!zin(m) && ok && k < NKZ) ? ld_nt(X + k) : czero<R>();
+            for (int m = 0; m < E; m++) xa[m] = ok ? ld_nt(X + t + P * m) : czero<R>();
+            xa[E] = (ok && t == 0) ? X[LZ] : czero<R>();
+        } else {
+            const cplx<R>* X = B + a * g.cB + off;
+#pragma unroll
+            for (int m = 0; m < E; m++) {
+                const int k = t + P * m;
+                xa[m] = (!zin(m) && ok && k < NKZ) ? ld_nt(X + k) : czero<R>();
+            }
         }
     };
     // ... and the real line: c2r packing and half-length FFT
-    auto inverse = [&](cplx<R> (&xa)[E], cplx<R> (&u)[E]) {
+    auto inverse = [&](cplx<R> (&xa)[XE], cplx<R> (&u)[E]) {
         wave_sync();
         // every position is written (the zeros too): mixed registers read mirrors up to LZ - NKZ + P
 #pragma unroll
         for (int m = 0; m < E; m++) Z[t + P * m] = xa[m];
+        if (FULL && t == 0) Z[LZ] = xa[XE - 1];
         wave_sync();
         const cplx<R>* tw = tws + opaque_zero();   // re-read per line: no registers held between lines
 #pragma unroll
         for (int m = 0; m < E; m++) {
             cplx<R> w = conjg(tw[LZ + t + P * m]);
-            if (zmir(m)) {                    // s = d = x_k
+            if (!FULL && zmir(m)) {           // s = d = x_k
                 cplx<R> xv = xa[m];
                 if (t == 0 && m == 0) xv.y = R(0);
                 u[zreg<E, FI::R0>(m)] = add_iwd(xv, w, xv);
-            } else if (zin(m)) {              // s = conj(x_{LZ-k}), d = -s
+            } else if (!FULL && zin(m)) {     // s = conj(x_{LZ-k}), d = -s
                 cplx<R> xb = conjg(Z[LZ - t - P * m]);
                 u[zreg<E, FI::R0>(m)] = add_iwd(xb, mk<R>(-w.x, -w.y), xb);
             } else {
                 cplx<R> xb = Z[LZ - t - P * m];
                 cplx<R> xv = xa[m];
+                if (FULL && t == 0 && m == 0) xv.y = xb.y = R(0);   // FFTW's c2r ignores Im of kz = 0 and N3/2
                 xb.y = -xb.y;
                 cplx<R> s = xv + xb, d = xv - xb;
                 u[zreg<E, FI::R0>(m)] = add_iwd(s, w, d);
@@ -299,7 +311,7 @@ __global__ __launch_bounds__(TZ * P) void k_fz(FG g, const cplx<R>* __restrict__
     // FP64 and the 3 2^a lines, and two waves in FP32 MHD; now two to five waves and no spill.  z pass, us, before /
     // after: 192^3 FP64 NS 124 / 85, FP64 MHD 239 / 179, 256^3 FP64 MHD 427 / 287, FP32 MHD 190 / 160, FP32 RB
     // 136 / 132, 192^3 FP32 NS 62 / 52 (the radix-12 schedules among it); 512^3 FP32 NS 0.68 / 0.69 ms.
-    cplx<R> xa[E], x[E], w[E];
+    cplx<R> xa[XE], x[E], w[E];
     auto mul = [&](cplx<R> (&o)[E], const cplx<R> (&p)[E], const cplx<R> (&q)[E]) {
 #pragma unroll
         for (int i = 0; i < E; i++) o[i] = mk<R>(p[i].x * q[i].x, p[i].y * q[i].y);
@@ -1125,7 +1137,7 @@ static int launch_yinv(const FG& g, const cplx<R>* A, cplx<R>* B, int ncomp, con
     TH_CHECK_HIP(hipGetLastError());
     return OK;
 }
-template <typename R, int LZ, int MODE, int V>
+template <typename R, int LZ, int MODE, int V, bool FULL = false>
 static int launch_z(const FG& g, const cplx<R>* B, cplx<R>* Cc, const cplx<R>* twL, const cplx<R>* twN, hipStream_t st)
 {
     constexpr int E = (V == 3) ? 16 : pts_per_thread(LZ), P = LZ / E;
@@ -1136,7 +1148,7 @@ static int launch_z(const FG& g, const cplx<R>* B, cplx<R>* Cc, const cplx<R>* t
         return E_UNSUPPORTED;
     }
     const long lines = (long)g.N1 * g.N2;
-    hipLaunchKernelGGL((k_fz<R, LZ, P, TZ, MODE>), dim3((unsigned)((lines + TZ - 1) / TZ), g.nbox), dim3(TZ * P), 0, st, g, B, Cc,
+    hipLaunchKernelGGL((k_fz<R, LZ, P, TZ, MODE, FULL>), dim3((unsigned)((lines + TZ - 1) / TZ), g.nbox), dim3(TZ * P), 0, st, g, B, Cc,
                        twL, twN);
     TH_CHECK_HIP(hipGetLastError());
     return OK;

@@ -24,6 +24,15 @@ enum {
     SC_FW0 = 43,     // W.Force1..3 (forced MHD) 43..45
 };
 struct Fused;        // dealias-pruned pipeline (th_fused.hip)
+
+// Workspace of the plain steppers (th_plain.hpp), kept in the plan and grown to the largest physics it has stepped
+struct PlainBufs {
+    void *X = nullptr, *Y = nullptr, *rhs = nullptr, *acc = nullptr, *zero = nullptr, *junk = nullptr, *Fs = nullptr;
+    void* coef = nullptr;
+    size_t bX = 0, bY = 0, bC = 0, bF = 0;
+    int ensure(size_t esz, size_t X, size_t Y, size_t C, size_t Fs, hipStream_t st);
+    void release();
+};
 }  // namespace th
 
 struct th_plan {
@@ -36,6 +45,7 @@ struct th_plan {
     double* radii_dev = nullptr;
     int radii_cap = 0;
     th::Fused* fused = nullptr;
+    th::PlainBufs plain;
     int nstates = 0;                 // fused states created on this plan and not yet destroyed
     bool dead = false;               // th_plan_destroy called while states were alive
     void* scr(int i);
@@ -48,4 +58,7 @@ void release_fused(th_plan* p);
 void plan_free(th_plan* p);           // waits for the plan's stream, frees it, uncounts it in its context
 template <typename R> int plain_forward(th_plan* p, cplx<R>* A, int parity);
 template <typename R> int plain_inverse(th_plan* p, cplx<R>* A, int parity);
+// The plain steppers through the fused passes (th_plain.hpp)
+template <typename R> int plain_step(th_plan* p, int physics, int scheme, cplx<R>* const* F, double dt, double d0, double d1,
+                                     const ForceBand* fu, const ForceBand* fw, cplx<R>* const* keep);
 }  // namespace th
