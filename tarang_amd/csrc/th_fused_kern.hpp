@@ -572,14 +572,29 @@ __global__ __launch_bounds__(T * P) __attribute__((amdgpu_waves_per_eu((MODE == 
     // (!ok) still lies inside its row, so the loads are unconditional: such a column's values only ever reach its
     // own lines, which are never stored.  Wider tiles (short lines) keep the guard.
     constexpr bool PADOK = (sizeof(R) == 4 ? 16 : 8) % T == 0;
-#pragma unroll 1
-    for (int p = 0; p < NP; p++) {
-        cplx<R> v[E];
+    auto load = [&](int p, cplx<R> (&v)[E]) {
         const cplx<R>* src = D + p * g.cA + mu;
 #pragma unroll
         for (int i = 0; i < E; i++) {
             const cplx<R>* row = src + (long)F::in_pos(0, i) * g.sx;
             v[i] = (PADOK || ok) ? *at_byte(row, lane_b) : czero<R>();
+        }
+    };
+    // The next product's loads are issued before this one's transform where that costs no wave per SIMD (XPRE): FP32
+    // MHD and FP64 NS with 8 points per thread, chained FP32 NS on the long 3 2^a lines.  us, before / after: 256^3 FP32
+    // MHD 227 / 210, 384^3 FP32 NS 470 / 443, 128^3 FP64 NS 30.2 / 27.8; RB (k_sx_fwd_rb) 256^3 FP32 207 / 165.
+    constexpr bool XPRE = sizeof(R) == 4 ? (MODE == 1 && E == 8) || (CHAIN && L % 3 == 0 && L >= 192) : MODE == 0 && E == 8;
+    cplx<R> nv[XPRE ? E : 1];
+    if constexpr (XPRE) load(0, nv);
+#pragma unroll 1
+    for (int p = 0; p < NP; p++) {
+        cplx<R> v[E];
+        if constexpr (XPRE) {
+#pragma unroll
+            for (int i = 0; i < E; i++) v[i] = nv[i];
+            if (p + 1 < NP) load(p + 1, nv);
+        } else {
+            load(p, v);
         }
         F::template run<T, false, NoPad, true>(v, lds + c, t, twl + opaque_zero());
         // contributions (a1 <- K_k1) and (a2 <- K_k2) of product p; k = 0 means Kx (per row)
@@ -873,20 +888,31 @@ __global__ __launch_bounds__(T * P) void k_sx_fwd_rb(FG g, const cplx<R>* __rest
         for (int i = 0; i < E; i++) Nacc[a][i] = czero<R>();
     const long mu = (long)cy * g.KZP + (long)(tile % ntz) * T;
     const int lane_off = c + t * (int)g.sx;
+    auto load = [&](int p, cplx<R> (&v)[E]) {
+        const cplx<R>* src = D + p * g.cA + mu;
+#pragma unroll
+        for (int i = 0; i < E; i++) {
+            const cplx<R>* row = src + (long)F::in_pos(0, i) * g.sx;
+            v[i] = ok ? row[lane_off] : czero<R>();
+        }
+    };
+    // FP32: the next product's tile is loaded before this one's transform (no wave per SIMD is lost to it)
+    constexpr bool XPRE = sizeof(R) == 4;
+    cplx<R> nv[E];
+    if constexpr (XPRE) load(0, nv);
 #pragma unroll 1
     for (int p = 0; p < 9; p++) {
         // forward kind of product p: sine for V1V2 (3), V3V1 (5), V2T (7), V3T (8)
         const bool psin = ((0x1A8u >> p) & 1u) != 0;
         cplx<R> v[E];
-        const cplx<R>* src = D + p * g.cA + mu;
+        if constexpr (!XPRE) load(p, nv);
 #pragma unroll
         for (int i = 0; i < E; i++) {
-            const int j0 = F::in_pos(0, i);
-            const cplx<R>* row = src + (long)j0 * g.sx;
-            const cplx<R> x = ok ? row[lane_off] : czero<R>();
-            const R sg = (psin && j0 + t >= L / 2) ? R(-1) : R(1);
-            v[i] = cscale(x, sg);
+            const R sg = (psin && F::in_pos(0, i) + t >= L / 2) ? R(-1) : R(1);
+            v[i] = cscale(nv[i], sg);
         }
+        if constexpr (XPRE)
+            if (p < 8) load(p + 1, nv);
         F::template run<T, false, NoPad, true, 1>(v, lds + c, t, twl + opaque_zero());
         if constexpr (F::NST < 2) __syncthreads();    // no exchange: the previous product's mirror reads
 #pragma unroll
@@ -1023,12 +1049,25 @@ __global__ __launch_bounds__(T * P) void k_fx_fwd_et(FG g, const cplx<R>* __rest
     for (int a = 0; a < 3; a++)
 #pragma unroll
         for (int i = 0; i < E; i++) Nacc[a][i] = czero<R>();
-#pragma unroll 1
-    for (int p = 0; p < 9; p++) {
-        cplx<R> v[E];
+    auto load = [&](int p, cplx<R> (&v)[E]) {
         const cplx<R>* src = D + p * g.cA + m;
 #pragma unroll
         for (int i = 0; i < E; i++) v[i] = ok ? src[(long)F::in_pos(t, i) * g.sx] : czero<R>();
+    };
+    // the next product's tile is loaded before this one's transform where that costs no wave per SIMD
+    constexpr bool XPRE = (sizeof(R) == 8) == (E == 8);
+    cplx<R> nv[E];
+    if constexpr (XPRE) load(0, nv);
+#pragma unroll 1
+    for (int p = 0; p < 9; p++) {
+        cplx<R> v[E];
+        if constexpr (XPRE) {
+#pragma unroll
+            for (int i = 0; i < E; i++) v[i] = nv[i];
+            if (p < 8) load(p + 1, nv);
+        } else {
+            load(p, v);
+        }
         F::template run<T, false, NoPad, true>(v, lds + c, t, twl + opaque_zero());
         const int pi = p / 3, pj = p % 3;        // P(pi,pj) = G_pi H_pj -> N_pi += i K_pj P
         R al[3], be[3];
@@ -1223,8 +1262,8 @@ static int launch_sxinv(const FG& g, const cplx<R>* S, cplx<R>* A, const cplx<R>
     TH_CHECK_HIP(hipGetLastError());
     return OK;
 }
-// variant 1: half-width tiles (more, smaller workgroups: less idle tail at 256^3, where full tiles leave
-// 1026 workgroups for 256 CUs holding one each)
+// variant 1: half-width tiles (more, smaller workgroups; full tiles are the faster ones since the next product's
+// tile is loaded ahead, 165 against 179 us at 256^3 FP32)
 template <typename R, int L, int V>
 static int launch_sxfwd(const FG& g, const cplx<R>* D, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw,
                         const cplx<R>* tw4, const StageCoef* sc, hipStream_t st)
