@@ -854,7 +854,7 @@ static int et_shell_rows(th_state* s, const double* radii, int nsh, int ngiv, in
     TH_CHECK_HIP(hipMemcpyAsync(s->radii, radii, nr * sizeof(double), hipMemcpyHostToDevice, st));
     int nblk = 0;
     TRY(d_xfwd_et<R>(g, X1, S, twx, s->radii, nr, 0, nullptr, &nblk, st));
-    size_t need = (size_t)nblk * (2 * nr) + (2 * nr);
+    size_t need = (size_t)nblk * (2 * nr) + (size_t)ngiv * nrecv * (2 * nr);
     if (need > s->partial_cap) {
         if (s->partial) (void)hipFree(s->partial);
         s->partial = nullptr;
@@ -867,11 +867,11 @@ static int et_shell_rows(th_state* s, const double* radii, int nsh, int ngiv, in
     TRY((d_xinv<R, 0>(g, S + (long)hoff * g.cS, X1, 3, twx, all, 0, st)));
     // the y passes take the step's tuned launch shapes (the same kernels, any component count)
     TRY(d_yinv<R>(g, X1, X2, 3, twy, s->var[PASS_YINV], st));
-    std::vector<double> hostbuf(2 * nr);
     for (int r = 0; r < nrecv; r++) {
         Yb[r].assign((size_t)(ngiv + 1) * nr, 0.0);
         Yc[r].assign((size_t)(ngiv + 1) * nr, 0.0);
     }
+    // the sums of every giver and receiver stay on the device until the last one is done
     double* outd = s->partial + (size_t)nblk * (2 * nr);
     for (int n = 1; n <= ngiv; n++) {
         ShellSel sel{radii[n - 1], radii[n]};
@@ -881,16 +881,21 @@ static int et_shell_rows(th_state* s, const double* radii, int nsh, int ngiv, in
         TRY(d_yfwd<R>(g, X3, X1, 9, twy, s->var[PASS_YFWD], st));
         for (int r = 0; r < nrecv; r++) {
             TRY(d_xfwd_et<R>(g, X1, S + (long)roff[r] * g.cS, twx, s->radii, nr, kin, s->partial, &nblk, st));
-            launch_finalize((const double*)s->partial, nblk, 2 * nr, 2 * nr, outd, st);
+            launch_finalize((const double*)s->partial, nblk, 2 * nr, 2 * nr, outd + ((size_t)(n - 1) * nrecv + r) * 2 * nr, st);
             TH_CHECK_HIP(hipGetLastError());
-            TH_CHECK_HIP(hipMemcpyAsync(hostbuf.data(), outd, 2 * nr * sizeof(double), hipMemcpyDeviceToHost, st));
-            TH_CHECK_HIP(hipStreamSynchronize(st));
-            for (int m = 0; m < nr; m++) {
-                Yb[r][(size_t)n * nr + m] = hostbuf[m];
-                Yc[r][(size_t)n * nr + m] = hostbuf[nr + m];
-            }
         }
     }
+    std::vector<double> hostbuf((size_t)ngiv * nrecv * 2 * nr);
+    TH_CHECK_HIP(hipMemcpyAsync(hostbuf.data(), outd, hostbuf.size() * sizeof(double), hipMemcpyDeviceToHost, st));
+    TH_CHECK_HIP(hipStreamSynchronize(st));
+    for (int n = 1; n <= ngiv; n++)
+        for (int r = 0; r < nrecv; r++) {
+            const double* h = &hostbuf[((size_t)(n - 1) * nrecv + r) * 2 * nr];
+            for (int m = 0; m < nr; m++) {
+                Yb[r][(size_t)n * nr + m] = h[m];
+                Yc[r][(size_t)n * nr + m] = h[nr + m];
+            }
+        }
     return OK;
 }
 
