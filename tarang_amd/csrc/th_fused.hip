@@ -486,75 +486,69 @@ static void diss_of(const th_state* s, const th_phys* ph, double* d0, double* d1
 // rhs gains +P(F), P the projection.  Every stage output (the stage field, the accumulator, the state
 // in stage 4) is linear in the rhs and F lives on a few thousand band modes, so instead of changing
 // the x-forward epilogue, k_force_pre stores P(F) of the stage input for the band box before the
-// stage's passes, and k_force_post adds the stage's share of it afterwards:
+// stage's passes, and k_force_out adds the stage's share of it afterwards:
 //   stage 1: Vs += dt/2 e_h P(F), acc += dt/6 e_1 P(F)      stage 2: Vs += dt/2 P(F), acc += dt/3 e_h P(F)
 //   stage 3: Vs += dt e_h P(F),   acc += dt/3 e_h P(F)      stage 4: S += dt/6 P(F)
 // with e_h = exp(-nu dt K^2 / 2), e_1 = exp(-nu dt K^2) (the integrating factors of rk_store).
-// A chained forced step writes no stage field: in stages 2-4, k_force_recon recovers the stage input's band
-// modes from the A lines (the x-inverse of that input, which the previous stage's x-forward wrote) by a direct
-// DFT along x; the x-forward has transformed the stage output without the force share into the next stage's A
-// lines, so k_force_post records the share it adds to the next stage's input (S in stage 4) per band mode, and
-// k_force_chain_fix adds its x-inverse to the A lines of the band's columns.
+// A chained forced step writes no stage field: in stages 2-4, k_force_in recovers the stage input's band modes from
+// the A lines (the x-inverse of that input, which the previous stage's x-forward wrote) by a direct DFT along x, and
+// the x-forward has transformed the stage output without the force share into the next stage's A lines, so k_force_out
+// adds the x-inverse of the shares to the A lines of the band's columns.  192^3 FP32: the two launches take 13 us per
+// stage; as four (recover, project, add, correct), with the phases from sincospi, they took 25.
 // ------------------------------------------------------------------------------------------
 __host__ __device__ __forceinline__ bool fused_stored(const FG& g, int lx, int ly, int lz)
 {
     return lz < g.nkz && lkept(g.mx, lx) && lkept(g.my, ly);
 }
 
-// Chained forced step, stages 2-4: the stage input at every band mode's reality source (sx, sy, lz),
-// v_c = (1/N1) sum_x A[c][x][sy][lz] e^{-2 pi i sx x / N1}, into vbox (6 doubles per band mode; 0 where the
-// state stores no such mode).  One workgroup of 256 threads per band mode.
+// Before a stage's passes: P(F) of the stage input for every mode of the band box, into fbox (6 doubles per mode).  One
+// workgroup per mode.  The input comes from src (the state, or an unchained stage field), or, chained in stages 2-4,
+// from the A lines: v_c = (1/N1) sum_x A[c][x][sy][lz] e^{-2 pi i sx x / N1} at the mode's reality source (sx, sy, lz),
+// with the FP64 twiddle table tw (0 where the state stores no such mode).  Modes off the band end at once: the box of a
+// shell has about twice its modes.  Bound by launch latency (the band is some hundred columns of N1 points).
+constexpr int FIN_THREADS = 128;
 template <typename R>
-__global__ __launch_bounds__(256) void k_force_recon(ForceBand b, FG g, const cplx<R>* __restrict__ A,
-                                                     double* __restrict__ vbox)
+__global__ __launch_bounds__(FIN_THREADS) void k_force_in(ForceBand b, FG g, const cplx<R>* __restrict__ src,
+                                                          const cplx<R>* __restrict__ A, const c64* __restrict__ tw,
+                                                          double* __restrict__ fbox)
 {
     const long t = blockIdx.x;
     int lx, ly, lz, sx, sy;
     band_mode(b, t, lx, ly, lz);
-    (void)reality_source(b, lx, ly, lz, sx, sy);
-    __shared__ double red[6][256];
-    double acc[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    const bool st = fused_stored(g, sx, sy, lz);
-    if (st) {
-        const cplx<R>* col = A + (long)lq(g.my, sy) * g.KZP + lz;
-        for (int x = threadIdx.x; x < g.N1; x += blockDim.x) {
-            const long m = ((long)sx * x) % g.N1;   // e^{-2 pi i sx x / N1} from the exact phase index
-            double sn, cs;
-            sincospi(2.0 * (double)m / g.N1, &sn, &cs);
-            for (int c = 0; c < 3; c++) {
-                const cplx<R> a = col[c * g.cA + (long)x * g.sx];
-                acc[2 * c] += (double)a.x * cs + (double)a.y * sn;
-                acc[2 * c + 1] += (double)a.y * cs - (double)a.x * sn;
-            }
-        }
-    }
-    for (int j = 0; j < 6; j++) red[j][threadIdx.x] = acc[j];
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int j = 0; j < 6; j++) red[j][threadIdx.x] += red[j][threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x < 6) vbox[6 * t + threadIdx.x] = st ? red[threadIdx.x][0] / g.N1 : 0.0;
-}
-
-// vbox (chained stages 2-4): the stage input's band modes from k_force_recon instead of src
-template <typename R>
-__global__ void k_force_pre(ForceBand b, FG g, const cplx<R>* __restrict__ src, const double* __restrict__ vbox,
-                            double* __restrict__ fbox)
-{
-    const long n = (long)b.nx * b.ny * b.nz;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    int lx, ly, lz, sx, sy;
-    band_mode(b, t, lx, ly, lz);
     const bool mirror = reality_source(b, lx, ly, lz, sx, sy);
-    cplx<R> v[3] = {czero<R>(), czero<R>(), czero<R>()};
-    if (vbox) {
-        for (int c = 0; c < 3; c++) v[c] = mk<R>((R)vbox[6 * t + 2 * c], (R)vbox[6 * t + 2 * c + 1]);
-    } else if (fused_stored(g, sx, sy, lz)) {
+    const double ks = kmag3(kx_four(sx, b.N1) * b.f1, ky_of(sy, b.N2) * b.f2, lz * b.f3);
+    const bool stored = fused_stored(g, sx, sy, lz);
+    if (!(ks > b.inner && ks <= b.outer) || !stored) {     // mode_force is 0 there, and on a zero field
+        if (threadIdx.x < 6) fbox[6 * t + threadIdx.x] = 0.0;
+        return;
+    }
+    cplx<R> v[3];
+    if (src) {
+        if (threadIdx.x) return;
         const long i = (long)lq(g.mx, sx) * g.sx + (long)lq(g.my, sy) * g.KZP + lz;
         for (int c = 0; c < 3; c++) v[c] = src[c * g.cS + i];
+    } else {
+        __shared__ double red[FIN_THREADS / 64][6];
+        double s[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        const cplx<R>* col = A + (long)lq(g.my, sy) * g.KZP + lz;
+        for (int x = threadIdx.x; x < g.N1; x += FIN_THREADS) {
+            const c64 w = tw[(sx * x) % g.N1];             // the exact phase index
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                const cplx<R> a = col[c * g.cA + (long)x * g.sx];
+                s[2 * c] += (double)a.x * w.x - (double)a.y * w.y;
+                s[2 * c + 1] += (double)a.x * w.y + (double)a.y * w.x;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 6; j++)
+            for (int w = 32; w > 0; w >>= 1) s[j] += __shfl_xor(s[j], w);
+        if (threadIdx.x % 64 == 0)
+            for (int j = 0; j < 6; j++) red[threadIdx.x / 64][j] = s[j];
+        __syncthreads();
+        if (threadIdx.x) return;
+        for (int c = 0; c < 3; c++)
+            v[c] = mk<R>((R)((red[0][2 * c] + red[1][2 * c]) / g.N1), (R)((red[0][2 * c + 1] + red[1][2 * c + 1]) / g.N1));
     }
     double fr[3], fi[3];
     mode_force<R>(b, v, sx, sy, lz, fr, fi);
@@ -576,86 +570,62 @@ __global__ void k_force_pre(ForceBand b, FG g, const cplx<R>* __restrict__ src, 
     }
 }
 
-// chained: no stage field to update (the next stage's A lines get the share through k_force_chain_fix) except
-// the stage-3 output, which the chained x-forward keeps for a forced state
+// After a stage's passes, one workgroup per column (ty, tz) of the band box and component: the stage's share of P(F) to
+// the accumulator (the state in stage 4) and to the stage field (chained: only the kept stage-3 output, FG::keep3), and
+// in a chained step to the next stage's A lines of the column, A[x] += sum over the column's modes of
+// share e^{+2 pi i lx x / N1} (the unnormalised inverse line transform).  Columns the state does not store are left alone.
 template <typename R>
-__global__ void k_force_post(ForceBand b, FG g, const StageCoef* __restrict__ coef, cplx<R>* S, cplx<R>* Vs,
-                             cplx<R>* acc, double* __restrict__ fbox, int chained)
+__global__ __launch_bounds__(256) void k_force_out(ForceBand b, FG g, const StageCoef* __restrict__ coef, cplx<R>* S,
+                                                   cplx<R>* Vs, cplx<R>* acc, cplx<R>* A, const c64* __restrict__ tw,
+                                                   const double* __restrict__ fbox, int chained)
 {
-    const long n = (long)b.nx * b.ny * b.nz;
-    const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    double* share = fbox + 6 * n + 6 * t;   // what this stage adds to the next stage's input (0: nothing)
-    for (int j = 0; j < 6; j++) share[j] = 0.0;
-    int lx, ly, lz;
-    band_mode(b, t, lx, ly, lz);
-    if (!fused_stored(g, lx, ly, lz)) return;
-    double f[6];
-    bool any = false;
-    for (int j = 0; j < 6; j++) {
-        f[j] = fbox[6 * t + j];
-        any = any || f[j] != 0.0;
-    }
-    if (!any) return;
-    const StageCoef sc = *coef;
-    const double kx = kx_four(lx, g.N1) * g.f1, ky = ky_of(ly, g.N2) * g.f2, kz = lz * g.f3;
-    const double kx2 = ksq_f(kx, 0.0, 0.0), kyz2 = ksq_f(0.0, ky, kz);
-    const double eh = exp(sc.fh[0] * kx2) * exp(sc.fh[0] * kyz2), e1 = exp(sc.f1[0] * kx2) * exp(sc.f1[0] * kyz2);
-    double cv = 0.0, ca = 0.0;
-    if (sc.stage == 1) { cv = 0.5 * sc.dt * eh; ca = sc.dt / 6 * e1; }
-    else if (sc.stage == 2) { cv = 0.5 * sc.dt; ca = sc.dt / 3 * eh; }
-    else if (sc.stage == 3) { cv = sc.dt * eh; ca = sc.dt / 3 * eh; }
-    const long i = (long)lq(g.mx, lx) * g.sx + (long)lq(g.my, ly) * g.KZP + lz;
-    for (int c = 0; c < 3; c++) {
-        const long j = c * g.cS + i;
-        if (sc.stage < 4) {
-            if (!chained || sc.stage == 3) {   // chained: only the kept stage-3 output (FG::keep3)
-                const cplx<R> v = Vs[j];
-                Vs[j] = mk<R>((R)((double)v.x + cv * f[2 * c]), (R)((double)v.y + cv * f[2 * c + 1]));
-            }
-            const cplx<R> a = acc[j];
-            acc[j] = mk<R>((R)((double)a.x + ca * f[2 * c]), (R)((double)a.y + ca * f[2 * c + 1]));
-            share[2 * c] = cv * f[2 * c];
-            share[2 * c + 1] = cv * f[2 * c + 1];
-        } else {
-            const cplx<R> v = S[j];
-            const double c4 = sc.dt / 6;
-            S[j] = mk<R>((R)((double)v.x + c4 * f[2 * c]), (R)((double)v.y + c4 * f[2 * c + 1]));
-            share[2 * c] = c4 * f[2 * c];
-            share[2 * c + 1] = c4 * f[2 * c + 1];
-        }
-    }
-}
-
-// Chained forced step: A[c][x][column] += sum over the column's band modes lx of share * e^{+2 pi i lx x / N1}
-// (the unnormalised inverse line transform of the shares k_force_post recorded).  One workgroup per band
-// column (ty, tz) and component; columns the state does not store, or without a nonzero share, are left alone.
-template <typename R>
-__global__ void k_force_chain_fix(ForceBand b, FG g, cplx<R>* A, const double* __restrict__ share)
-{
+    __shared__ double share[512][2];                       // per mode of the column (nx <= N1)
     const int ty = blockIdx.x / b.nz, tz = blockIdx.x % b.nz, c = blockIdx.y;
     int lx, ly, lz;
     band_mode(b, (long)ty * b.nz + tz, lx, ly, lz);
     if (lz >= g.nkz || !lkept(g.my, ly)) return;
-    bool any = false;
-    for (int tx = 0; tx < b.nx; tx++) {
-        const double* d = share + 6 * (((long)tx * b.ny + ty) * b.nz + tz) + 2 * c;
-        any = any || d[0] != 0.0 || d[1] != 0.0;
+    const StageCoef sc = *coef;
+    const double ky = ky_of(ly, g.N2) * g.f2, kz = lz * g.f3, kyz2 = ksq_f(0.0, ky, kz);
+    int any = 0;
+    for (int tx = threadIdx.x; tx < b.nx; tx += 256) {
+        const long t = ((long)tx * b.ny + ty) * b.nz + tz;
+        const double fr = fbox[6 * t + 2 * c], fi = fbox[6 * t + 2 * c + 1];
+        band_mode(b, t, lx, ly, lz);
+        double sr = 0.0, si = 0.0;
+        if ((fr != 0.0 || fi != 0.0) && lkept(g.mx, lx)) {
+            const double kx = kx_four(lx, g.N1) * g.f1, kx2 = ksq_f(kx, 0.0, 0.0);
+            const double eh = exp(sc.fh[0] * kx2) * exp(sc.fh[0] * kyz2), e1 = exp(sc.f1[0] * kx2) * exp(sc.f1[0] * kyz2);
+            const long j = c * g.cS + (long)lq(g.mx, lx) * g.sx + (long)lq(g.my, ly) * g.KZP + lz;
+            double cv, ca = 0.0;
+            if (sc.stage == 1) { cv = 0.5 * sc.dt * eh; ca = sc.dt / 6 * e1; }
+            else if (sc.stage == 2) { cv = 0.5 * sc.dt; ca = sc.dt / 3 * eh; }
+            else if (sc.stage == 3) { cv = sc.dt * eh; ca = sc.dt / 3 * eh; }
+            else cv = sc.dt / 6;
+            sr = cv * fr;
+            si = cv * fi;
+            auto add = [&](cplx<R>& q, double r, double i) { q = mk<R>((R)((double)q.x + r), (R)((double)q.y + i)); };
+            if (sc.stage == 4) {
+                add(S[j], sr, si);
+            } else {
+                if (!chained || sc.stage == 3) add(Vs[j], sr, si);
+                add(acc[j], ca * fr, ca * fi);
+            }
+            any = 1;
+        }
+        share[tx][0] = sr;
+        share[tx][1] = si;
     }
-    if (!any) return;
+    if (!__syncthreads_or(any) || !chained) return;
     cplx<R>* col = A + c * g.cA + (long)lq(g.my, ly) * g.KZP + lz;
-    for (int x = threadIdx.x; x < g.N1; x += blockDim.x) {
+    for (int x = threadIdx.x; x < g.N1; x += 256) {
         double sr = 0.0, si = 0.0;
         for (int tx = 0; tx < b.nx; tx++) {
-            const long t = ((long)tx * b.ny + ty) * b.nz + tz;
-            const double dr = share[6 * t + 2 * c], di = share[6 * t + 2 * c + 1];
-            if (dr == 0.0 && di == 0.0) continue;
-            band_mode(b, t, lx, ly, lz);
-            const long m = ((long)lx * x) % g.N1;   // e^{+2 pi i lx x / N1} from the exact phase index
-            double sn, cs;
-            sincospi(2.0 * (double)m / g.N1, &sn, &cs);
-            sr += dr * cs - di * sn;
-            si += dr * sn + di * cs;
+            const double dr = share[tx][0], di = share[tx][1];
+            if (dr == 0.0 && di == 0.0) continue;          // uniform
+            const int kx = b.fullx ? tx : tx - b.kxm, l = kx >= 0 ? kx : kx + g.N1;
+            const c64 w = tw[(l * x) % g.N1];              // e^{-2 pi i l x / N1}
+            sr += dr * w.x + di * w.y;
+            si += di * w.x - dr * w.y;
         }
         cplx<R>& a = col[(long)x * g.sx];
         a = mk<R>((R)((double)a.x + sr), (R)((double)a.y + si));
@@ -664,23 +634,16 @@ __global__ void k_force_chain_fix(ForceBand b, FG g, cplx<R>* A, const double* _
 
 // One RK4 step of every box in s, as 4 stages x 5 pass launches on stream st (forced: plus the
 // band kernels around each stage); chained: 4 passes per stage, the x-inverse done by the previous
-// stage's x-forward (the first stage's by the step before, or by the priming launch in th_step), and a forced
-// chained stage adds k_force_recon before and k_force_chain_fix after.
+// stage's x-forward (the first stage's by the step before, or by the priming launch in th_step).
 template <typename R> static int enqueue_step(th_state* s, hipStream_t st, bool chained = false)
 {
     const long nb = (long)s->fb.nx * s->fb.ny * s->fb.nz;
-    const dim3 fgrid((unsigned)((nb + 255) / 256));
+    const c64* tw64 = s->forced ? (const c64*)s->plan->tw.get(s->fg.N1, 0, st) : nullptr;
     for (int stage = 1; stage <= 4; stage++) {
         if (s->forced) {
-            const cplx<R>* src = (const cplx<R>*)(stage == 1 ? s->S : s->Vs);
-            const double* vbox = nullptr;
-            if (chained && stage > 1) {   // no stage field: its band modes from the A lines
-                vbox = (const double*)s->fbox + 12 * nb;
-                hipLaunchKernelGGL((k_force_recon<R>), dim3((unsigned)nb), dim3(256), 0, st, s->fb, s->fg,
-                                   (const cplx<R>*)s->X1, (double*)vbox);
-                TH_CHECK_HIP(hipGetLastError());
-            }
-            hipLaunchKernelGGL((k_force_pre<R>), fgrid, dim3(256), 0, st, s->fb, s->fg, src, vbox, s->fbox);
+            const cplx<R>* src = (const cplx<R>*)(stage == 1 ? s->S : chained ? nullptr : s->Vs);
+            hipLaunchKernelGGL((k_force_in<R>), dim3((unsigned)nb), dim3(FIN_THREADS), 0, st, s->fb, s->fg, src,
+                               (const cplx<R>*)s->X1, tw64, s->fbox);
             TH_CHECK_HIP(hipGetLastError());
         }
         for (int k = 0; k < NPASS; k++) {
@@ -688,15 +651,11 @@ template <typename R> static int enqueue_step(th_state* s, hipStream_t st, bool 
             TRY(run_pass<R>(s, k, s->var[k], stage, st, chained));
         }
         if (s->forced) {
-            hipLaunchKernelGGL((k_force_post<R>), fgrid, dim3(256), 0, st, s->fb, s->fg,
+            hipLaunchKernelGGL((k_force_out<R>), dim3((unsigned)(s->fb.ny * s->fb.nz), 3), dim3(256), 0, st, s->fb, s->fg,
                                (const StageCoef*)(s->dcoef + (size_t)(stage - 1) * s->nbox), (cplx<R>*)s->S,
-                               (cplx<R>*)s->Vs, (cplx<R>*)s->acc, (double*)s->fbox, chained ? 1 : 0);
+                               (cplx<R>*)s->Vs, (cplx<R>*)s->acc, (cplx<R>*)s->X1, tw64, (const double*)s->fbox,
+                               chained ? 1 : 0);
             TH_CHECK_HIP(hipGetLastError());
-            if (chained) {
-                hipLaunchKernelGGL((k_force_chain_fix<R>), dim3((unsigned)(s->fb.ny * s->fb.nz), 3), dim3(256), 0, st,
-                                   s->fb, s->fg, (cplx<R>*)s->X1, (const double*)s->fbox + 6 * nb);
-                TH_CHECK_HIP(hipGetLastError());
-            }
         }
     }
     return OK;
@@ -737,8 +696,7 @@ extern "C" int th_state_set_force(th_state* s, const th_force* f)
                 return E_UNSUPPORTED;
             }
         }
-        // per band mode: P(F); the stage's share and the reconstructed stage input (chained steps)
-        const size_t need = (size_t)nb * 18;
+        const size_t need = (size_t)nb * 6;   // P(F) per band mode
         if (need > s->fbox_cap) {
             // the old buffer goes away: the state is unforced (and its captured step void) until this succeeds
             s->forced = false;
@@ -769,6 +727,7 @@ static int ensure_twiddles(th_plan* p, const FG& g, hipStream_t st)
 {
     for (int L : {g.N1, g.N2, g.LZ, g.N3, g.scft ? 4 * g.N1 : g.N1})
         if (!p->tw.get(L, p->prec, st)) { set_error("twiddle table allocation failed"); return E_NOMEM; }
+    if (!p->tw.get(g.N1, 0, st)) { set_error("twiddle table allocation failed"); return E_NOMEM; }   // band kernels
     return OK;
 }
 
