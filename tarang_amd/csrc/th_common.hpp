@@ -72,6 +72,16 @@ __host__ __device__ __forceinline__ unsigned fdiv(unsigned n, const FastDiv& f)
     return (unsigned)(((unsigned long long)n * f.m) >> 32) >> (f.s - 1);
 }
 
+// Workgroups are dispatched round-robin over the 8 XCDs (linear id mod 8), each XCD with its own
+// L2.  xcd_tile renumbers a linear workgroup id so that every XCD gets one contiguous range of
+// logical tiles: neighbouring tiles, which share 128-byte lines, then meet in the same L2.
+__device__ __forceinline__ int xcd_tile(int bid, int nblk)
+{
+    const int xcd = bid & 7, loc = bid >> 3;
+    const int per = nblk >> 3, rem = nblk & 7;
+    return (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + loc;
+}
+
 // Wavenumber helpers (trunk/lib/four/four_inline.h:88-138, trunk/lib/scft/scft_inline.h:86)
 __host__ __device__ __forceinline__ int kx_four(int l1, int N1) { return (l1 <= N1 / 2) ? l1 : l1 - N1; }
 __host__ __device__ __forceinline__ int ky_of(int l2, int N2) { return (l2 <= N2 / 2) ? l2 : l2 - N2; }

@@ -20,9 +20,6 @@ __host__ __device__ __forceinline__ bool lkept(const LMap& m, int l) { return l 
 __host__ __device__ __forceinline__ int lq(const LMap& m, int l) { return l < m.h ? l : l - (m.N - m.nk); }
 __host__ __device__ __forceinline__ int ll(const LMap& m, int q) { return q < m.h ? q : q + (m.N - m.nk); }
 
-// Workgroups are dispatched round-robin over the 8 XCDs (linear id mod 8), each XCD with its own
-// L2.  xcd_tile renumbers a linear workgroup id so that every XCD gets one contiguous range of
-// logical tiles: neighbouring tiles, which share 128-byte lines, then meet in the same L2.
 // A zero the compiler cannot see through.  Offsetting a table pointer by it inside a rolled loop
 // keeps the table loads in the loop (L1 hits) instead of hoisting every twiddle into registers
 // for the whole kernel, which would cost occupancy.
@@ -40,13 +37,6 @@ template <int L, int P, int E, int RL> __host__ __device__ constexpr bool xdrop(
 {
     const int m = i / RL + (i % RL) * (E / RL), h = L / 3;
     return m * P >= h && m * P + P - 1 <= L - h;
-}
-
-__device__ __forceinline__ int xcd_tile(int bid, int nblk)
-{
-    const int xcd = bid & 7, loc = bid >> 3;
-    const int per = nblk >> 3, rem = nblk & 7;
-    return (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + loc;
 }
 
 struct FG {
