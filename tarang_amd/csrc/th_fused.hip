@@ -5,6 +5,7 @@
 // kernels are described in th_fused_kern.hpp; NS and MHD states step chained (four launches per stage: each
 // stage's x-forward also performs the next stage's x-inverse).
 #include <stdio.h>
+#include <algorithm>
 #include <array>
 #include <string>
 #include <vector>
@@ -151,6 +152,8 @@ struct th_state {
     bool stage_kept = true;
     bool forced = false;         // energy / helicity forcing (th_state_set_force)
     ForceBand fb{};
+    void* et = nullptr;          // energy transfer: workspace of several giver shells at once
+    size_t et_cap = 0;
     double* fbox = nullptr;      // projected force P(F) of the stage input, 3 complex FP64 per band-box mode
     size_t fbox_cap = 0;
     hipGraphExec_t gexec = nullptr;
@@ -160,6 +163,7 @@ struct th_state {
         if (gexec) (void)hipGraphExecDestroy(gexec);
         if (graph) (void)hipGraphDestroy(graph);
         if (fbox) (void)hipFree(fbox);
+        if (et) (void)hipFree(et);
         for (void* q : {S, Vs, acc, X1, X2, X3}) if (q) (void)hipFree(q);
         if (partial) (void)hipFree(partial);
         if (radii) (void)hipFree(radii);
@@ -209,6 +213,8 @@ static const PlaneTab& plane_tab(int physics)
     static const PlaneTab rb = {3, {0, 1, 2}, {{0, 3, 1}, {1, 3, 2}, {2, 3, 0}}, {{0, 6, 3}, {1, 7, 4}, {2, 8, 5}}};
     return physics == TH_NS ? ns : physics == TH_MHD ? mhd : rb;
 }
+// energy transfer: helper lines 0-2, every giver's the same, giver lines 3-5; product (i, j) = G_i H_j
+static const PlaneTab et_tab = {3, {3, 4, 5}, {{0, 1, 2}, {2, 1, 0}, {0, 1, 2}}, {{0, 1, 2}, {5, 4, 3}, {6, 7, 8}}, 3};
 
 // Fused state for nbox boxes of the plan's size. Single states (nbox == 1) also keep room for the
 // energy-transfer pipeline (6 B-layout and 9 C-layout comps); batched states hold only what the
@@ -448,7 +454,7 @@ template <typename R> static int run_pass(th_state* s, int pass, int var, int st
     case PASS_Z: {
         const cplx<R>* twz = p->twd<R>(g.LZ);
         const cplx<R>* twn = p->twd<R>(g.N3);
-        if (s->plane) return d_plane<R>(g, plane_tab(ph), plane_groups(g, nout), X1, X3, twy, twz, twn, st);
+        if (s->plane) return d_plane<R>(g, plane_tab(ph), plane_groups(g, nout), X1, X3, g.bA, twy, twz, twn, st);
         if (ph == TH_RB) return d_z<R, 3>(g, X2, X3, twz, twn, var, st);
         return ph == TH_MHD ? d_z<R, 1>(g, X2, X3, twz, twn, var, st) : d_z<R, 0>(g, X2, X3, twz, twn, var, st);
     }
@@ -782,7 +788,7 @@ extern "C" int th_step(th_plan* p, th_state* s, double dt, const th_phys* ph, in
 // T(n, m) (Shell_mult_all, |K| <= kmax_inside) and the same sums over |K| > kmax_inside ("corner",
 // which Shell_mult_single counts); then Pi(R_i) = sum_{n<=i} sum_{m>i} [T(n,m) - corner(n,m)]
 // (sphere i = union of shells 1..i and N[G] is linear in G).
-// Per giver shell n (inner radii[n-1] < |K| <= radii[n], n = 1..ngiv) of the energy-transfer pipeline with
+// For every giver shell n (inner radii[n-1] < |K| <= radii[n], n = 1..ngiv) of the energy-transfer pipeline with
 // helper H = state components hoff..hoff+2, giver G = components goff..goff+2 and each receiver R_r =
 // components roff[r]..roff[r]+2 of the state, the sums over the modes of receiver shell m (Get_shell_index
 // basis_basicfn.cc:288-299 on |K|) of 2 mult Re(N[H, G_n] . R_r*), N = EnergyTr_Compute_nlin
@@ -813,34 +819,84 @@ static int et_shell_rows(th_state* s, const double* radii, int nsh, int ngiv, in
     TH_CHECK_HIP(hipMemcpyAsync(s->radii, radii, nr * sizeof(double), hipMemcpyHostToDevice, st));
     int nblk = 0;
     TRY(d_xfwd_et<R>(g, X1, S, twx, s->radii, nr, 0, nullptr, &nblk, st));
-    size_t need = (size_t)nblk * (2 * nr) + (size_t)ngiv * nrecv * (2 * nr);
+    const int kin = max_radius_inside(p->g);
+    // Givers are independent, so small boxes run several at once as boxes of one launch: one by one, each cost 70 us of
+    // launches and dependent passes whatever the box size (15 givers, FP64: 32^3 1250 -> 97 us, 64^3 1397 -> 297).  As
+    // many as 128 MB of pipeline buffers hold, so that those stay in the 256 MB last-level cache (96^3: one, which
+    // fills the chip by itself), and at most 64, which bounds the partial sums; one needs no buffers of its own.
+    const bool plane = s->plane;
+    const size_t per = (plane ? 3 * g.cA + 9 * g.cA : 3 * g.cA + 3 * g.cB + 9 * g.cB + 9 * g.cA) * sizeof(cplx<R>);
+    const size_t shared = (plane ? 3 * g.cA : 3 * g.cB) * sizeof(cplx<R>);
+    int G = (int)std::min<size_t>(std::min<size_t>(std::max<size_t>((128u << 20) / per, 1), 64), ngiv);
+    if (G > 1 && shared + G * per > s->et_cap) {
+        if (s->et) TH_CHECK_HIP(hipFree(s->et));
+        s->et = nullptr;
+        s->et_cap = 0;
+        if (hipMalloc(&s->et, shared + G * per) == hipSuccess) {
+            s->et_cap = shared + G * per;
+            TH_CHECK_HIP(hipMemsetAsync(s->et, 0, s->et_cap, st));   // row padding is read (never used)
+        } else {
+            (void)hipGetLastError();
+            s->et = nullptr;
+            G = 1;   // no room: one at a time in the state's own buffers
+        }
+    }
+    size_t need = (size_t)G * nblk * (2 * nr) + (size_t)ngiv * nrecv * (2 * nr);
     if (need > s->partial_cap) {
         if (s->partial) (void)hipFree(s->partial);
         s->partial = nullptr;
+        s->partial_cap = 0;
         TH_CHECK_HIP(hipMalloc(&s->partial, need * sizeof(double)));
         s->partial_cap = need;
     }
-    const int kin = max_radius_inside(p->g);
-    ShellSel all{-1.0, 1e300};
-    // helper H: inverse x, y once, kept in X2 comps 0..2 (B layout)
-    TRY((d_xinv<R, 0>(g, S + (long)hoff * g.cS, X1, 3, twx, all, 0, st)));
-    // the y passes take the step's tuned launch shapes (the same kernels, any component count)
-    TRY(d_yinv<R>(g, X1, X2, 3, twy, s->var[PASS_YINV], st));
     for (int r = 0; r < nrecv; r++) {
         Yb[r].assign((size_t)(ngiv + 1) * nr, 0.0);
         Yc[r].assign((size_t)(ngiv + 1) * nr, 0.0);
     }
-    // the sums of every giver and receiver stay on the device until the last one is done
-    double* outd = s->partial + (size_t)nblk * (2 * nr);
-    for (int n = 1; n <= ngiv; n++) {
-        ShellSel sel{radii[n - 1], radii[n]};
-        TRY((d_xinv<R, 2>(g, S + (long)goff * g.cS, X1, 3, twx, sel, 0, st)));
-        TRY(d_yinv<R>(g, X1, X2 + 3 * g.cB, 3, twy, s->var[PASS_YINV], st));
-        TRY((d_z<R, 2>(g, X2, X3, twz, twn, 0, st)));
-        TRY(d_yfwd<R>(g, X3, X1, 9, twy, s->var[PASS_YFWD], st));
+    // the sums of every giver and receiver stay on the device until the last one is done: [receiver][giver][2 nr]
+    double* outd = s->partial + (size_t)G * nblk * (2 * nr);
+    // buffers: Ag the givers' A lines (plane: behind the helper's), B the helper's three B components and then the
+    // givers', C and D the product lines, box-major
+    cplx<R>*A0 = X1, *B = X2, *C = X3, *D = plane ? X3 : X1;
+    if (G > 1) {
+        cplx<R>* w = (cplx<R>*)s->et;
+        if (plane) {
+            A0 = w;
+            D = w + (3 + 3 * (size_t)G) * g.cA;
+        } else {
+            B = w;
+            C = B + (3 + 3 * (size_t)G) * g.cB;
+            A0 = C + 9 * (size_t)G * g.cB;
+            D = A0 + 3 * (size_t)G * g.cA;
+        }
+    }
+    FG gb = g;
+    gb.bS = 0;
+    ShellSel all{-1.0, 1e300};
+    // the helper: x-inverse (plane: its A lines are kept; else x and y, kept in B)
+    TRY((d_xinv<R, 0>(g, S + (long)hoff * g.cS, A0, 3, twx, all, 0, st)));
+    // the y passes take the step's tuned launch shapes (the same kernels, any component count)
+    if (!plane) TRY(d_yinv<R>(g, A0, B, 3, twy, s->var[PASS_YINV], st));
+    cplx<R>* Ag = plane ? A0 + 3 * g.cA : A0;
+    for (int n0 = 1; n0 <= ngiv; n0 += G) {
+        gb.nbox = std::min(G, ngiv - n0 + 1);
+        ShellSel sel{0.0, 0.0, s->radii + n0 - 1};
+        gb.bA = 3 * g.cA;
+        TRY((d_xinv<R, 2>(gb, S + (long)goff * g.cS, Ag, 3, twx, sel, 0, st)));
+        if (plane) {
+            TRY(d_plane<R>(gb, et_tab, plane_groups(gb, 9), A0, D, 9 * g.cA, twy, twz, twn, st));
+        } else {
+            TRY(d_yinv<R>(g, Ag, B + 3 * g.cB, 3 * gb.nbox, twy, s->var[PASS_YINV], st));
+            gb.bB = 3 * g.cB;
+            gb.bC = 9 * g.cB;
+            TRY((d_z<R, 2>(gb, B, C, twz, twn, 0, st)));
+            TRY(d_yfwd<R>(g, C, D, 9 * gb.nbox, twy, s->var[PASS_YFWD], st));
+        }
+        gb.bA = 9 * g.cA;
         for (int r = 0; r < nrecv; r++) {
-            TRY(d_xfwd_et<R>(g, X1, S + (long)roff[r] * g.cS, twx, s->radii, nr, kin, s->partial, &nblk, st));
-            launch_finalize((const double*)s->partial, nblk, 2 * nr, 2 * nr, outd + ((size_t)(n - 1) * nrecv + r) * 2 * nr, st);
+            TRY(d_xfwd_et<R>(gb, D, S + (long)roff[r] * g.cS, twx, s->radii, nr, kin, s->partial, &nblk, st));
+            launch_finalize((const double*)s->partial, nblk, 2 * nr, 2 * nr, outd + ((size_t)r * ngiv + n0 - 1) * 2 * nr, st,
+                            gb.nbox);
             TH_CHECK_HIP(hipGetLastError());
         }
     }
@@ -849,7 +905,7 @@ static int et_shell_rows(th_state* s, const double* radii, int nsh, int ngiv, in
     TH_CHECK_HIP(hipStreamSynchronize(st));
     for (int n = 1; n <= ngiv; n++)
         for (int r = 0; r < nrecv; r++) {
-            const double* h = &hostbuf[((size_t)(n - 1) * nrecv + r) * 2 * nr];
+            const double* h = &hostbuf[((size_t)r * ngiv + n - 1) * 2 * nr];
             for (int m = 0; m < nr; m++) {
                 Yb[r][(size_t)n * nr + m] = h[m];
                 Yc[r][(size_t)n * nr + m] = h[nr + m];

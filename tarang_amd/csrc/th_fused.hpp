@@ -68,6 +68,7 @@ struct StageCoef {
 
 struct ShellSel {       // giver mask inner < |K| <= outer (Fill_array_shell universal_ET.cc:45-65)
     double inner, outer;
+    const double* r = nullptr;   // device radii: box b takes r[b] < |K| <= r[b + 1] instead
 };
 
 __device__ __forceinline__ double kmag_f(double a, double b, double c)
@@ -113,7 +114,7 @@ template <typename R>
 bool d_xfwd_chainable(const FG& g);
 template <typename R>
 int d_xfwd_et(const FG& g, const cplx<R>* D, const cplx<R>* U, const cplx<R>* tw, const double* radii, int nr, int kin,
-              double* partial, int* nblk, hipStream_t st);
+              double* partial, int* nblk, hipStream_t st);   // box b: D + b bA, partials of block k at (b nblk + k) 2 nr
 template <typename R>
 int d_sx_inv(const FG& g, const cplx<R>* S, cplx<R>* A, const cplx<R>* tw, const cplx<R>* tw4, hipStream_t st);
 template <typename R>
@@ -124,12 +125,12 @@ template <typename R> int d_scatter(const FG& g, const cplx<R>* S, cplx<R>* ref,
 
 // ---- short boxes (th_plane.hpp) ----
 // Passes 2 to 4 in one launch, A (nin lines) -> D (nout lines), for boxes with plane_ok; ngrp = 3 or nout workgroups
-// per x-plane.  D may not be A.
+// per x-plane.  D may not be A; its box stride is bD.
 struct PlaneTab;
 bool plane_ok(const FG& g);
 template <typename R>
-int d_plane(const FG& g, const PlaneTab& tab, int ngrp, const cplx<R>* A, cplx<R>* D, const cplx<R>* tw2, const cplx<R>* twL,
-            const cplx<R>* twN, hipStream_t st);
+int d_plane(const FG& g, const PlaneTab& tab, int ngrp, const cplx<R>* A, cplx<R>* D, long bD, const cplx<R>* tw2,
+            const cplx<R>* twL, const cplx<R>* twN, hipStream_t st);
 // The x-forward with the products side by side (N1 <= 128), NS (MODE 0) and MHD (MODE 1); chained for every N1
 template <typename R, int MODE>
 int d_xsplit(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw,
@@ -140,6 +141,7 @@ int d_xsplit(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* 
 struct PlaneTab {
     signed char npr;
     signed char x[3], y[3][3], o[3][3];
+    signed char shared;   // inputs below this one are the same for every box (no box stride)
 };
 
 FG make_fg(const Geo& geo, int prec);

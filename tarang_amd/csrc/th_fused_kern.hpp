@@ -55,6 +55,10 @@ __global__ __launch_bounds__(T * P) void k_fx_inv(FG g, const cplx<R>* __restric
     S += blockIdx.z * g.bS;
     A += blockIdx.z * g.bA;
     double Ky = 0, Kz = 0;
+    if (MODE == 2 && sel.r) {
+        sel.inner = sel.r[blockIdx.z];
+        sel.outer = sel.r[blockIdx.z + 1];
+    }
     if (MODE == 2) {
         Ky = ky_of(ll(g.my, cy), g.N2) * g.f2;
         Kz = cz * g.f3;
@@ -203,7 +207,8 @@ __global__ __launch_bounds__(TZ * P) void k_fz(FG g, const cplx<R>* __restrict__
     const long q = (long)blockIdx.x * TZ + c;
     const bool ok = q < (long)g.N1 * g.N2;
     const long off = q * g.KZP;
-    B += blockIdx.y * g.bB;
+    const long boff = blockIdx.y * g.bB;   // energy transfer: the helper's lines (0-2) are every box's
+    if (MODE != 2) B += boff;
     Cout += blockIdx.y * g.bC;
     cplx<R>* Z = lds + c * LZS;
     // The half-length packing pairs point k = t + P m with LZ - k.  The line's points go to
@@ -227,7 +232,7 @@ __global__ __launch_bounds__(TZ * P) void k_fz(FG g, const cplx<R>* __restrict__
             for (int m = 0; m < E; m++) xa[m] = ok ? ld_nt(X + t + P * m) : czero<R>();
             xa[E] = (ok && t == 0) ? X[LZ] : czero<R>();
         } else {
-            const cplx<R>* X = B + a * g.cB + off;
+            const cplx<R>* X = B + a * g.cB + off + (MODE == 2 && a >= 3 ? boff : 0);
 #pragma unroll
             for (int m = 0; m < E; m++) {
                 const int k = t + P * m;
@@ -1042,6 +1047,7 @@ __global__ __launch_bounds__(T * P) void k_fx_fwd_et(FG g, const cplx<R>* __rest
     const int cz = (blockIdx.x % ntz) * T + c;
     const bool ok = cz < g.nkz;
     const long m = (long)cy * g.KZP + cz;
+    D += blockIdx.y * g.bA;
     const R Ky = (R)(ky_of(ll(g.my, cy), g.N2) * g.f2);
     const R Kz = (R)(cz * g.f3);
     cplx<R> Nacc[3][E];
@@ -1112,7 +1118,7 @@ __global__ __launch_bounds__(T * P) void k_fx_fwd_et(FG g, const cplx<R>* __rest
         }
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < 2 * nr; b += T * P) partial[(long)blockIdx.x * (2 * nr) + b] = bins[b];
+    for (int b = threadIdx.x; b < 2 * nr; b += T * P) partial[((long)blockIdx.y * gridDim.x + blockIdx.x) * (2 * nr) + b] = bins[b];
 }
 
 // compact <-> reference layout.  Both are bound by memory (a download writes the whole reference array, non-temporally:
@@ -1247,7 +1253,7 @@ static int launch_xfwd_et(const FG& g, const cplx<R>* D, const cplx<R>* U, const
     const int ntz = (g.nkz + T - 1) / T;
     *nblk = g.my.nk * ntz;
     if (!partial) return OK;
-    hipLaunchKernelGGL((k_fx_fwd_et<R, L, P, T>), dim3(*nblk), dim3(T * P), 2 * nr * sizeof(double), st, g, D, U, tw,
+    hipLaunchKernelGGL((k_fx_fwd_et<R, L, P, T>), dim3(*nblk, g.nbox), dim3(T * P), 2 * nr * sizeof(double), st, g, D, U, tw,
                        radii, nr, kin, partial);
     TH_CHECK_HIP(hipGetLastError());
     return OK;

@@ -185,6 +185,8 @@ static __global__ __launch_bounds__(FIN_T) void k_finalize_bins(const double* __
 {
     __shared__ double ss[FIN_T], cc[FIN_T];
     const int b = blockIdx.x, t = threadIdx.x;
+    partial += (long)blockIdx.y * nblk * stride;           // set y of nblk partials each -> out + y * (values)
+    out += (long)blockIdx.y * gridDim.x;
     double s = 0.0, c = 0.0;
     for (int k = t; k < nblk; k += FIN_T) {
         const double v = partial[(long)k * stride + b];
@@ -206,9 +208,10 @@ static __global__ __launch_bounds__(FIN_T) void k_finalize_bins(const double* __
     }
     if (t == 0) out[b] = ss[0] + cc[0];
 }
-static inline void launch_finalize(const double* partial, int nblk, long stride, int nval, double* out, hipStream_t st)
+static inline void launch_finalize(const double* partial, int nblk, long stride, int nval, double* out, hipStream_t st,
+                                   int nset = 1)
 {
-    hipLaunchKernelGGL(k_finalize_bins, dim3((unsigned)nval), dim3(FIN_T), 0, st, partial, nblk, stride, out);
+    hipLaunchKernelGGL(k_finalize_bins, dim3((unsigned)nval, (unsigned)nset), dim3(FIN_T), 0, st, partial, nblk, stride, out);
 }
 #endif
 

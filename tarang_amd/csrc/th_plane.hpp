@@ -22,7 +22,7 @@ template <typename R> constexpr size_t plane_lds(int L2, int LZ, int line) { ret
 
 template <typename R, int L2, int LZ>
 __global__ __launch_bounds__(L2 * (LZ / plane_EZ(LZ))) void k_plane(FG g, PlaneTab tab, int ngrp, const cplx<R>* __restrict__ A,
-                                                                     cplx<R>* __restrict__ D, const cplx<R>* __restrict__ tw2,
+                                                                     cplx<R>* __restrict__ D, long bD, const cplx<R>* __restrict__ tw2,
                                                                      const cplx<R>* __restrict__ twL,
                                                                      const cplx<R>* __restrict__ twN)
 {
@@ -44,8 +44,8 @@ __global__ __launch_bounds__(L2 * (LZ / plane_EZ(LZ))) void k_plane(FG g, PlaneT
     // workgroups of one plane are neighbours (they read the same operands), and neighbours share an XCD's L2
     const int lin = xcd_tile(blockIdx.x, gridDim.x);
     const int q = lin % ngrp, xb = lin / ngrp, x = xb % g.N1, box = xb / g.N1;
-    A += box * g.bA + (long)x * g.sx;
-    D += box * g.bA + (long)x * g.sx;
+    A += (long)x * g.sx;
+    D += box * bD + (long)x * g.sx;
     const int np = 3 * tab.npr, s0 = q * np / ngrp, s1 = (q + 1) * np / ngrp;
     // column threads: lanes along kz (memory order), row threads: the PZ lanes of one row in one wavefront
     const int c = threadIdx.x % NKZ, tc = threadIdx.x / NKZ;
@@ -58,7 +58,7 @@ __global__ __launch_bounds__(L2 * (LZ / plane_EZ(LZ))) void k_plane(FG g, PlaneT
     // once every thread is at the column transform's first barrier.
     auto operand = [&](int a, cplx<R> (&u)[EZ]) {
         cplx<R> v[E2];
-        const cplx<R>* src = A + a * g.cA + c;
+        const cplx<R>* src = A + a * g.cA + (a < tab.shared ? 0 : box * g.bA) + c;
 #pragma unroll
         for (int i = 0; i < E2; i++) {
             const int l = YI::in_pos(tc, i);
@@ -353,7 +353,7 @@ static int launch_xsplit(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* 
 }
 
 template <typename R, int L2, int LZ>
-static int launch_plane(const FG& g, const PlaneTab& tab, int ngrp, const cplx<R>* A, cplx<R>* D, const cplx<R>* tw2,
+static int launch_plane(const FG& g, const PlaneTab& tab, int ngrp, const cplx<R>* A, cplx<R>* D, long bD, const cplx<R>* tw2,
                         const cplx<R>* twL, const cplx<R>* twN, hipStream_t st)
 {
     constexpr size_t lds = plane_lds<R>(L2, LZ, ZPad<LZ>::line);
@@ -361,7 +361,7 @@ static int launch_plane(const FG& g, const PlaneTab& tab, int ngrp, const cplx<R
     auto k = k_plane<R, L2, LZ>;
     if (lds > 64 * 1024)
         TH_CHECK_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(k, dim3((unsigned)(g.N1 * g.nbox * ngrp)), dim3(L2 * (LZ / plane_EZ(LZ))), lds, st, g, tab, ngrp, A, D,
+    hipLaunchKernelGGL(k, dim3((unsigned)(g.N1 * g.nbox * ngrp)), dim3(L2 * (LZ / plane_EZ(LZ))), lds, st, g, tab, ngrp, A, D, bD,
                        tw2, twL, twN);
     TH_CHECK_HIP(hipGetLastError());
     return OK;
@@ -369,10 +369,10 @@ static int launch_plane(const FG& g, const PlaneTab& tab, int ngrp, const cplx<R
 
 // ---- dispatch (each translation unit instantiates the half of the plane lengths it names) ----
 template <typename R, int L2>
-static int plane_z(const FG& g, const PlaneTab& tab, int ngrp, const cplx<R>* A, cplx<R>* D, const cplx<R>* tw2,
+static int plane_z(const FG& g, const PlaneTab& tab, int ngrp, const cplx<R>* A, cplx<R>* D, long bD, const cplx<R>* tw2,
                    const cplx<R>* twL, const cplx<R>* twN, hipStream_t st)
 {
-#define C_(n) case n: return launch_plane<R, L2, n>(g, tab, ngrp, A, D, tw2, twL, twN, st);
+#define C_(n) case n: return launch_plane<R, L2, n>(g, tab, ngrp, A, D, bD, tw2, twL, twN, st);
     switch (g.LZ) {
         C_(8) C_(12) C_(16) C_(24) C_(32) C_(48) C_(64)
         default: set_error("plane pass: N3 %d unsupported", g.N3); return E_UNSUPPORTED;
