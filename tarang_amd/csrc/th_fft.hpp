@@ -334,7 +334,10 @@ template <typename R, int L, int P, int SIGN, bool R16 = false> struct LineFFT {
                 for (int r = 1; r < Rr; r++) {
                     cplx<R> w = tw[r * k * (L / (Ns * Rr))];
                     if (SIGN > 0) w.y = -w.y;
-                    v[b * Rr + r] = cmul(v[b * Rr + r], w);
+                    // which product is fused is spelled out: left to the compiler it changes with the surrounding
+                    // code, and the same line in two kernels would differ in the last bit
+                    const cplx<R> q = v[b * Rr + r];
+                    v[b * Rr + r] = mk<R>(fma(q.x, w.x, -(q.y * w.y)), fma(q.x, w.y, q.y * w.x));
                 }
             }
             DFT<Rr, SIGN, R>::run(&v[b * Rr]);

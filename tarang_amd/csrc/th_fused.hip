@@ -181,10 +181,9 @@ static std::string tune_key(const th_state* s)
     return k;
 }
 
-// Short boxes (th_plane.hpp).  Both rules are on the grid alone, so that a box computes the same bits alone and in an
-// ensemble.
+// Short boxes (th_plane.hpp).
 //
-// Passes 2 to 4 as one launch: N2 and N3 up to 128 with at most 8192 points per plane (74 KB of LDS in FP64), and in
+// Passes 2 to 4 as one launch, by the grid alone (a box computes the same bits alone and in an ensemble): N2 and N3 up to 128 with at most 8192 points per plane (74 KB of LDS in FP64), and in
 // FP64 planes past 4608 points only on long boxes, where the three passes wait on memory rather than on launches.
 // us per step, three passes / plane pass: 32^3 FP64 160 / 98, 64^3 FP64 174 / 125, eight 64^3 FP32 306 / 187,
 // 512 x 64 x 64 FP64 465 / 309, 512 x 128 x 64 FP32 564 / 369; past the line 96^3 FP32 213 / 202 to 248,
@@ -196,12 +195,19 @@ bool th::plane_ok(const FG& g)
     return pts <= (g.fp64 && g.N1 < 256 ? 4608 : 8192);
 }
 // The x-forward with the products side by side, NS and MHD: where one workgroup per tile of columns leaves CUs idle
-// or waiting.  us per step, one after another / side by side: 16 x 64 x 64 FP64 107 / 59, 64 x 128 x 128 FP32
-// 207 / 180, 128 x 64 x 64 FP64 173 / 130; past the line 64 x 256 x 256 FP32 347 / 392, eight 96^3 FP32 561 / 743.
+// or waiting, that is up to so many kept points in all boxes, and in FP64 on lines to 48 points always (a tile of
+// k_fx_fwd is 16 to 48 threads there).  Both kernels compute the same bits (from 24 points on; lines of 16 take other
+// radices, so there the boxes do not count).  us per step, one after another / side by side: 96^3 FP32 210 / 163, two
+// of them 272 / 263, four 371 / 426; 64^3 FP32 alone 107 / 71, eight 191 / 186, sixteen 273 / 303; 128 x 64 x 96 FP64
+// 227 / 210, 128^3 FP64 351 / 383; MHD 96^3 FP32 313 / 231, 128^3 FP32 363 / 448, 64 x 128 x 128 FP64 347 / 354;
+// 48 x 512 x 512 FP32 939 / 1080, FP64 2034 / 1974, 24 x 256 x 256 FP64 MHD 833 / 474.
 static bool split_ok(const FG& g, int physics)
 {
-    const long pts = (long)g.N1 * g.my.nk * g.nkz;
-    return physics != TH_RB && ((g.N1 <= 64 && pts <= 250000) || (g.N1 <= 128 && pts <= 120000));
+    if (physics == TH_RB || g.N1 > 128) return false;
+    if (g.fp64 && g.N1 <= 48) return true;
+    const long pts = (long)g.N1 * g.my.nk * g.nkz * (g.N1 == 16 ? 1 : g.nbox);
+    if (physics == TH_MHD) return pts <= (g.fp64 ? 220000 : 350000);
+    return pts <= (g.N1 <= 48 ? 600000 : g.N1 <= 64 ? 500000 : 400000);
 }
 
 // Products of the pipelines (numbered as ZProd in th_fused_kern.hpp), in an order that hands operands on: each

@@ -109,3 +109,24 @@ def test_short_boxes_in_an_ensemble_equal_single_boxes(ctx, prec):
         s.step(1e-3, nu=5e-3, steps=2)
         for got, ref in zip(e.download(b), s.download()):
             assert np.array_equal(got.cpu().numpy(), ref.cpu().numpy())
+
+
+# enough boxes for the x-forward with one tile of columns per workgroup, where one box takes the side-by-side one
+@pytest.mark.parametrize("N,boxes", [((24, 128, 128), 8), ((32, 96, 128), 8), ((48, 96, 96), 7), ((64, 64, 64), 10),
+                                     ((96, 96, 96), 3), ((96, 24, 48), 40), ((128, 64, 64), 4), ((16, 64, 64), 60)])
+@pytest.mark.parametrize("prec", ("fp64", "fp32"))
+def test_many_boxes_equal_one_box(ctx, N, boxes, prec):
+    from tarang_amd import Ensemble, Plan, State
+    print(N, boxes, prec, flush=True)
+    V = Oracle(N).ic_random(3, E0=0.5, kp=3.0)
+    e = Ensemble(ctx, [N] * boxes, precision=prec)
+    for b in range(boxes):
+        e.upload(b, [e.plan(b).to_dev(v * (1.0 if b < boxes - 1 else 0.5)) for v in V])
+    e.step(np.full(boxes, 1e-3), np.full(boxes, 5e-3), steps=2)
+    p = Plan(ctx, N, precision=prec)
+    for b, f in ((0, 1.0), (boxes - 1, 0.5)):
+        s = State(p)
+        s.upload([p.to_dev(v * f) for v in V])
+        s.step(1e-3, nu=5e-3, steps=2)
+        for got, ref in zip(e.download(b), s.download()):
+            assert np.array_equal(got.cpu().numpy(), ref.cpu().numpy())
