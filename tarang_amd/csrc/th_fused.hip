@@ -147,8 +147,7 @@ struct th_state {
     // single x-inverse launch restores after anything else has used the buffers or changed S.
     bool chain_ok = false;
     bool graph_chained = false;
-    // the stage-field buffer holds the last step's last-stage input (false after a chained step of an unforced
-    // state, which never writes it)
+    // the stage-field buffer holds the last step's last-stage input (false after a chained step that writes none)
     bool stage_kept = true;
     bool forced = false;         // energy / helicity forcing (th_state_set_force)
     ForceBand fb{};
@@ -222,6 +221,11 @@ static const PlaneTab& plane_tab(int physics)
 // energy transfer: helper lines 0-2, every giver's the same, giver lines 3-5; product (i, j) = G_i H_j
 static const PlaneTab et_tab = {3, {3, 4, 5}, {{0, 1, 2}, {2, 1, 0}, {0, 1, 2}}, {{0, 1, 2}, {5, 4, 3}, {6, 7, 8}}, 3};
 
+// whether a chained step writes its stage-3 output, the last stage's input (th_state_download_buffer): a forced state's
+// host driver evaluates the outputs' force from it, and on short lines, which could always be asked for it, it costs
+// nothing measurable (32^3 FP64: 49 us per step with and without)
+static int keeps_last(const th_state* s) { return s->forced || (s->nbox == 1 && s->fg.N1 <= 32); }
+
 // Fused state for nbox boxes of the plan's size. Single states (nbox == 1) also keep room for the
 // energy-transfer pipeline (6 B-layout and 9 C-layout comps); batched states hold only what the
 // RK step needs.
@@ -270,6 +274,7 @@ static int state_create(th_plan* p, th_state** out, int physics, int nbox)
     }
     s->plane = plane_ok(g);
     s->split = split_ok(g, physics);
+    g.keep3 = keeps_last(s);
     std::vector<int> tv;
     if (tune_lookup(p->ctx, tune_key(s), tv) && (int)tv.size() == NPASS)
         for (int k = 0; k < NPASS; k++) s->var[k] = (tv[k] >= 0 && tv[k] < pass_nvar(k)) ? tv[k] : 0;
@@ -356,7 +361,7 @@ extern "C" int th_state_download_buffer(th_state* s, int which, int comp, void* 
 {
     if (!s || which < 0 || which > 2) { set_error("th_state_download_buffer: bad args"); return E_ARG; }
     if (which == 1 && !s->stage_kept) {
-        set_error("th_state_download_buffer: the chained step of an unforced NS or MHD state keeps no stage field");
+        set_error("th_state_download_buffer: the chained step of an unforced NS or MHD state with N1 > 32 keeps no stage field");
         return E_UNSUPPORTED;
     }
     void* keep = s->S;
@@ -712,7 +717,7 @@ extern "C" int th_state_set_force(th_state* s, const th_force* f)
         if (need > s->fbox_cap) {
             // the old buffer goes away: the state is unforced (and its captured step void) until this succeeds
             s->forced = false;
-            s->fg.keep3 = 0;
+            s->fg.keep3 = keeps_last(s);
             if (s->gexec) { (void)hipGraphExecDestroy(s->gexec); s->gexec = nullptr; }
             if (s->graph) { (void)hipGraphDestroy(s->graph); s->graph = nullptr; }
             if (s->fbox) TH_CHECK_HIP(hipFree(s->fbox));
@@ -728,7 +733,7 @@ extern "C" int th_state_set_force(th_state* s, const th_force* f)
         s->fb = fb;
         s->forced = true;
     }
-    s->fg.keep3 = s->forced ? 1 : 0;
+    s->fg.keep3 = keeps_last(s);
     // the captured step changes
     if (s->gexec) { (void)hipGraphExecDestroy(s->gexec); s->gexec = nullptr; }
     if (s->graph) { (void)hipGraphDestroy(s->graph); s->graph = nullptr; }
@@ -784,7 +789,7 @@ extern "C" int th_step(th_plan* p, th_state* s, double dt, const th_phys* ph, in
     for (int i = 0; i < nsteps; i++) TH_CHECK_HIP(hipGraphLaunch(s->gexec, st));
     if (nsteps > 0) {
         s->chain_ok = chained;
-        s->stage_kept = !chained || s->forced;
+        s->stage_kept = !chained || s->fg.keep3 || s->physics == TH_RB;
     }
     return OK;
 }

@@ -56,7 +56,7 @@ struct FG {
     double norm; // 1 / (2 N1 N2 N3): the line transforms' 1 / (N1 N2 N3) and the z pass's unpacking 1/2 (SCFT: 1/2 more)
     int KZPi = 0;  // z pass on unpruned lines: line and component strides of its input
     long cBi = 0;
-    int keep3 = 0; // chained x-forward of a forced state: write the stage-3 output (the last stage's input field)
+    int keep3 = 0; // chained x-forward: write the stage-3 output (the last stage's input field)
 };
 
 struct StageCoef {

@@ -508,7 +508,7 @@ template <int L, int P, int E, int RL> constexpr int xnext(int i)
 // state in stage 4) stays in the accumulator registers in place of N and is transformed back along x, and the
 // A lines are written to this tile's columns of Aout, which may be D itself (every product of the tile has been read
 // by then, and no other workgroup reads these columns); the stage field itself is not written, except the stage-3 output (the
-// last stage's input) of a forced state (FG::keep3), from which the host evaluates the outputs' force.  NS: components 0-2 = U.
+// last stage's input) with FG::keep3.  NS: components 0-2 = U.
 // MHD: the Elsasser lines of k_fx_inv MODE 1, Z+ = U + B into components 0-2 and Z- = U - B into 3-5.
 template <typename R, int L, int P, int T, int MODE, bool CHAIN = false>
 __global__ __launch_bounds__(T * P) __attribute__((amdgpu_waves_per_eu((MODE == 0 && sizeof(R) == 4 && L % 3 != 0) ? 4 : 1))) void k_fx_fwd(FG g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs,

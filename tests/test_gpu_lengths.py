@@ -130,3 +130,25 @@ def test_many_boxes_equal_one_box(ctx, N, boxes, prec):
         s.step(1e-3, nu=5e-3, steps=2)
         for got, ref in zip(e.download(b), s.download()):
             assert np.array_equal(got.cpu().numpy(), ref.cpu().numpy())
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("fp32", 1e-5)])
+@pytest.mark.parametrize("N", [(16, 32, 24), (24, 64, 64), (32, 16, 128)])
+def test_short_lines_keep_the_last_stage_field(ctx, N, prec, tol):
+    """The input of the last RK4 stage after a step, from the oracle's step with a force of zero supply; NS, and MHD's
+    U with B = 0."""
+    from tarang_amd import Plan, State, abi
+    print(N, prec, flush=True)
+    o = Oracle(N)
+    p = Plan(ctx, N, precision=prec)
+    V = o.ic_random(8, E0=0.5, kp=3.0)
+    d = [p.to_dev(v) for v in V]
+    last = o.zeros(3)
+    o.step_ns_forced(V, 0.01, 1e-3, 1, 1.0, 2.0, 0.0, 0.0, steps=2, last_stage=last)
+    m = max(np.abs(v).max() for v in last)
+    for physics in (abi.TH_NS, abi.TH_MHD):
+        s = State(p, physics)
+        s.upload(d + [p.to_dev(np.zeros_like(v)) for v in V] * (physics == abi.TH_MHD))
+        s.step(1e-3, nu=0.01, eta=0.01, steps=2)
+        for got, ref in zip(s.download_buffer(1)[:3], last):
+            assert np.abs(got.cpu().numpy() - ref).max() <= tol * m
