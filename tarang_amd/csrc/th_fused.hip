@@ -142,7 +142,7 @@ struct th_state {
     int var[NPASS] = {0, 0, 0, 0, 0};   // launch-shape variant per pass (autotuner)
     bool plane = false;          // passes 2-4 as one launch, X1 -> X3 (th_plane.hpp); the y passes launch nothing
     bool split = false;          // x-forward with the products side by side (th_plane.hpp)
-    // Chained step (NS or MHD, unforced): each stage's x-forward also does the next stage's x-inverse, so a
+    // Chained step (NS, MHD, RB with the split x-forward): each stage's x-forward also does the next stage's x-inverse, so a
     // step runs 4 passes per stage; X1 must then hold the x-inverse of S when a step starts (chain_ok), which a
     // single x-inverse launch restores after anything else has used the buffers or changed S.
     bool chain_ok = false;
@@ -193,19 +193,20 @@ bool th::plane_ok(const FG& g)
     const int pts = g.N2 * g.N3;
     return pts <= (g.fp64 && g.N1 < 256 ? 4608 : 8192);
 }
-// The x-forward with the products side by side, NS and MHD: where one workgroup per tile of columns leaves CUs idle
+// The x-forward with the products side by side: where one workgroup per tile of columns leaves CUs idle
 // or waiting, that is up to so many kept points in all boxes, and in FP64 on lines to 48 points always (a tile of
 // k_fx_fwd is 16 to 48 threads there).  Both kernels compute the same bits (from 24 points on; lines of 16 take other
 // radices, so there the boxes do not count).  us per step, one after another / side by side: 96^3 FP32 210 / 163, two
 // of them 272 / 263, four 371 / 426; 64^3 FP32 alone 107 / 71, eight 191 / 186, sixteen 273 / 303; 128 x 64 x 96 FP64
 // 227 / 210, 128^3 FP64 351 / 383; MHD 96^3 FP32 313 / 231, 128^3 FP32 363 / 448, 64 x 128 x 128 FP64 347 / 354;
-// 48 x 512 x 512 FP32 939 / 1080, FP64 2034 / 1974, 24 x 256 x 256 FP64 MHD 833 / 474.
+// 48 x 512 x 512 FP32 939 / 1080, FP64 2034 / 1974, 24 x 256 x 256 FP64 MHD 833 / 474; RB 32^3 FP64 165 / 61, 64^3 FP32
+// 174 / 91, FP64 204 / 125, 96 x 128 x 128 FP32 332 / 301, 128^3 FP32 376 / 423, FP64 574 / 592.
 static bool split_ok(const FG& g, int physics)
 {
-    if (physics == TH_RB || g.N1 > 128) return false;
+    if (g.N1 > 128) return false;
     if (g.fp64 && g.N1 <= 48) return true;
     const long pts = (long)g.N1 * g.my.nk * g.nkz * (g.N1 == 16 ? 1 : g.nbox);
-    if (physics == TH_MHD) return pts <= (g.fp64 ? 220000 : 350000);
+    if (physics != TH_NS) return pts <= (g.fp64 && physics == TH_MHD ? 220000 : 350000);
     return pts <= (g.N1 <= 48 ? 600000 : g.N1 <= 64 ? 500000 : 400000);
 }
 
@@ -472,7 +473,9 @@ template <typename R> static int run_pass(th_state* s, int pass, int var, int st
     case PASS_YFWD: return s->plane ? (int)OK : d_yfwd<R>(g, X3, X1, nout, twy, var, st);
     default: {
         const cplx<R>* D = s->plane ? X3 : X1;
-        if (ph == TH_RB) return d_sx_fwd_rb<R>(g, D, S, Vs, acc, twx, p->twd<R>(4 * g.N1), sc, var, st);
+        if (ph == TH_RB)
+            return s->split ? d_sxsplit<R>(g, D, X1, S, Vs, acc, twx, p->twd<R>(4 * g.N1), sc, st, chain)
+                            : d_sx_fwd_rb<R>(g, D, S, Vs, acc, twx, p->twd<R>(4 * g.N1), sc, var, st);
         if (s->split)
             return ph == TH_MHD ? d_xsplit<R, 1>(g, D, X1, S, Vs, acc, twx, sc, st, chain)
                                 : d_xsplit<R, 0>(g, D, X1, S, Vs, acc, twx, sc, st, chain);
@@ -748,12 +751,12 @@ static int ensure_twiddles(th_plan* p, const FG& g, hipStream_t st)
     return OK;
 }
 
-// whether a step runs this state chained (NS, forced or not, or MHD; N1 with a chained x-forward; any number of
-// boxes)
+// whether a step runs this state chained: the split x-forward always is, else NS (forced or not) and MHD with a
+// chained x-forward for N1
 static bool step_chained(const th_state* s)
 {
-    return (s->physics == TH_NS || s->physics == TH_MHD) &&
-           (s->split || (s->plan->prec ? d_xfwd_chainable<float>(s->fg) : d_xfwd_chainable<double>(s->fg)));
+    if (s->split) return true;
+    return s->physics != TH_RB && (s->plan->prec ? d_xfwd_chainable<float>(s->fg) : d_xfwd_chainable<double>(s->fg));
 }
 
 extern "C" int th_step(th_plan* p, th_state* s, double dt, const th_phys* ph, int nsteps)
@@ -1079,8 +1082,8 @@ template <typename R> static int profile_impl(th_state* s, double dt, double nu,
     double b[5] = {e * (nst * cS + nin * cA), e * (nin * cA + nin * cB), e * (nin * cB + nout * cB),
                    e * (nout * cB + nout * cA), e * (nout * cA + state_rw * nst * cS + extra)};
     if (chained) {
-        // no stage-field write (stages 1-3), the next stage's A lines written instead
-        b[PASS_XFWD] = e * (nout * cA + (state_rw - (stage < 4 ? 1 : 0)) * nst * cS + nin * cA);
+        // the next stage's A lines written too, and (NS, MHD) no stage field in stages 1-3
+        b[PASS_XFWD] = e * (nout * cA + (state_rw - (stage < 4 && s->physics != TH_RB ? 1 : 0)) * nst * cS + extra + nin * cA);
         b[PASS_XINV] = 0;
     }
     if (s->plane) {

@@ -135,6 +135,9 @@ int d_plane(const FG& g, const PlaneTab& tab, int ngrp, const cplx<R>* A, cplx<R
 template <typename R, int MODE>
 int d_xsplit(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw,
              const StageCoef* sc, hipStream_t st, bool chain);
+template <typename R>   // RB
+int d_sxsplit(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw,
+              const cplx<R>* tw4, const StageCoef* sc, hipStream_t st, bool chain);
 
 // Operand and product table of a pipeline (ZProd of th_fused_kern.hpp as plain numbers): product j of rotation step r
 // multiplies input x[r] by input y[r][j] into output o[r][j]; operands are kept from one product to the next where the order allows it.

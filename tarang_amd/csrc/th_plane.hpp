@@ -335,6 +335,183 @@ __global__ __launch_bounds__((XSplit<R, L, T, MODE>::NT)) void k_fx_split(FG g, 
     }
 }
 
+// The same for the sine / cosine lines of RB (k_sx_fwd_rb, k_sx_inv): the nine product lines side by side; the mirror
+// value V_{N-k} of a point's DCT / DST comes from LDS, where the whole line is.  CHAIN: the stage outputs become the
+// next stage's A lines, groups 0-3 transforming V1 (sine), V2, V3 (cosine), T (sine); the stage field is written all
+// the same (the next stage's force reads V1 and T of it).
+template <typename R, int L, int T, bool CHAIN>
+__global__ __launch_bounds__((XSplit<R, L, T, 1>::NT)) void k_sx_split(FG g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S,
+                                                                  cplx<R>* Vs, cplx<R>* acc,
+                                                                  const cplx<R>* __restrict__ tw,
+                                                                  const cplx<R>* __restrict__ tw4,
+                                                                  const StageCoef* __restrict__ coefs)
+{
+    using X = XSplit<R, L, T, 1>;
+    constexpr int E = X::E, P = X::P, NP = X::NP, NT = X::NT, NX = 4;
+    constexpr int RS = P * NP;
+    static_assert(2 * L / 3 <= RS, "one kept row per thread");
+    using F = LineFFT<R, L, P, -1>;
+    using FI = LineFFT<R, L, P, +1>;
+    extern __shared__ __attribute__((aligned(16))) char split_raw[];
+    cplx<R>* const lds = (cplx<R>*)split_raw;
+    cplx<R>* const twl = lds + NP * L * T;
+    double* const exl = (double*)(twl + L);     // as in k_fx_split
+    double* const eyz = exl + NX * L;
+    cplx<R>* const w4 = (cplx<R>*)(eyz + NX * T);
+    const int c = threadIdx.x % T, row = threadIdx.x / T, t = row % P, gi = row / P;
+    const int ntz = (g.nkz + T - 1) / T;
+    const int lin = xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
+    const int tile = lin % gridDim.x, box = lin / gridDim.x;
+    const int cy = tile / ntz;
+    const int cz = (tile % ntz) * T + c;
+    const bool ok = cz < g.nkz;
+    const long m = (long)cy * g.KZP + cz;
+    D += box * g.bA + m;
+    Aout += box * g.bA + m;
+    S += box * g.bS + m;
+    Vs += box * g.bS + m;
+    acc += box * g.bS + m;
+    const StageCoef sc = coefs[box];
+    const int stage = sc.stage;
+    const bool psin = ((0x1A8u >> gi) & 1u) != 0;     // sine products, see k_sx_fwd_rb
+    cplx<R> v[E];
+#pragma unroll
+    for (int i = 0; i < E; i++) {
+        const int j = F::in_pos(t, i);
+        const cplx<R> d = ok ? D[gi * g.cA + (long)j * g.sx] : czero<R>();
+        v[i] = cscale(d, (psin && j >= L / 2) ? R(-1) : R(1));
+    }
+    const cplx<R>* accr = stage > 1 ? acc : S;        // stage 1 has no accumulator yet (value unused)
+    const cplx<R>* F0 = stage == 1 ? S : Vs;          // field the stage's rhs is evaluated on
+    const int l = row;                                // this thread's kept mode
+    const bool on = ok && l < g.mx.nk;
+    cplx<R> s0[4], a0[4], f0[2];
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
+        s0[a] = on ? S[a * g.cS + (long)l * g.sx] : czero<R>();
+        a0[a] = on ? accr[a * g.cS + (long)l * g.sx] : czero<R>();
+    }
+    f0[0] = on ? F0[(long)l * g.sx] : czero<R>();
+    f0[1] = on ? F0[3 * g.cS + (long)l * g.sx] : czero<R>();
+    for (int i = threadIdx.x; i < L; i += NT) {
+        twl[i] = tw[i];
+        w4[i] = tw4[i];
+        const double kx = i * g.f1, kx2 = kx * kx;
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            exl[2 * q * L + i] = exp(sc.fh[q] * kx2);
+            exl[(2 * q + 1) * L + i] = exp(sc.f1[q] * kx2);
+        }
+    }
+    const double dKy = ky_of(ll(g.my, cy), g.N2) * g.f2, dKz = cz * g.f3;
+    if (row < NX) {
+        const double kyz2 = dKy * dKy + dKz * dKz;
+        const double cf = row == 0 ? sc.fh[0] : row == 1 ? sc.f1[0] : row == 2 ? sc.fh[1] : sc.f1[1];
+        eyz[row * T + c] = exp(cf * kyz2);
+    }
+    __syncthreads();
+    cplx<R>* const buf = lds + gi * (L * T);
+    F::template run<T, false, NoPad, false, 0>(v, buf + c, t, twl);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < E; i++) buf[F::out_pos(t, i) * T + c] = v[i];
+    __syncthreads();
+    cplx<R> keep[4];
+    if (on) {
+        const double dKx = l * g.f1;
+        const R Kx = (R)dKx, Ky = (R)dKy, Kz = (R)dKz;
+        const cplx<R> w = w4[l];
+        cplx<R> n[4];
+#pragma unroll
+        for (int a = 0; a < 4; a++) n[a] = czero<R>();
+#pragma unroll
+        for (int p = 0; p < NP; p++) {                // the terms and their order are k_sx_fwd_rb's
+            const bool sn = ((0x1A8u >> p) & 1u) != 0;
+            const cplx<R> Pv = cmul(w, lds[(p * L + l) * T + c]);
+            const cplx<R> Qv = cmul(conjg(w), lds[(p * L + (l ? L - l : 0)) * T + c]);
+            const cplx<R> dv = Pv - Qv, sv = Pv + Qv;
+            cplx<R> Av = sn ? mk<R>(-dv.y, dv.x) : sv;
+            if (sn && l == 0) Av = czero<R>();
+            const int a1 = (p == 0 || p == 3 || p == 5) ? 0 : (p == 1 || p == 4) ? 1 : (p == 2) ? 2 : 3;
+            if (p == 0 || p == 6) n[a1] = mk<R>(n[a1].x - Kx * Av.x, n[a1].y - Kx * Av.y);
+            else acc_iK(n[a1], (p == 1 || p == 3 || p == 7) ? Ky : Kz, Av);
+            const int a2 = p == 3 ? 1 : 2;
+            if (p == 3 || p == 5) n[a2] = mk<R>(n[a2].x + Kx * Av.x, n[a2].y + Kx * Av.y);
+            else if (p == 4) acc_iK(n[a2], Ky, Av);
+        }
+        const double K2 = ksq_f(dKx, dKy, dKz);
+        Dc Nn[4];
+#pragma unroll
+        for (int a = 0; a < 4; a++) Nn[a] = dsc(dl(n[a]), g.norm);
+        const Dc V1 = dl(f0[0]), Tf = dl(f0[1]);
+        Nn[0] = dmk(Nn[0].x - Tf.x, Nn[0].y - Tf.y);
+        Nn[3] = dmk(Nn[3].x - V1.x, Nn[3].y - V1.y);
+        Dc pr = dmk(0.0, 0.0);
+        if (K2 > 0) {
+            const double iK2 = 1.0 / K2;
+            const double dr = dKx * Nn[0].x - dKy * Nn[1].y - dKz * Nn[2].y;
+            const double di = dKx * Nn[0].y + dKy * Nn[1].x + dKz * Nn[2].x;
+            pr = dmk(dr * iK2, di * iK2);
+        }
+        Dc rhs[4];
+        rhs[0] = dmk(-(Nn[0].x - dKx * pr.x), -(Nn[0].y - dKx * pr.y));
+        rhs[1] = dmk(-(Nn[1].x - dKy * pr.y), -(Nn[1].y + dKy * pr.x));
+        rhs[2] = dmk(-(Nn[2].x - dKz * pr.y), -(Nn[2].y + dKz * pr.x));
+        rhs[3] = dmk(-Nn[3].x, -Nn[3].y);
+        const double eh = exl[l] * eyz[c], e1 = exl[L + l] * eyz[T + c];
+        const double ehT = exl[2 * L + l] * eyz[2 * T + c], e1T = exl[3 * L + l] * eyz[3 * T + c];
+        const long o = (long)l * g.sx;
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+            keep[a] = rk_store<R, false>(stage, sc.dt, a < 3 ? eh : ehT, a < 3 ? e1 : e1T, rhs[a], s0[a], a0[a],
+                                         S + a * g.cS + o, Vs + a * g.cS + o, acc + a * g.cS + o);
+    }
+    if constexpr (CHAIN) {
+        __syncthreads();                              // every point has read its mirror values
+        if (on) {
+#pragma unroll
+            for (int a = 0; a < 4; a++) lds[(a * L + l) * T + c] = keep[a];
+        }
+        __syncthreads();
+        const bool sn = gi == 0 || gi == 3;
+        const int nk = g.mx.nk;
+#pragma unroll
+        for (int i = 0; i < E; i++) {                 // conj(w_k) (X_k - i X_{N-k}), see k_sx_inv
+            const int k = FI::in_pos(t, i);
+            const cplx<R> ck = (ok && k < nk && !(sn && k == 0)) ? buf[k * T + c] : czero<R>();
+            const cplx<R> cm = (ok && k > 0 && L - k < nk) ? buf[(L - k) * T + c] : czero<R>();
+            const cplx<R> a = sn ? cm : ck, b = sn ? ck : cm;
+            v[i] = cmul(conjg(w4[k]), mk<R>(a.x + b.y, a.y - b.x));
+        }
+        FI::template run<T, false, NoPad, false, 1>(v, buf + c, t, twl);   // groups past 3 run on their own lines
+        if (ok && gi < 4) {
+#pragma unroll
+            for (int i = 0; i < E; i++) {
+                const int j = FI::out_pos(t, i);
+                Aout[gi * g.cA + (long)j * g.sx] = cscale(v[i], (sn && j >= L / 2) ? R(-1) : R(1));
+            }
+        }
+    }
+}
+
+template <typename R, int L, int T>
+static int launch_sxsplit(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc,
+                          const cplx<R>* tw, const cplx<R>* tw4, const StageCoef* sc, hipStream_t st, bool chain)
+{
+    using X = XSplit<R, L, T, 1>;
+    constexpr size_t lds = X::lds + L * sizeof(cplx<R>);
+    static_assert(X::NT <= 1024 && lds <= 160 * 1024, "split x-forward shape");
+    const dim3 grid(g.my.nk * ((g.nkz + T - 1) / T), g.nbox);
+    auto go = [&](auto k) -> int {
+        if (lds > 64 * 1024)
+            TH_CHECK_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL(k, grid, dim3(X::NT), lds, st, g, D, Aout, S, Vs, acc, tw, tw4, sc);
+        TH_CHECK_HIP(hipGetLastError());
+        return OK;
+    };
+    return chain ? go(k_sx_split<R, L, T, true>) : go(k_sx_split<R, L, T, false>);
+}
+
 template <typename R, int L, int T, int MODE>
 static int launch_xsplit(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc,
                          const cplx<R>* tw, const StageCoef* sc, hipStream_t st, bool chain)

@@ -29,4 +29,17 @@ int d_xsplit<float, 1>(const FG& g, const cplx<float>* D, cplx<float>* Aout, cpl
     return xsplit<1>(g, D, Aout, S, Vs, acc, tw, sc, st, chain);
 }
 
+template <>
+int d_sxsplit<float>(const FG& g, const cplx<float>* D, cplx<float>* Aout, cplx<float>* S, cplx<float>* Vs, cplx<float>* acc,
+                     const cplx<float>* tw, const cplx<float>* tw4, const StageCoef* sc, hipStream_t st, bool chain)
+{
+    constexpr int T = 64 / sizeof(cplx<float>);
+#define C_(n) case n: return launch_sxsplit<float, n, (n == 128 && T > 4) ? T / 2 : T>(g, D, Aout, S, Vs, acc, tw, tw4, sc, st, chain);
+    switch (g.N1) {
+        C_(16) C_(24) C_(32) C_(48) C_(64) C_(96) C_(128)
+        default: set_error("split x-forward: N1 %d unsupported", g.N1); return E_UNSUPPORTED;
+    }
+#undef C_
+}
+
 }  // namespace th

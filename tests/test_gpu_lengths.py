@@ -133,6 +133,39 @@ def test_many_boxes_equal_one_box(ctx, N, boxes, prec):
 
 
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("fp32", 1e-5)])
+def test_chained_rb_step_after_other_uses_of_the_state(ctx, prec, tol):
+    """Short RB boxes step chained: what else uses the state's buffers between steps must not reach the next step, and
+    the stage field stays readable."""
+    from tarang_amd import Plan, State, abi
+    N = (32, 24, 48)
+    print(N, prec, flush=True)
+    o = Oracle(N, basis="SCFT")
+    p = Plan(ctx, N, basis="SCFT", precision=prec)
+    F = o.ic_random(7, E0=0.5, kp=3.0) + [o.ic_random_scalar(4, 1e-2)]
+    s = State(p, abi.TH_RB)
+    s.upload([p.to_dev(v) for v in F])
+
+    def step_and_check(what):
+        s.step(1e-3, Ra=1e4, Pr=1.0, steps=1)
+        o.rk4_rb(F[:3], F[3], 1e4, 1.0, 1e-3, steps=1)
+        m = max(np.abs(v).max() for v in F)
+        for got, ref in zip(s.download(), F):
+            assert np.abs(got.cpu().numpy() - ref).max() <= tol * m, what
+
+    step_and_check("start")
+    step_and_check("again")
+    assert all(np.isfinite(b.cpu().numpy()).all() for b in s.download_buffer(1))
+    for stage in (1, 2, 3, 4):
+        s.profile_passes(1e-3, Ra=1e4, Pr=1.0, stage=stage, nrep=2)
+    step_and_check("profile")
+    s.tune(1e-3, Ra=1e4, Pr=1.0, nrep=1)
+    step_and_check("tune")
+    F = [0.5 * v for v in F]
+    s.upload([p.to_dev(v) for v in F])
+    step_and_check("upload")
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-12), ("fp32", 1e-5)])
 @pytest.mark.parametrize("N", [(16, 32, 24), (24, 64, 64), (32, 16, 128)])
 def test_short_lines_keep_the_last_stage_field(ctx, N, prec, tol):
     """The input of the last RK4 stage after a step, from the oracle's step with a force of zero supply; NS, and MHD's
