@@ -1027,11 +1027,15 @@ __global__ __launch_bounds__(T * P) void k_sx_fwd_rb(FG g, const cplx<R>* __rest
 // energy-transfer epilogue: x-forward of the 9 ET product lines, N_i = sum_j i K_j F(H_j G_i), then
 // 2 mult Re(N . U*) binned by shell (Get_shell_index over radii) separately for |K| <= kmax_inside
 // (Shell_mult_all) and |K| > kmax_inside (which only Shell_mult_single counts).
+//
+// One component i per workgroup (blockIdx.z): three products each and a third of the accumulators, so that a 128^3
+// box is 1530 workgroups instead of 510 and more of them fit a CU; and the shell search reads each radius once for all
+// points of a thread.  128^3 FP64 35.7 -> 30.9 us; 15 givers 96^3 FP64 1769 -> 1455 us, 256^3 FP32 7.76 -> 6.89 ms.
 // ------------------------------------------------------------------------------------------
 template <typename R, int L, int P, int T>
 __global__ __launch_bounds__(T * P) void k_fx_fwd_et(FG g, const cplx<R>* __restrict__ D, const cplx<R>* __restrict__ U,
                                                      const cplx<R>* __restrict__ tw, const double* __restrict__ radii,
-                                                     int nr, int kin, double* __restrict__ partial)
+                                                     int nr, int nc, int kin, double* __restrict__ partial)
 {
     using F = LineFFT<R, L, P, -1>;
     constexpr int E = F::E;
@@ -1039,86 +1043,82 @@ __global__ __launch_bounds__(T * P) void k_fx_fwd_et(FG g, const cplx<R>* __rest
     __shared__ cplx<R> twl[L];
     stage_tw<R, L>(twl, tw);
     __syncthreads();
-    extern __shared__ double bins[];      // 2 nr doubles: |K| <= kin binned by shell, then |K| > kin by shell
-    for (int b = threadIdx.x; b < 2 * nr; b += T * P) bins[b] = 0.0;
+    // 2 nr bins: |K| <= kin by shell, then |K| > kin by shell; nc copies of each, as the neighbouring columns of a row
+    // mostly add to one shell
+    extern __shared__ double bins[];
+    for (int b = threadIdx.x; b < 2 * nr * nc; b += T * P) bins[b] = 0.0;
     const int c = threadIdx.x % T, t = threadIdx.x / T;
     const int ntz = (g.nkz + T - 1) / T;
     const int cy = blockIdx.x / ntz;
     const int cz = (blockIdx.x % ntz) * T + c;
     const bool ok = cz < g.nkz;
     const long m = (long)cy * g.KZP + cz;
-    D += blockIdx.y * g.bA;
+    const int comp = blockIdx.z;
+    D += blockIdx.y * g.bA + 3 * comp * g.cA;
+    U += comp * g.cS;
     const R Ky = (R)(ky_of(ll(g.my, cy), g.N2) * g.f2);
     const R Kz = (R)(cz * g.f3);
-    cplx<R> Nacc[3][E];
+    cplx<R> N[E];
 #pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-        for (int i = 0; i < E; i++) Nacc[a][i] = czero<R>();
+    for (int i = 0; i < E; i++) N[i] = czero<R>();
     auto load = [&](int p, cplx<R> (&v)[E]) {
         const cplx<R>* src = D + p * g.cA + m;
 #pragma unroll
         for (int i = 0; i < E; i++) v[i] = ok ? src[(long)F::in_pos(t, i) * g.sx] : czero<R>();
     };
-    // the next product's tile is loaded before this one's transform where that costs no wave per SIMD
-    constexpr bool XPRE = (sizeof(R) == 8) == (E == 8);
-    cplx<R> nv[E];
-    if constexpr (XPRE) load(0, nv);
+    cplx<R> nv[E];                        // the next product's tile, loaded before this one's transform
+    load(0, nv);
 #pragma unroll 1
-    for (int p = 0; p < 9; p++) {
+    for (int p = 0; p < 3; p++) {         // P(comp, p) = G_comp H_p -> N_comp += i K_p P
         cplx<R> v[E];
-        if constexpr (XPRE) {
 #pragma unroll
-            for (int i = 0; i < E; i++) v[i] = nv[i];
-            if (p < 8) load(p + 1, nv);
-        } else {
-            load(p, v);
-        }
+        for (int i = 0; i < E; i++) v[i] = nv[i];
+        if (p < 2) load(p + 1, nv);
         F::template run<T, false, NoPad, true>(v, lds + c, t, twl + opaque_zero());
-        const int pi = p / 3, pj = p % 3;        // P(pi,pj) = G_pi H_pj -> N_pi += i K_pj P
-        R al[3], be[3];
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-            al[a] = (a == pi && pj == 0) ? R(1) : R(0);
-            be[a] = (a == pi && pj != 0) ? (pj == 1 ? Ky : Kz) : R(0);
-        }
+        const R al = p == 0 ? R(1) : R(0), be = p == 0 ? R(0) : p == 1 ? Ky : Kz;
 #pragma unroll
         for (int i = 0; i < E; i++) {
             if (xdrop<L, P, E, F::RL>(i)) continue;
             const R Kx = (R)(kx_four(F::out_pos(t, i), g.N1) * g.f1);
-#pragma unroll
-            for (int a = 0; a < 3; a++) acc_iK(Nacc[a][i], al[a] * Kx + be[a], v[i]);
+            acc_iK(N[i], al * Kx + be, v[i]);
         }
     }
     __syncthreads();
     if (ok) {
         const double dKy = ky_of(ll(g.my, cy), g.N2) * g.f2, dKz = cz * g.f3;
         const int l2 = ll(g.my, cy);
+        double km[E];
+        int b[E];
+#pragma unroll
+        for (int i = 0; i < E; i++) {
+            km[i] = kmag_f(kx_four(F::out_pos(t, i), g.N1) * g.f1, dKy, dKz);
+            b[i] = nr;
+        }
+        for (int j = nr - 1; j >= 0; j--) {          // first shell j with |K| <= radii[j]
+            const double r = radii[j];
+#pragma unroll
+            for (int i = 0; i < E; i++)
+                if (!xdrop<L, P, E, F::RL>(i)) b[i] = km[i] <= r ? j : b[i];
+        }
 #pragma unroll
         for (int i = 0; i < E; i++) {
             const int l = F::out_pos(t, i);
-            if (xdrop<L, P, E, F::RL>(i) || !lkept(g.mx, l)) continue;
-            const int kx = kx_four(l, g.N1);
-            const double km = kmag_f(kx * g.f1, dKy, dKz);
+            if (xdrop<L, P, E, F::RL>(i) || !lkept(g.mx, l) || b[i] >= nr) continue;
             // Multiplicity_factor_FOUR four_inline.h:347-365
             double f = (cz > 0) ? 1.0 : 0.5;
-            if (kx == g.N1 / 2 || ky_of(l2, g.N2) == g.N2 / 2) f *= 2;
-            const long idx = (long)lq(g.mx, l) * g.sx + m;
-            double s = 0;
-#pragma unroll
-            for (int a = 0; a < 3; a++) {
-                cplx<R> u = U[a * g.cS + idx];
-                s += (double)Nacc[a][i].x * (double)u.x + (double)Nacc[a][i].y * (double)u.y;
-            }
-            s *= 2 * f * g.norm;
-            int b = 0;
-            while (b < nr && !(km <= radii[b])) b++;
-            if (b >= nr) continue;
-            atomicAdd(&bins[(km <= (double)kin) ? b : nr + b], s);
+            if (kx_four(l, g.N1) == g.N1 / 2 || ky_of(l2, g.N2) == g.N2 / 2) f *= 2;
+            const cplx<R> u = U[(long)lq(g.mx, l) * g.sx + m];
+            const double s = (double)N[i].x * (double)u.x + (double)N[i].y * (double)u.y;
+            atomicAdd(&bins[((km[i] <= (double)kin) ? b[i] : nr + b[i]) * nc + (threadIdx.x & (nc - 1))], s * (2 * f * g.norm));
         }
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < 2 * nr; b += T * P) partial[((long)blockIdx.y * gridDim.x + blockIdx.x) * (2 * nr) + b] = bins[b];
+    const long q = ((long)blockIdx.y * 3 + comp) * gridDim.x + blockIdx.x;
+    for (int b = threadIdx.x; b < 2 * nr; b += T * P) {
+        double a = bins[b * nc];
+        for (int k = 1; k < nc; k++) a += bins[b * nc + k];
+        partial[q * (2 * nr) + b] = a;
+    }
 }
 
 // compact <-> reference layout.  Both are bound by memory (a download writes the whole reference array, non-temporally:
@@ -1251,10 +1251,13 @@ static int launch_xfwd_et(const FG& g, const cplx<R>* D, const cplx<R>* U, const
 {
     constexpr int E = xfwd_E(L), P = L / E, T = xfwd_T<R, L, 0>();
     const int ntz = (g.nkz + T - 1) / T;
-    *nblk = g.my.nk * ntz;
+    *nblk = 3 * g.my.nk * ntz;
     if (!partial) return OK;
-    hipLaunchKernelGGL((k_fx_fwd_et<R, L, P, T>), dim3(*nblk, g.nbox), dim3(T * P), 2 * nr * sizeof(double), st, g, D, U, tw,
-                       radii, nr, kin, partial);
+    // copies of the bins, 4 KB of LDS: 256^3 FP32, 15 givers, with 1 / 2 / 4 / 8 copies 7.19 / 6.96 / 6.89 / 6.92 ms,
+    // 192^3 FP64 (eight cost a workgroup per CU) 6.63 / 6.60 / 6.60 / 6.89
+    const int nc = nr <= 64 ? 4 : nr <= 128 ? 2 : 1;
+    hipLaunchKernelGGL((k_fx_fwd_et<R, L, P, T>), dim3(g.my.nk * ntz, g.nbox, 3), dim3(T * P), 2 * nr * nc * sizeof(double), st, g, D,
+                       U, tw, radii, nr, nc, kin, partial);
     TH_CHECK_HIP(hipGetLastError());
     return OK;
 }

@@ -32,8 +32,10 @@ def state(ctx, N, prec, physics, seed):
     return s
 
 
-# planes of 16 to 64 points in one launch and not, more givers than one launch takes (64^3 FP64: 10), odd remainders
-SIZES = [((16, 16, 16), 5), ((24, 48, 32), 11), ((64, 64, 64), 21), ((32, 96, 96), 9), ((48, 128, 24), 7)]
+# planes of 16 to 64 points in one launch and not, more givers than one launch takes (64^3 FP64: 10), odd remainders,
+# the numbers of shells at which the bins have fewer copies
+SIZES = [((16, 16, 16), 5), ((24, 48, 32), 11), ((64, 64, 64), 21), ((32, 96, 96), 9), ((48, 128, 24), 7),
+         ((32, 24, 32), 70), ((32, 24, 32), 140)]
 
 
 @pytest.mark.parametrize("prec,tol", [("fp64", 1e-11), ("fp32", 2e-5)])
@@ -41,7 +43,7 @@ SIZES = [((16, 16, 16), 5), ((24, 48, 32), 11), ((64, 64, 64), 21), ((32, 96, 96
 def test_givers_together_and_alone(ctx, N, nsh, prec, tol):
     print(f"transfer {prec} N={N} nsh={nsh}", flush=True)
     s = state(ctx, N, prec, 0, 7)
-    radii = np.concatenate([np.arange(nsh, dtype=float) * 1.25, [1e4]])
+    radii = np.concatenate([np.arange(nsh, dtype=float) * min(1.25, 20.0 / nsh), [1e4]])
     Pi, T = s.flux_shell_tr(radii)
     again = s.flux_shell_tr(radii)
     scale = np.abs(T).max()
