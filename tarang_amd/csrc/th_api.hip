@@ -1,5 +1,5 @@
 // th_api.hip -- the C-ABI (include/tarang_hip.h): contexts, plans, the boundary transforms and
-// spectral operators, the plain GPU step (the reference's operation sequence), diagnostics and ICs.
+// spectral operators, the plain step's general path (the reference's operation sequence), diagnostics and ICs.
 #include <math.h>
 #include <stdarg.h>
 #include <stdio.h>

@@ -2,8 +2,8 @@
 // device-resident states (single boxes and batched boxes of one size), the hipGraph-captured RK4
 // step, per-box stage coefficients, energy transfer from shell givers, the per-pass profiler, the
 // launch-shape autotuner, the uneven-box ensemble and the forced step.  The five passes and their
-// kernels are described in th_fused_kern.hpp; NS and MHD states step chained (four launches per stage: each
-// stage's x-forward also performs the next stage's x-inverse).
+// kernels are described in th_fused_kern.hpp; NS, MHD and short RB states step chained (each stage's
+// x-forward also performs the next stage's x-inverse: four launches per stage, two on short boxes).
 #include <stdio.h>
 #include <algorithm>
 #include <array>
@@ -142,8 +142,8 @@ struct th_state {
     int var[NPASS] = {0, 0, 0, 0, 0};   // launch-shape variant per pass (autotuner)
     bool plane = false;          // passes 2-4 as one launch, X1 -> X3 (th_plane.hpp); the y passes launch nothing
     bool split = false;          // x-forward with the products side by side (th_plane.hpp)
-    // Chained step (NS, MHD, RB with the split x-forward): each stage's x-forward also does the next stage's x-inverse, so a
-    // step runs 4 passes per stage; X1 must then hold the x-inverse of S when a step starts (chain_ok), which a
+    // Chained step (NS, MHD, RB with the split x-forward): each stage's x-forward also does the next stage's
+    // x-inverse; X1 must then hold the x-inverse of S when a step starts (chain_ok), which a
     // single x-inverse launch restores after anything else has used the buffers or changed S.
     bool chain_ok = false;
     bool graph_chained = false;
@@ -210,7 +210,7 @@ static bool split_ok(const FG& g, int physics)
     return pts <= (g.N1 <= 48 ? 600000 : g.N1 <= 64 ? 500000 : 400000);
 }
 
-// Products of the pipelines (numbered as ZProd in th_fused_kern.hpp), in an order that hands operands on: each
+// Products of the pipelines (numbered as k_fz's in th_fused_kern.hpp), in an order that hands operands on: each
 // rotation step's last operand is the next one's first (NS, RB) or its first y (MHD)
 static const PlaneTab& plane_tab(int physics)
 {
@@ -505,7 +505,7 @@ static void diss_of(const th_state* s, const th_phys* ph, double* d0, double* d1
 // reference subtracts the force F of the stage field from nlin before the projection, so the stage's
 // rhs gains +P(F), P the projection.  Every stage output (the stage field, the accumulator, the state
 // in stage 4) is linear in the rhs and F lives on a few thousand band modes, so instead of changing
-// the x-forward epilogue, k_force_pre stores P(F) of the stage input for the band box before the
+// the x-forward epilogue, k_force_in stores P(F) of the stage input for the band box before the
 // stage's passes, and k_force_out adds the stage's share of it afterwards:
 //   stage 1: Vs += dt/2 e_h P(F), acc += dt/6 e_1 P(F)      stage 2: Vs += dt/2 P(F), acc += dt/3 e_h P(F)
 //   stage 3: Vs += dt e_h P(F),   acc += dt/3 e_h P(F)      stage 4: S += dt/6 P(F)

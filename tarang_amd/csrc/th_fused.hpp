@@ -131,7 +131,7 @@ bool plane_ok(const FG& g);
 template <typename R>
 int d_plane(const FG& g, const PlaneTab& tab, int ngrp, const cplx<R>* A, cplx<R>* D, long bD, const cplx<R>* tw2,
             const cplx<R>* twL, const cplx<R>* twN, hipStream_t st);
-// The x-forward with the products side by side (N1 <= 128), NS (MODE 0) and MHD (MODE 1); chained for every N1
+// The x-forward with the products side by side (N1 <= 128), NS (MODE 0) and MHD (MODE 1)
 template <typename R, int MODE>
 int d_xsplit(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw,
              const StageCoef* sc, hipStream_t st, bool chain);
@@ -139,7 +139,7 @@ template <typename R>   // RB
 int d_sxsplit(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw,
               const cplx<R>* tw4, const StageCoef* sc, hipStream_t st, bool chain);
 
-// Operand and product table of a pipeline (ZProd of th_fused_kern.hpp as plain numbers): product j of rotation step r
+// Operand and product table of a pipeline (k_fz's of th_fused_kern.hpp as plain numbers): product j of rotation step r
 // multiplies input x[r] by input y[r][j] into output o[r][j]; operands are kept from one product to the next where the order allows it.
 struct PlaneTab {
     signed char npr;

@@ -13,8 +13,9 @@
 //                  exp(-nu K^2 a dt) and the RK4 stage update (single_time_step.cc, Compute_RK4_parts)
 // MHD uses the Elsasser form (compute_nlin_VF_MHD.cc) with 6 inverse and 9 product lines; the energy
 // transfer (ET_compute_nlin.cc) uses helper U and a shell-masked giver G and bins 2 mult Re(N U*)
-// (four_ET.cc) in the pass-5 epilogue instead of writing N.  Chained NS and MHD steps fold pass 1 of the
-// next stage into pass 5 (k_fx_fwd CHAIN).  Each pipeline buffer is written once and read once by the next
+// (four_ET.cc) in the pass-5 epilogue instead of writing N.  Chained steps fold pass 1 of the next stage into pass 5
+// (k_fx_fwd CHAIN); short boxes run passes 2 to 4 as one launch and pass 5 with its products side by side
+// (th_plane.hpp).  Each pipeline buffer is written once and read once by the next
 // pass, so outputs go out with non-temporal stores and the y and z passes load non-temporally.
 
 #pragma once
@@ -22,8 +23,6 @@
 #include "th_fused.hpp"
 
 namespace th {
-
-template <typename R> __device__ __forceinline__ cplx<R> ld(const cplx<R>* p) { return *p; }
 
 // ------------------------------------------------------------------------------------------
 // pass 1: x-inverse.  MODE 0: copy comps; 1: Elsasser Z+ = U + B (comps 0-2), Z- = U - B (3-5);
@@ -154,20 +153,7 @@ __global__ __launch_bounds__(T * P) void k_fy_inv(FG g, const cplx<R>* __restric
 // MODE 0 (NS):  in u0..u2,            out u0u0 u1u1 u2u2 u0u1 u1u2 u2u0          (RSprod.cc:52-77)
 // MODE 1 (MHD): in Z+0..2, Z-0..2,    out P(i,j) = Z+_i Z-_j at 3i+j             (RSprod.cc:117-151)
 // MODE 2 (ET):  in H0..2,  G0..2,     out P(i,j) = G_i H_j at 3i+j               (ET_RSprod.cc:49-85)
-template <int MODE> struct ZProd;
-template <> struct ZProd<0> {
-    static constexpr int NIN = 3, NOUT = 6;
-};
-template <> struct ZProd<1> {
-    static constexpr int NIN = 6, NOUT = 9;
-};
-template <> struct ZProd<2> {
-    static constexpr int NIN = 6, NOUT = 9;
-};
 // MODE 3 (RB): in V1 V2 V3 T, out V1V1 V2V2 V3V3 V1V2 V2V3 V3V1 V1T V2T V3T (compute_nlin_SF.cc:80-177)
-template <> struct ZProd<3> {
-    static constexpr int NIN = 4, NOUT = 9;
-};
 
 // Lane t of a z line holds the points at positions t + P m, m = 0..E-1, in a register order fixed
 // by the radix Rr of the FFT stage that reads (first stage) or writes (last stage) them.
@@ -191,7 +177,6 @@ __global__ __launch_bounds__(TZ * P) void k_fz(FG g, const cplx<R>* __restrict__
     using FI = LineFFT<R, LZ, P, +1, R16>;
     using FF = LineFFT<R, LZ, P, -1, R16>;
     using Lay = std::conditional_t<R16, ZPad16<LZ>, ZPad<LZ>>;
-    using ZP = ZProd<MODE>;
     constexpr int E = FI::E;
     static_assert(64 % P == 0, "a z line's threads must share one wavefront");
     constexpr int LZS = Lay::line;   // padded line stride in LDS
@@ -486,14 +471,6 @@ __device__ __forceinline__ cplx<R> rk_store(int stage, double dt, double eh, dou
     }
     if (wvs) *Vs = out;
     return out;
-}
-template <typename R>
-__device__ __forceinline__ void rk_update(int stage, double dt, double eh, double e1, const Dc& rhs, cplx<R>* S,
-                                          cplx<R>* Vs, cplx<R>* acc)
-{
-    const cplx<R> s0 = *S;
-    const cplx<R> a0 = stage > 1 ? *acc : czero<R>();
-    rk_store<R>(stage, dt, eh, e1, rhs, s0, a0, S, Vs, acc);
 }
 
 // first register after (i) that xdrop keeps, or -1

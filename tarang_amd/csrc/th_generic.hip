@@ -1,7 +1,8 @@
 // th_generic.hip -- full (unpruned) transform passes and spectral element-wise kernels on the
 // reference layout (N1, N2, N3/2+1).  These back the boundary calls th_forward / th_inverse /
-// th_deriv ... and the "plain" GPU step that keeps the reference's operation sequence
-// (trunk/lib/IncFlow/nlin_calc/compute_nlin.cc:58-108): every pass reads and writes a whole array.
+// th_deriv ... and the plain step's general path, which keeps the reference's operation sequence
+// (trunk/lib/IncFlow/nlin_calc/compute_nlin.cc:58-108; th_plain.hpp has the fused one): every pass reads and writes a
+// whole array.
 #include <math.h>
 #include "th_fft.hpp"
 #include "th_internal.hpp"
