@@ -863,7 +863,9 @@ template <typename R> static int do_step_plain(th_plan* p, int physics, int sche
     if (plain_fast(p, physics, nullptr)) {
         cplx<R>* F[6] = {};
         for (int q = 0; q < o.nc; q++) F[q] = CP(R, fields[q]);
-        return plain_step<R>(p, physics, scheme, F, dt, nu, physics == TH_MHD ? eta : kap, nullptr, nullptr, nullptr);
+        const int r = plain_step<R>(p, physics, scheme, F, dt, nu, physics == TH_MHD ? eta : kap, nullptr, nullptr, nullptr);
+        if (r != E_NOMEM) return r;
+        p->plain.release();      // no room for its workspace: the operation sequence
     }
     for (int q = 0; q < o.nc; q++) {
         o.F[q] = CP(R, fields[q]);
@@ -892,7 +894,9 @@ template <typename R> static int do_step_plain_forced(th_plan* p, int scheme, vo
         for (int c = 0; c < 3; c++) o.keep[c] = CP(R, last[c]);
     if (plain_fast(p, TH_NS, fb)) {
         cplx<R>* F[3] = {CP(R, V[0]), CP(R, V[1]), CP(R, V[2])};
-        return plain_step<R>(p, TH_NS, scheme, F, dt, ph->nu, 0.0, fb, nullptr, o.keep);
+        const int r = plain_step<R>(p, TH_NS, scheme, F, dt, ph->nu, 0.0, fb, nullptr, o.keep);
+        if (r != E_NOMEM) return r;
+        p->plain.release();
     }
     for (int q = 0; q < 3; q++) {
         o.F[q] = CP(R, V[q]);
@@ -918,7 +922,9 @@ template <typename R> static int do_step_plain_forced_mhd(th_plan* p, int scheme
         for (int q = 0; q < 6; q++) F[q] = CP(R, q < 3 ? U[q] : B[q - 3]);
         // each part only when its level per mode exceeds MYEPS (compute_rhs above)
         const bool u = fu->proc == 3 || fu->per_mode > 1e-15, w = fw->proc == 3 || fw->per_mode > 1e-15;
-        return plain_step<R>(p, TH_MHD, scheme, F, dt, ph->nu, ph->eta, u ? fu : nullptr, w ? fw : nullptr, o.keep);
+        const int r = plain_step<R>(p, TH_MHD, scheme, F, dt, ph->nu, ph->eta, u ? fu : nullptr, w ? fw : nullptr, o.keep);
+        if (r != E_NOMEM) return r;
+        p->plain.release();
     }
     for (int q = 0; q < 6; q++) {
         o.F[q] = CP(R, q < 3 ? U[q] : B[q - 3]);

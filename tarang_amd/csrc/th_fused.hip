@@ -73,6 +73,14 @@ FG make_fg(const Geo& geo, int prec)
 
 using namespace th;
 
+// The plain steps' workspace.  Cleared and filled by kernels: a call on a stream under capture must record no memset node
+// and no copy from the host's stack.
+__global__ void k_clear(double* p, size_t n)
+{
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = 0.0;
+}
+__global__ void k_put_coef(StageCoef c, StageCoef* p) { *p = c; }
+
 int PlainBufs::ensure(size_t esz, size_t nX, size_t nY, size_t nC, size_t nF, hipStream_t st)
 {
     auto grow = [&](void** q, size_t bytes, bool clear) -> int {
@@ -80,10 +88,14 @@ int PlainBufs::ensure(size_t esz, size_t nX, size_t nY, size_t nC, size_t nF, hi
         *q = nullptr;
         if (hipMalloc(q, bytes) != hipSuccess) {
             *q = nullptr;
+            (void)hipGetLastError();
             set_error("plain step: workspace allocation of %zu bytes failed", bytes);
             return E_NOMEM;
         }
-        if (clear) TH_CHECK_HIP(hipMemsetAsync(*q, 0, bytes, st));
+        if (clear) {
+            hipLaunchKernelGGL(k_clear, dim3(2048), dim3(256), 0, st, (double*)*q, bytes / sizeof(double));
+            TH_CHECK_HIP(hipGetLastError());
+        }
         return OK;
     };
     if (nX * esz > bX) { bX = 0; TRY(grow(&X, nX * esz, true)); bX = nX * esz; }
@@ -103,7 +115,8 @@ int PlainBufs::ensure(size_t esz, size_t nX, size_t nY, size_t nC, size_t nF, hi
         c.stage = 1;
         c.dt = 2.0;
         TRY(grow(&coef, sizeof c, false));
-        TH_CHECK_HIP(hipMemcpy(coef, &c, sizeof c, hipMemcpyHostToDevice));
+        hipLaunchKernelGGL(k_put_coef, dim3(1), dim3(1), 0, st, c, (StageCoef*)coef);
+        TH_CHECK_HIP(hipGetLastError());
     }
     return OK;
 }
@@ -182,8 +195,9 @@ static std::string tune_key(const th_state* s)
 
 // Short boxes (th_plane.hpp).
 //
-// Passes 2 to 4 as one launch, by the grid alone (a box computes the same bits alone and in an ensemble): N2 and N3 up to 128 with at most 8192 points per plane (74 KB of LDS in FP64), and in
-// FP64 planes past 4608 points only on long boxes, where the three passes wait on memory rather than on launches.
+// Passes 2 to 4 as one launch, by the grid alone (a box computes the same bits alone and in an ensemble): N2 and N3 up
+// to 128 with at most 8192 points per plane (74 KB of LDS in FP64), and in FP64 planes past 4608 points only on long
+// boxes, where the three passes wait on memory rather than on launches.
 // us per step, three passes / plane pass: 32^3 FP64 160 / 98, 64^3 FP64 174 / 125, eight 64^3 FP32 306 / 187,
 // 512 x 64 x 64 FP64 465 / 309, 512 x 128 x 64 FP32 564 / 369; past the line 96^3 FP32 213 / 202 to 248,
 // 128^3 FP64 359 / 479 (one 147 KB plane per CU), 64 x 64 x 128 FP64 178 / 185.
@@ -191,7 +205,7 @@ bool th::plane_ok(const FG& g)
 {
     if (g.N2 > 128 || g.LZ > 64 || g.nkz != g.N3 / 3) return false;
     const int pts = g.N2 * g.N3;
-    return pts <= (g.fp64 && g.N1 < 256 ? 4608 : 8192);
+    return pts <= (g.fp64 && g.N1 < 256 ? 4608 : PLANE_MAX);
 }
 // The x-forward with the products side by side: where one workgroup per tile of columns leaves CUs idle
 // or waiting, that is up to so many kept points in all boxes, and in FP64 on lines to 48 points always (a tile of

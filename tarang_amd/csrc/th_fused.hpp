@@ -127,6 +127,7 @@ template <typename R> int d_scatter(const FG& g, const cplx<R>* S, cplx<R>* ref,
 // Passes 2 to 4 in one launch, A (nin lines) -> D (nout lines), for boxes with plane_ok; ngrp = 3 or nout workgroups
 // per x-plane.  D may not be A; its box stride is bD.
 struct PlaneTab;
+constexpr int PLANE_MAX = 8192;   // points of a plane
 bool plane_ok(const FG& g);
 template <typename R>
 int d_plane(const FG& g, const PlaneTab& tab, int ngrp, const cplx<R>* A, cplx<R>* D, long bD, const cplx<R>* tw2,

@@ -538,23 +538,25 @@ static int launch_plane(const FG& g, const PlaneTab& tab, int ngrp, const cplx<R
     auto k = k_plane<R, L2, LZ>;
     if (lds > 64 * 1024)
         TH_CHECK_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL(k, dim3((unsigned)(g.N1 * g.nbox * ngrp)), dim3(L2 * (LZ / plane_EZ(LZ))), lds, st, g, tab, ngrp, A, D, bD,
-                       tw2, twL, twN);
+    hipLaunchKernelGGL(k, dim3((unsigned)(g.N1 * g.nbox * ngrp)), dim3(L2 * (LZ / plane_EZ(LZ))), lds, st, g, tab, ngrp, A, D,
+                       bD, tw2, twL, twN);
     TH_CHECK_HIP(hipGetLastError());
     return OK;
 }
 
-// ---- dispatch (each translation unit instantiates the half of the plane lengths it names) ----
+// ---- dispatch: the planes that plane_ok can name ----
 template <typename R, int L2>
 static int plane_z(const FG& g, const PlaneTab& tab, int ngrp, const cplx<R>* A, cplx<R>* D, long bD, const cplx<R>* tw2,
                    const cplx<R>* twL, const cplx<R>* twN, hipStream_t st)
 {
-#define C_(n) case n: return launch_plane<R, L2, n>(g, tab, ngrp, A, D, bD, tw2, twL, twN, st);
-    switch (g.LZ) {
-        C_(8) C_(12) C_(16) C_(24) C_(32) C_(48) C_(64)
-        default: set_error("plane pass: N3 %d unsupported", g.N3); return E_UNSUPPORTED;
-    }
+#define C_(n)                                                                                                                   \
+    case n:                                                                                                                     \
+        if constexpr (2 * n * L2 <= PLANE_MAX) return launch_plane<R, L2, n>(g, tab, ngrp, A, D, bD, tw2, twL, twN, st);        \
+        break;
+    switch (g.LZ) { C_(8) C_(12) C_(16) C_(24) C_(32) C_(48) C_(64) }
 #undef C_
+    set_error("plane pass: %d x %d planes unsupported", g.N2, g.N3);
+    return E_UNSUPPORTED;
 }
 
 }  // namespace th
