@@ -287,6 +287,12 @@ static int state_create(th_plan* p, th_state** out, int physics, int nbox)
         delete s;
         return r;
     }
+    // the clears run on the null stream, which the context's non-blocking stream does not wait for
+    if (hipStreamSynchronize(nullptr) != hipSuccess) {
+        set_error("th_state_create: clearing the buffers failed");
+        delete s;
+        return E_HIP;
+    }
     s->plane = plane_ok(g);
     s->split = split_ok(g, physics);
     g.keep3 = keeps_last(s);

@@ -41,10 +41,18 @@ void mean_modes(void* const V[3], size_t esize, double out[3])
 Context::Context(int device) { check(th_ctx_create(&h, device, nullptr), "th_ctx_create"); }
 Context::~Context() { th_ctx_destroy(h); }
 
+// A memset or a device-to-device copy returns before it has run, on the null stream, which the context's non-blocking
+// stream does not wait for: a kernel launched next could be overtaken by the clear of the array it writes.
+static void null_stream_done(hipError_t e, const char* what)
+{
+    hipc(e, what);
+    hipc(hipStreamSynchronize(nullptr), what);
+}
+
 DField::DField(size_t elems, size_t esize) : n_(elems), es_(esize)
 {
     hipc(hipMalloc(&p_, n_ * es_), "hipMalloc");
-    hipc(hipMemset(p_, 0, n_ * es_), "hipMemset");
+    null_stream_done(hipMemset(p_, 0, n_ * es_), "hipMemset");
 }
 DField::~DField()
 {
@@ -64,8 +72,11 @@ DField& DField::operator=(DField&& o) noexcept
 }
 void DField::upload(const void* host) { hipc(hipMemcpy(p_, host, bytes(), hipMemcpyHostToDevice), "upload"); }
 void DField::download(void* host) const { hipc(hipMemcpy(host, p_, bytes(), hipMemcpyDeviceToHost), "download"); }
-void DField::copy_from(const DField& o) { hipc(hipMemcpy(p_, o.p_, bytes(), hipMemcpyDeviceToDevice), "copy"); }
-void DField::zero() { hipc(hipMemset(p_, 0, bytes()), "zero"); }
+void DField::copy_from(const DField& o)
+{
+    null_stream_done(hipMemcpy(p_, o.p_, bytes(), hipMemcpyDeviceToDevice), "copy");
+}
+void DField::zero() { null_stream_done(hipMemset(p_, 0, bytes()), "zero"); }
 
 // ---------------------------------------------------------------- CVF
 CVF::CVF(Context& ctx, const Grid& g) : grid(g), ctx_(ctx)
