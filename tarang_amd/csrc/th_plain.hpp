@@ -101,6 +101,16 @@ __global__ __launch_bounds__(256) void k_plain_stage(FG g, FastDiv dH, FastDiv d
                                                      FieldPtrs v0, FieldPtrs in, FieldPtrs out, const cplx<R>* __restrict__ rhs,
                                                      cplx<R>* __restrict__ acc)
 {
+    // every product and sum rounded by itself, as the separate operations of the general path round them
+#pragma clang fp contract(off)
+    auto sc = [](Dc a, double b) {
+#pragma clang fp contract(off)
+        return dmk(a.x * b, a.y * b);
+    };
+    auto add = [](Dc a, Dc b) {
+#pragma clang fp contract(off)
+        return dmk(a.x + b.x, a.y + b.y);
+    };
     const unsigned n = (unsigned)g.N1 * g.N2 * dH.d;
     for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         const unsigned rw = fdiv(i, dH), x = fdiv(rw, dN2);
@@ -140,15 +150,15 @@ __global__ __launch_bounds__(256) void k_plain_stage(FG g, FastDiv dH, FastDiv d
             const double eh = c < 3 ? h0 : h1, e1 = eh * eh;
             const Dc V = dl(s[c]);
             Dc o;
-            if (kind == 0) o = dsc(dadd(V, dsc(q[c], dt)), e1);
-            else if (kind == 1) o = dsc(dadd(V, dsc(q[c], 0.5 * dt)), eh);
-            else if (kind == 2) o = dadd(dsc(V, eh), dsc(q[c], 0.5 * dt));
-            else if (kind == 4) o = dadd(dsc(V, e1), dadd(dl(a[c]), dsc(q[c], dt / 6)));
-            else o = dsc(dadd(dsc(V, eh), dsc(q[c], dt)), eh);
+            if (kind == 0) o = sc(add(V, sc(q[c], dt)), e1);
+            else if (kind == 1) o = sc(add(V, sc(q[c], 0.5 * dt)), eh);
+            else if (kind == 2) o = add(sc(V, eh), sc(q[c], 0.5 * dt));
+            else if (kind == 4) o = add(sc(V, e1), add(dl(a[c]), sc(q[c], dt / 6)));
+            else o = sc(add(sc(V, eh), sc(q[c], dt)), eh);
             ((cplx<R>*)out.v[c])[i] = ds<R>(o);
             if (kept && acc) {
-                if (kind == 1) acc[c * g.cS + j] = ds<R>(dsc(q[c], dt / 6 * e1));
-                else if (kind == 2 || kind == 3) acc[c * g.cS + j] = ds<R>(dadd(dl(a[c]), dsc(q[c], dt / 3 * eh)));
+                if (kind == 1) acc[c * g.cS + j] = ds<R>(sc(q[c], dt / 6 * e1));
+                else if (kind == 2 || kind == 3) acc[c * g.cS + j] = ds<R>(add(dl(a[c]), sc(q[c], dt / 3 * eh)));
             }
         }
     }
