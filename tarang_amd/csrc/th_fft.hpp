@@ -38,9 +38,10 @@ constexpr Sched sched3(int L, int E)
 
 // Greedy radix schedule: each radix must divide the remaining length and the points per thread.
 // Radix 16 only on request (it needs all 16 points of a butterfly live at once).
-constexpr Sched make_sched(int L, int E, bool r16 = false)
+// pf: with the radix 6 and 12 schedules
+constexpr Sched make_sched(int L, int E, bool r16 = false, bool pf = true)
 {
-    if (sched3(L, E).n > 0) return sched3(L, E);
+    if (pf && sched3(L, E).n > 0) return sched3(L, E);
     Sched s{0, {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0}};
     int m = L;
     while (m > 1) {
@@ -104,10 +105,15 @@ template <int L> struct ZPad16 {
 struct NoPad {
     static constexpr int map(int, int A) { return A; }
 };
-template <int L> struct ZPad {
+template <int L, bool FORCED = false> struct ZPad {   // FORCED: for schedules without radix 6 and 12
     static constexpr int code(int s)
     {
         // sh * 16 + k; 0 = identity
+        if (FORCED && L % 3 == 0)
+            return L == 24 || L == 48 ? (s <= 1 ? 2 * 16 + 1 : 0)
+                 : L == 96 ? (s <= 2 ? 3 * 16 + 1 : 0)
+                 : L == 192 ? (s == 0 || s == 2 ? 4 * 16 + 1 : s == 1 ? 2 * 16 + 1 : 0)
+                 : 0;
         return L == 12 ? (s == 0 ? 1 * 16 + 1 : 0)
              : L == 16 ? (s == 0 ? 3 * 16 + 1 : 0)
              : L == 24 ? (s == 0 ? 1 * 16 + 1 : 0)
@@ -127,7 +133,7 @@ template <int L> struct ZPad {
         for (int s = 0; s < 8; s++) m = map(s, L - 1) + 1 > m ? map(s, L - 1) + 1 : m;
         return m;
     }
-    static constexpr int line = L == 12 ? 18 : L == 16 ? 18 : L == 24 ? 38 : L == 32 ? 36 : L == 48 ? 60 : L == 64 ? 72 : L == 96 ? 120 : L == 128 ? 144 : L == 192 ? 208 : L == 256 ? 318 : L + 1;
+    static constexpr int line = FORCED && L == 12 ? 13 : FORCED && L == 24 ? 30 : FORCED && L == 192 ? 240 : L == 12 ? 18 : L == 16 ? 18 : L == 24 ? 38 : L == 32 ? 36 : L == 48 ? 60 : L == 64 ? 72 : L == 96 ? 120 : L == 128 ? 144 : L == 192 ? 208 : L == 256 ? 318 : L + 1;
     static_assert(line >= need(), "ZPad line stride too short");
 };
 
@@ -283,9 +289,14 @@ template <int SIGN, typename R> struct DFT<12, SIGN, R> {
 // One line of length L, P cooperating threads, E = L/P points per thread.
 //   before run(): v[i] = x[in_pos(t, i)]       after run(): v[i] = X[out_pos(t, i)]
 // lds points at element 0 of this line; element m lives at lds[m * LS].
-template <typename R, int L, int P, int SIGN, bool R16 = false> struct LineFFT {
+//
+// FORCED: the arithmetic of forced FP32 states (th_state_set_force): schedules without radix 6 and 12, and each twiddle
+// product fused as the compiler chooses in its kernel.  The force of a weak or nearly helical mode amplifies the last bit
+// of the FP32 fields, so a forced result follows every rounding of the passes: on two of 30 random 192^3 inputs
+// other schedules moved it by 1e-6 to 3e-5 (unforced: 5e-8).  Those states therefore stay with one set of roundings.
+template <typename R, int L, int P, int SIGN, bool R16 = false, bool FORCED = false> struct LineFFT {
     static constexpr int E = L / P;
-    static constexpr Sched S = make_sched(L, E, R16);
+    static constexpr Sched S = make_sched(L, E, R16, !FORCED);
     static_assert(L % P == 0, "P must divide L");
     static_assert(S.n > 0, "no radix schedule for (L, E)");
     static constexpr int NST = S.n;
@@ -337,7 +348,8 @@ template <typename R, int L, int P, int SIGN, bool R16 = false> struct LineFFT {
                     // which product is fused is spelled out: left to the compiler it changes with the surrounding
                     // code, and the same line in two kernels would differ in the last bit
                     const cplx<R> q = v[b * Rr + r];
-                    v[b * Rr + r] = mk<R>(fma(q.x, w.x, -(q.y * w.y)), fma(q.x, w.y, q.y * w.x));
+                    if constexpr (FORCED) v[b * Rr + r] = cmul(q, w);
+                    else v[b * Rr + r] = mk<R>(fma(q.x, w.x, -(q.y * w.y)), fma(q.x, w.y, q.y * w.x));
                 }
             }
             DFT<Rr, SIGN, R>::run(&v[b * Rr]);

@@ -457,11 +457,30 @@ static int plane_groups(const FG& g, int nout)
     return n <= 384 ? 3 : n < 1024 ? (nout == 6 ? 2 : 3) : 1;
 }
 
+// Whether the state's passes are those of forced FP32 states (th_forced_f32.hip).  A supply or level of 0 adds nothing to
+// any mode, so such a state steps like an unforced one.
+static bool forced_passes(const th_state* s) { return s->forced && s->esz == 8 && s->fb.per_mode != 0.0; }
+static int run_forced_pass(th_state* s, int pass, int var, int stage, hipStream_t st, bool chain)
+{
+    th_plan* p = s->plan;
+    const FG& g = s->fg;
+    c32 *S = (c32*)s->S, *Vs = (c32*)s->Vs, *X1 = (c32*)s->X1, *X2 = (c32*)s->X2, *X3 = (c32*)s->X3;
+    const c32 *twx = p->twd<float>(g.N1), *twy = p->twd<float>(g.N2);
+    switch (pass) {
+    case PASS_XINV: return d_xinv<float, 0, true>(g, stage == 1 ? S : Vs, X1, 3, twx, ShellSel{0, 0}, var, st);
+    case PASS_YINV: return d_yinv<float, true>(g, X1, X2, 3, twy, var, st);
+    case PASS_Z: return d_z_forced(g, X2, X3, p->twd<float>(g.LZ), p->twd<float>(g.N3), var, st);
+    case PASS_YFWD: return d_yfwd<float, true>(g, X3, X1, 6, twy, var, st);
+    default: return d_xfwd<float, 0, true>(g, X1, X1, S, Vs, (c32*)s->acc, twx, s->dcoef + (stage - 1), var, st, chain);
+    }
+}
+
 // Pass `pass` of RK stage `stage` (1..4) for every box of s, launch-shape variant var.  Stage 1
 // reads the state, later stages the stage field; pass 5 writes the stage field / accumulator
 // (and the state in stage 4).
 template <typename R> static int run_pass(th_state* s, int pass, int var, int stage, hipStream_t st, bool chain = false)
 {
+    if (forced_passes(s)) return run_forced_pass(s, pass, var, stage, st, chain);
     th_plan* p = s->plan;
     const FG& g = s->fg;
     const cplx<R>* twx = p->twd<R>(g.N1);
@@ -775,6 +794,7 @@ static int ensure_twiddles(th_plan* p, const FG& g, hipStream_t st)
 // chained x-forward for N1
 static bool step_chained(const th_state* s)
 {
+    if (forced_passes(s)) return d_xfwd_chainable<float, true>(s->fg);
     if (s->split) return true;
     return s->physics != TH_RB && (s->plan->prec ? d_xfwd_chainable<float>(s->fg) : d_xfwd_chainable<double>(s->fg));
 }
@@ -1106,7 +1126,7 @@ template <typename R> static int profile_impl(th_state* s, double dt, double nu,
         b[PASS_XFWD] = e * (nout * cA + (state_rw - (stage < 4 && s->physics != TH_RB ? 1 : 0)) * nst * cS + extra + nin * cA);
         b[PASS_XINV] = 0;
     }
-    if (s->plane) {
+    if (s->plane && !forced_passes(s)) {
         b[PASS_Z] = e * (nin * cA + nout * cA);
         b[PASS_YINV] = b[PASS_YFWD] = 0;
     }
@@ -1152,7 +1172,8 @@ template <typename R> static int tune_impl(th_state* s, int nrep, hipStream_t st
     constexpr int ROUNDS = 3;
     for (int k = 0; k < NPASS && !r; k++) {
         // passes without launch shapes to choose from (the plane pass is one shape, the split x-forward too)
-        if ((s->plane && (k == PASS_YINV || k == PASS_Z || k == PASS_YFWD)) || (s->split && k == PASS_XFWD)) continue;
+        if (!forced_passes(s) && ((s->plane && (k == PASS_YINV || k == PASS_Z || k == PASS_YFWD)) || (s->split && k == PASS_XFWD)))
+            continue;
         const bool ch = chained && k == PASS_XFWD;
         double tv[8];
         for (int v = 0; v < 8; v++) tv[v] = 1e300;

@@ -96,21 +96,23 @@ __device__ __forceinline__ double ksq_f(double a, double b, double c)
 enum { PASS_XINV = 0, PASS_YINV = 1, PASS_Z = 2, PASS_YFWD = 3, PASS_XFWD = 4, NPASS = 5 };
 constexpr int pass_nvar(int pass) { return pass == PASS_Z ? 4 : pass == PASS_XFWD ? 3 : 4; }
 
-template <typename R, int MODE>
+// FORCED: the kernels of forced FP32 states (LineFFT; NS, float only, th_forced_f32.hip)
+template <typename R, int MODE, bool FORCED = false>
 int d_xinv(const FG& g, const cplx<R>* S, cplx<R>* A, int nc, const cplx<R>* tw, ShellSel sel, int var, hipStream_t st);
-template <typename R>
+template <typename R, bool FORCED = false>
 int d_yinv(const FG& g, const cplx<R>* A, cplx<R>* B, int nc, const cplx<R>* tw, int var, hipStream_t st);
 template <typename R, int MODE>
 int d_z(const FG& g, const cplx<R>* B, cplx<R>* Cc, const cplx<R>* twL, const cplx<R>* twN, int var, hipStream_t st);
-template <typename R>
+int d_z_forced(const FG& g, const c32* B, c32* Cc, const c32* twL, const c32* twN, int var, hipStream_t st);
+template <typename R, bool FORCED = false>
 int d_yfwd(const FG& g, const cplx<R>* Cc, cplx<R>* D, int nc, const cplx<R>* tw, int var, hipStream_t st);
-template <typename R, int MODE>
+template <typename R, int MODE, bool FORCED = false>
 int d_xfwd(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw,
            const StageCoef* sc, int var, hipStream_t st, bool chain = false);
 // chain: the x-forward also transforms its stage output back along x and writes the next stage's A lines to
 // Aout's first components (Aout may be D) (NS: U in 0-2; MHD: Z+ in 0-2, Z- in 3-5; the stage field is not written);
 // d_xfwd_chainable says whether N1 has that kernel
-template <typename R>
+template <typename R, bool FORCED = false>
 bool d_xfwd_chainable(const FG& g);
 template <typename R>
 int d_xfwd_et(const FG& g, const cplx<R>* D, const cplx<R>* U, const cplx<R>* tw, const double* radii, int nr, int kin,

@@ -35,11 +35,11 @@ template <typename R, int N> __device__ __forceinline__ void stage_tw(cplx<R>* d
     for (int i = threadIdx.x; i < N; i += blockDim.x) dst[i] = src[i];
 }
 
-template <typename R, int L, int P, int T, int MODE>
+template <typename R, int L, int P, int T, int MODE, bool FORCED>
 __global__ __launch_bounds__(T * P) void k_fx_inv(FG g, const cplx<R>* __restrict__ S, cplx<R>* __restrict__ A,
                                                   const cplx<R>* __restrict__ tw, ShellSel sel)
 {
-    using F = LineFFT<R, L, P, +1>;
+    using F = LineFFT<R, L, P, +1, false, FORCED>;
     __shared__ cplx<R> lds[L * T];
     __shared__ cplx<R> twl[L];
     stage_tw<R, L>(twl, tw);
@@ -119,11 +119,11 @@ __global__ __launch_bounds__(T * P) void k_fx_inv(FG g, const cplx<R>* __restric
 }
 
 // pass 2: y-inverse, A[x][cy][cz] -> B[x][y][cz]
-template <typename R, int L, int P, int T>
+template <typename R, int L, int P, int T, bool FORCED>
 __global__ __launch_bounds__(T * P) void k_fy_inv(FG g, const cplx<R>* __restrict__ A, cplx<R>* __restrict__ B,
                                                   const cplx<R>* __restrict__ tw, int ncomp)
 {
-    using F = LineFFT<R, L, P, +1>;
+    using F = LineFFT<R, L, P, +1, false, FORCED>;
     __shared__ cplx<R> lds[L * T];
     __shared__ cplx<R> twl[L];
     stage_tw<R, L>(twl, tw);
@@ -383,11 +383,11 @@ __global__ __launch_bounds__(TZ * P) void k_fz(FG g, const cplx<R>* __restrict__
 }
 
 // pass 4: y-forward, C[x][y][cz] -> D[x][cy][cz] (kept ky only)
-template <typename R, int L, int P, int T>
+template <typename R, int L, int P, int T, bool FORCED>
 __global__ __launch_bounds__(T * P) void k_fy_fwd(FG g, const cplx<R>* __restrict__ Cin, cplx<R>* __restrict__ D,
                                                   const cplx<R>* __restrict__ tw, int ncomp)
 {
-    using F = LineFFT<R, L, P, -1>;
+    using F = LineFFT<R, L, P, -1, false, FORCED>;
     __shared__ cplx<R> lds[L * T];
     __shared__ cplx<R> twl[L];
     stage_tw<R, L>(twl, tw);
@@ -487,12 +487,12 @@ template <int L, int P, int E, int RL> constexpr int xnext(int i)
 // by then, and no other workgroup reads these columns); the stage field itself is not written, except the stage-3 output (the
 // last stage's input) with FG::keep3.  NS: components 0-2 = U.
 // MHD: the Elsasser lines of k_fx_inv MODE 1, Z+ = U + B into components 0-2 and Z- = U - B into 3-5.
-template <typename R, int L, int P, int T, int MODE, bool CHAIN = false>
+template <typename R, int L, int P, int T, int MODE, bool CHAIN = false, bool FORCED = false>
 __global__ __launch_bounds__(T * P) __attribute__((amdgpu_waves_per_eu((MODE == 0 && sizeof(R) == 4 && L % 3 != 0) ? 4 : 1))) void k_fx_fwd(FG g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs,
                                                   cplx<R>* acc, const cplx<R>* __restrict__ tw,
                                                   const StageCoef* __restrict__ coefs)
 {
-    using F = LineFFT<R, L, P, -1>;
+    using F = LineFFT<R, L, P, -1, false, FORCED>;
     constexpr int E = F::E;
     constexpr int NP = (MODE == 0) ? 6 : 9;
     constexpr int NA = (MODE == 0) ? 3 : 6;
@@ -565,7 +565,7 @@ __global__ __launch_bounds__(T * P) __attribute__((amdgpu_waves_per_eu((MODE == 
     // The next product's loads are issued before this one's transform where that costs no wave per SIMD (XPRE): FP32
     // MHD and FP64 NS with 8 points per thread, chained FP32 NS on the long 3 2^a lines.  us, before / after: 256^3 FP32
     // MHD 227 / 210, 384^3 FP32 NS 470 / 443, 128^3 FP64 NS 30.2 / 27.8; RB (k_sx_fwd_rb) 256^3 FP32 207 / 165.
-    constexpr bool XPRE = sizeof(R) == 4 ? (MODE == 1 && E == 8) || (CHAIN && L % 3 == 0 && L >= 192) : MODE == 0 && E == 8;
+    constexpr bool XPRE = sizeof(R) == 4 ? (MODE == 1 && E == 8) || (CHAIN && !FORCED && L % 3 == 0 && L >= 192) : MODE == 0 && E == 8;
     cplx<R> nv[XPRE ? E : 1];
     if constexpr (XPRE) load(0, nv);
 #pragma unroll 1
@@ -728,7 +728,7 @@ __global__ __launch_bounds__(T * P) __attribute__((amdgpu_waves_per_eu((MODE == 
     if constexpr (CHAIN) {
         // the next stage's x-inverse (k_fx_inv MODE 0 / 1): register i holds row F::out_pos(t, i), which is
         // FI::in_pos(t, i) since the schedule's first and last radix agree
-        using FI = LineFFT<R, L, P, +1>;
+        using FI = LineFFT<R, L, P, +1, false, FORCED>;
 #pragma unroll
         for (int a = 0; a < NA; a++) {   // unrolled: Nacc[a] must stay a compile-time register
             FI::template run<T, false, NoPad, true>(Nacc[a], lds + c, t, twl + opaque_zero());
@@ -1139,22 +1139,22 @@ template <int L, int V> constexpr int var_E()
 }
 template <typename R, int L, int V> constexpr int var_T() { return ((V & 1) && L >= 128) ? tileT<R>() / 2 : tileT<R>(); }
 
-template <typename R, int L, int MODE, int V>
+template <typename R, int L, int MODE, int V, bool FORCED>
 static int launch_xinv(const FG& g, const cplx<R>* S, cplx<R>* A, int ncomp, const cplx<R>* tw, ShellSel sel, hipStream_t st)
 {
     constexpr int E = var_E<L, V>(), P = L / E, T = var_T<R, L, V>();
     const int ntz = (g.nkz + T - 1) / T;
     // MHD: one workgroup per component pair (U_c, B_c) writes both Elsasser components
     const int ny = (MODE == 1) ? ncomp / 2 : ncomp;
-    hipLaunchKernelGGL((k_fx_inv<R, L, P, T, MODE>), dim3(g.my.nk * ntz, ny, g.nbox), dim3(T * P), 0, st, g, S, A, tw, sel);
+    hipLaunchKernelGGL((k_fx_inv<R, L, P, T, MODE, FORCED>), dim3(g.my.nk * ntz, ny, g.nbox), dim3(T * P), 0, st, g, S, A, tw, sel);
     TH_CHECK_HIP(hipGetLastError());
     return OK;
 }
-template <typename R, int L, int V>
+template <typename R, int L, int V, bool FORCED>
 static int launch_yinv(const FG& g, const cplx<R>* A, cplx<R>* B, int ncomp, const cplx<R>* tw, hipStream_t st)
 {
     constexpr int E = var_E<L, V>(), P = L / E, T = var_T<R, L, V>();
-    hipLaunchKernelGGL((k_fy_inv<R, L, P, T>), dim3((g.nkz + T - 1) / T, g.N1, ncomp * g.nbox), dim3(T * P), 0, st, g, A, B,
+    hipLaunchKernelGGL((k_fy_inv<R, L, P, T, FORCED>), dim3((g.nkz + T - 1) / T, g.N1, ncomp * g.nbox), dim3(T * P), 0, st, g, A, B,
                        tw, ncomp);
     TH_CHECK_HIP(hipGetLastError());
     return OK;
@@ -1175,11 +1175,11 @@ static int launch_z(const FG& g, const cplx<R>* B, cplx<R>* Cc, const cplx<R>* t
     TH_CHECK_HIP(hipGetLastError());
     return OK;
 }
-template <typename R, int L, int V>
+template <typename R, int L, int V, bool FORCED>
 static int launch_yfwd(const FG& g, const cplx<R>* Cc, cplx<R>* D, int ncomp, const cplx<R>* tw, hipStream_t st)
 {
     constexpr int E = var_E<L, V>(), P = L / E, T = var_T<R, L, V>();
-    hipLaunchKernelGGL((k_fy_fwd<R, L, P, T>), dim3((g.nkz + T - 1) / T, g.N1, ncomp * g.nbox), dim3(T * P), 0, st, g, Cc, D,
+    hipLaunchKernelGGL((k_fy_fwd<R, L, P, T, FORCED>), dim3((g.nkz + T - 1) / T, g.N1, ncomp * g.nbox), dim3(T * P), 0, st, g, Cc, D,
                        tw, ncomp);
     TH_CHECK_HIP(hipGetLastError());
     return OK;
@@ -1194,7 +1194,14 @@ template <typename R, int L, int MODE> constexpr int xfwd_T()
     return (t * P > 512) ? (512 / P < 1 ? 1 : 512 / P) : t;
 }
 
-template <typename R, int L, int MODE, int V, bool CHAIN = false>
+// whether the chained x-forward exists for this line length (NS or MHD, first radix = last radix)
+template <typename R, int L, int MODE, bool FORCED> constexpr bool xfwd_chainable()
+{
+    using F = LineFFT<R, L, L / xfwd_E(L), -1, false, FORCED>;
+    return MODE <= 1 && F::R0 == F::RL;
+}
+
+template <typename R, int L, int MODE, int V, bool CHAIN, bool FORCED>
 static int launch_xfwd(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc,
                        const cplx<R>* tw, const StageCoef* sc, hipStream_t st)
 {
@@ -1208,15 +1215,15 @@ static int launch_xfwd(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S,
         return E_UNSUPPORTED;
     }
     if constexpr (CHAIN) {
-        if constexpr (MODE <= 1 && LineFFT<R, L, P, -1>::R0 == LineFFT<R, L, P, -1>::RL) {
-            hipLaunchKernelGGL((k_fx_fwd<R, L, P, T, MODE, true>), dim3(g.my.nk * ntz, g.nbox), dim3(T * P), 0, st, g, D,
+        if constexpr (xfwd_chainable<R, L, MODE, FORCED>()) {
+            hipLaunchKernelGGL((k_fx_fwd<R, L, P, T, MODE, true, FORCED>), dim3(g.my.nk * ntz, g.nbox), dim3(T * P), 0, st, g, D,
                                Aout, S, Vs, acc, tw, sc);
         } else {
             set_error("chained x-forward: no chained kernel for N1 = %d", L);
             return E_UNSUPPORTED;
         }
     } else {
-        hipLaunchKernelGGL((k_fx_fwd<R, L, P, T, MODE>), dim3(g.my.nk * ntz, g.nbox), dim3(T * P), 0, st, g, D, Aout, S, Vs,
+        hipLaunchKernelGGL((k_fx_fwd<R, L, P, T, MODE, false, FORCED>), dim3(g.my.nk * ntz, g.nbox), dim3(T * P), 0, st, g, D, Aout, S, Vs,
                            acc, tw, sc);
     }
     TH_CHECK_HIP(hipGetLastError());
@@ -1264,25 +1271,25 @@ static int launch_sxfwd(const FG& g, const cplx<R>* D, cplx<R>* S, cplx<R>* Vs, 
 }
 
 // variant dispatch per line length (short lines have one shape)
-template <typename R, int MODE, int L>
+template <typename R, int MODE, int L, bool FORCED>
 static int xinv_v(const FG& g, const cplx<R>* S, cplx<R>* A, int nc, const cplx<R>* tw, ShellSel sel, int var, hipStream_t st)
 {
     if constexpr (L >= 128) {
-        if (var == 1) return launch_xinv<R, L, MODE, 1>(g, S, A, nc, tw, sel, st);
-        if (var == 2) return launch_xinv<R, L, MODE, 2>(g, S, A, nc, tw, sel, st);
-        if (var == 3) return launch_xinv<R, L, MODE, 3>(g, S, A, nc, tw, sel, st);
+        if (var == 1) return launch_xinv<R, L, MODE, 1, FORCED>(g, S, A, nc, tw, sel, st);
+        if (var == 2) return launch_xinv<R, L, MODE, 2, FORCED>(g, S, A, nc, tw, sel, st);
+        if (var == 3) return launch_xinv<R, L, MODE, 3, FORCED>(g, S, A, nc, tw, sel, st);
     }
-    return launch_xinv<R, L, MODE, 0>(g, S, A, nc, tw, sel, st);
+    return launch_xinv<R, L, MODE, 0, FORCED>(g, S, A, nc, tw, sel, st);
 }
-template <typename R, int L>
+template <typename R, int L, bool FORCED>
 static int yinv_v(const FG& g, const cplx<R>* A, cplx<R>* B, int nc, const cplx<R>* tw, int var, hipStream_t st)
 {
     if constexpr (L >= 128) {
-        if (var == 1) return launch_yinv<R, L, 1>(g, A, B, nc, tw, st);
-        if (var == 2) return launch_yinv<R, L, 2>(g, A, B, nc, tw, st);
-        if (var == 3) return launch_yinv<R, L, 3>(g, A, B, nc, tw, st);
+        if (var == 1) return launch_yinv<R, L, 1, FORCED>(g, A, B, nc, tw, st);
+        if (var == 2) return launch_yinv<R, L, 2, FORCED>(g, A, B, nc, tw, st);
+        if (var == 3) return launch_yinv<R, L, 3, FORCED>(g, A, B, nc, tw, st);
     }
-    return launch_yinv<R, L, 0>(g, A, B, nc, tw, st);
+    return launch_yinv<R, L, 0, FORCED>(g, A, B, nc, tw, st);
 }
 template <typename R, int MODE, int LZ>
 static int z_v(const FG& g, const cplx<R>* B, cplx<R>* Cc, const cplx<R>* twL, const cplx<R>* twN, int var, hipStream_t st)
@@ -1298,52 +1305,46 @@ static int z_v(const FG& g, const cplx<R>* B, cplx<R>* Cc, const cplx<R>* twL, c
     }
     return launch_z<R, LZ, MODE, 0>(g, B, Cc, twL, twN, st);
 }
-template <typename R, int L>
+template <typename R, int L, bool FORCED>
 static int yfwd_v(const FG& g, const cplx<R>* Cc, cplx<R>* D, int nc, const cplx<R>* tw, int var, hipStream_t st)
 {
     if constexpr (L >= 128) {
-        if (var == 1) return launch_yfwd<R, L, 1>(g, Cc, D, nc, tw, st);
-        if (var == 2) return launch_yfwd<R, L, 2>(g, Cc, D, nc, tw, st);
-        if (var == 3) return launch_yfwd<R, L, 3>(g, Cc, D, nc, tw, st);
+        if (var == 1) return launch_yfwd<R, L, 1, FORCED>(g, Cc, D, nc, tw, st);
+        if (var == 2) return launch_yfwd<R, L, 2, FORCED>(g, Cc, D, nc, tw, st);
+        if (var == 3) return launch_yfwd<R, L, 3, FORCED>(g, Cc, D, nc, tw, st);
     }
-    return launch_yfwd<R, L, 0>(g, Cc, D, nc, tw, st);
+    return launch_yfwd<R, L, 0, FORCED>(g, Cc, D, nc, tw, st);
 }
-template <typename R, int MODE, int L>
+template <typename R, int MODE, int L, bool FORCED>
 static int xfwd_v(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw, const StageCoef* sc,
                   int var, hipStream_t st, bool chain)
 {
     if (chain) {
         if constexpr (L >= 128)
-            if (var == 1) return launch_xfwd<R, L, MODE, 1, true>(g, D, Aout, S, Vs, acc, tw, sc, st);
+            if (var == 1) return launch_xfwd<R, L, MODE, 1, true, FORCED>(g, D, Aout, S, Vs, acc, tw, sc, st);
         if constexpr (L >= 128 && sizeof(R) == 4 && MODE == 0 && L % 3 != 0 && 2 * xfwd_T<R, L, MODE>() * (L / xfwd_E(L)) <= 1024)
-            if (var == 2) return launch_xfwd<R, L, MODE, 2, true>(g, D, Aout, S, Vs, acc, tw, sc, st);
-        return launch_xfwd<R, L, MODE, 0, true>(g, D, Aout, S, Vs, acc, tw, sc, st);
+            if (var == 2) return launch_xfwd<R, L, MODE, 2, true, FORCED>(g, D, Aout, S, Vs, acc, tw, sc, st);
+        return launch_xfwd<R, L, MODE, 0, true, FORCED>(g, D, Aout, S, Vs, acc, tw, sc, st);
     }
     if constexpr (L >= 128)
-        if (var == 1) return launch_xfwd<R, L, MODE, 1>(g, D, Aout, S, Vs, acc, tw, sc, st);
+        if (var == 1) return launch_xfwd<R, L, MODE, 1, false, FORCED>(g, D, Aout, S, Vs, acc, tw, sc, st);
     // 1024-thread workgroups hold a wave to 128 VGPRs: only the FP32 NS kernels fit (124)
     if constexpr (L >= 128 && sizeof(R) == 4 && MODE == 0 && L % 3 != 0 && 2 * xfwd_T<R, L, MODE>() * (L / xfwd_E(L)) <= 1024)
-        if (var == 2) return launch_xfwd<R, L, MODE, 2>(g, D, Aout, S, Vs, acc, tw, sc, st);
-    return launch_xfwd<R, L, MODE, 0>(g, D, Aout, S, Vs, acc, tw, sc, st);
-}
-// whether the chained x-forward exists for this line length and variant (NS or MHD, first radix = last radix)
-template <typename R, int L, int MODE, int V> constexpr bool xfwd_chainable()
-{
-    constexpr int E = xfwd_E(L), P = L / E;
-    return MODE <= 1 && LineFFT<R, L, P, -1>::R0 == LineFFT<R, L, P, -1>::RL;
+        if (var == 2) return launch_xfwd<R, L, MODE, 2, false, FORCED>(g, D, Aout, S, Vs, acc, tw, sc, st);
+    return launch_xfwd<R, L, MODE, 0, false, FORCED>(g, D, Aout, S, Vs, acc, tw, sc, st);
 }
 
-template <typename R, int MODE>
+template <typename R, int MODE, bool FORCED>
 int d_xinv(const FG& g, const cplx<R>* S, cplx<R>* A, int nc, const cplx<R>* tw, ShellSel sel, int var, hipStream_t st)
 {
-#define C_(n) case n: return xinv_v<R, MODE, n>(g, S, A, nc, tw, sel, var, st);
+#define C_(n) case n: return xinv_v<R, MODE, n, FORCED>(g, S, A, nc, tw, sel, var, st);
     switch (g.N1) { TH_FLENS(C_) default: set_error("fused: N1 %d unsupported", g.N1); return E_UNSUPPORTED; }
 #undef C_
 }
-template <typename R>
+template <typename R, bool FORCED>
 int d_yinv(const FG& g, const cplx<R>* A, cplx<R>* B, int nc, const cplx<R>* tw, int var, hipStream_t st)
 {
-#define C_(n) case n: return yinv_v<R, n>(g, A, B, nc, tw, var, st);
+#define C_(n) case n: return yinv_v<R, n, FORCED>(g, A, B, nc, tw, var, st);
     switch (g.N2) { TH_FLENS(C_) default: set_error("fused: N2 %d unsupported", g.N2); return E_UNSUPPORTED; }
 #undef C_
 }
@@ -1354,26 +1355,26 @@ int d_z(const FG& g, const cplx<R>* B, cplx<R>* Cc, const cplx<R>* twL, const cp
     switch (g.LZ) { TH_ZLENS(C_) default: set_error("fused: N3 %d unsupported", g.N3); return E_UNSUPPORTED; }
 #undef C_
 }
-template <typename R>
+template <typename R, bool FORCED>
 int d_yfwd(const FG& g, const cplx<R>* Cc, cplx<R>* D, int nc, const cplx<R>* tw, int var, hipStream_t st)
 {
-#define C_(n) case n: return yfwd_v<R, n>(g, Cc, D, nc, tw, var, st);
+#define C_(n) case n: return yfwd_v<R, n, FORCED>(g, Cc, D, nc, tw, var, st);
     switch (g.N2) { TH_FLENS(C_) default: set_error("fused: N2 %d unsupported", g.N2); return E_UNSUPPORTED; }
 #undef C_
 }
-template <typename R, int MODE>
+template <typename R, int MODE, bool FORCED>
 int d_xfwd(const FG& g, const cplx<R>* D, cplx<R>* Aout, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw,
            const StageCoef* sc, int var, hipStream_t st, bool chain)
 {
-#define C_(n) case n: return xfwd_v<R, MODE, n>(g, D, Aout, S, Vs, acc, tw, sc, var, st, chain);
+#define C_(n) case n: return xfwd_v<R, MODE, n, FORCED>(g, D, Aout, S, Vs, acc, tw, sc, var, st, chain);
     switch (g.N1) { TH_FLENS(C_) default: set_error("fused: N1 %d unsupported", g.N1); return E_UNSUPPORTED; }
 #undef C_
 }
-template <typename R>
+template <typename R, bool FORCED>
 bool d_xfwd_chainable(const FG& g)
 {
     // every variant of a line length, NS or MHD, uses the same points per thread, hence the same radix schedule
-#define C_(n) case n: return xfwd_chainable<R, n, 0, 0>();
+#define C_(n) case n: return xfwd_chainable<R, n, 0, FORCED>();
     switch (g.N1) { TH_FLENS(C_) default: return false; }
 #undef C_
 }
@@ -1427,10 +1428,10 @@ template <typename R> int d_scatter(const FG& g, const cplx<R>* S, cplx<R>* ref,
 }
 
 #define TH_FUSED_INSTANTIATE(R)                                                                                       \
-    template int d_xinv<R, 0>(const FG&, const cplx<R>*, cplx<R>*, int, const cplx<R>*, ShellSel, int, hipStream_t);  \
-    template int d_xinv<R, 1>(const FG&, const cplx<R>*, cplx<R>*, int, const cplx<R>*, ShellSel, int, hipStream_t);  \
-    template int d_xinv<R, 2>(const FG&, const cplx<R>*, cplx<R>*, int, const cplx<R>*, ShellSel, int, hipStream_t);  \
-    template int d_yinv<R>(const FG&, const cplx<R>*, cplx<R>*, int, const cplx<R>*, int, hipStream_t);              \
+    template int d_xinv<R, 0, false>(const FG&, const cplx<R>*, cplx<R>*, int, const cplx<R>*, ShellSel, int, hipStream_t);  \
+    template int d_xinv<R, 1, false>(const FG&, const cplx<R>*, cplx<R>*, int, const cplx<R>*, ShellSel, int, hipStream_t);  \
+    template int d_xinv<R, 2, false>(const FG&, const cplx<R>*, cplx<R>*, int, const cplx<R>*, ShellSel, int, hipStream_t);  \
+    template int d_yinv<R, false>(const FG&, const cplx<R>*, cplx<R>*, int, const cplx<R>*, int, hipStream_t);              \
     template int d_z<R, 0>(const FG&, const cplx<R>*, cplx<R>*, const cplx<R>*, const cplx<R>*, int, hipStream_t);   \
     template int d_z<R, 1>(const FG&, const cplx<R>*, cplx<R>*, const cplx<R>*, const cplx<R>*, int, hipStream_t);   \
     template int d_z<R, 2>(const FG&, const cplx<R>*, cplx<R>*, const cplx<R>*, const cplx<R>*, int, hipStream_t);   \
@@ -1438,12 +1439,12 @@ template <typename R> int d_scatter(const FG& g, const cplx<R>* S, cplx<R>* ref,
     template int d_sx_inv<R>(const FG&, const cplx<R>*, cplx<R>*, const cplx<R>*, const cplx<R>*, hipStream_t);      \
     template int d_sx_fwd_rb<R>(const FG&, const cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, const cplx<R>*,            \
                                 const cplx<R>*, const StageCoef*, int, hipStream_t);                                  \
-    template int d_yfwd<R>(const FG&, const cplx<R>*, cplx<R>*, int, const cplx<R>*, int, hipStream_t);              \
-    template int d_xfwd<R, 0>(const FG&, const cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, const cplx<R>*,    \
+    template int d_yfwd<R, false>(const FG&, const cplx<R>*, cplx<R>*, int, const cplx<R>*, int, hipStream_t);              \
+    template int d_xfwd<R, 0, false>(const FG&, const cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, const cplx<R>*,    \
                               const StageCoef*, int, hipStream_t, bool);                                               \
-    template int d_xfwd<R, 1>(const FG&, const cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, const cplx<R>*,    \
+    template int d_xfwd<R, 1, false>(const FG&, const cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, cplx<R>*, const cplx<R>*,    \
                               const StageCoef*, int, hipStream_t, bool);                                               \
-    template bool d_xfwd_chainable<R>(const FG&);                                                                      \
+    template bool d_xfwd_chainable<R, false>(const FG&);                                                                      \
     template int d_xfwd_et<R>(const FG&, const cplx<R>*, const cplx<R>*, const cplx<R>*, const double*, int, int,    \
                               double*, int*, hipStream_t);                                                             \
     template int d_gather<R>(const FG&, const cplx<R>*, cplx<R>*, hipStream_t);                                        \
