@@ -260,7 +260,8 @@ template <typename R> int plain_step(th_plan* p, int physics, int scheme, cplx<R
         const FieldPtrs& in = s == 0 ? v0 : fs;
         if (last && keep && keep[0])
             for (int c = 0; c < nc; c++)
-                TH_CHECK_HIP(hipMemcpyAsync(keep[c], in.v[c], nfull * sizeof(cplx<R>), hipMemcpyDeviceToDevice, st));
+                if (keep[c] != F[c])        // the field's own array ends as the step's result
+                    TH_CHECK_HIP(hipMemcpyAsync(keep[c], in.v[c], nfull * sizeof(cplx<R>), hipMemcpyDeviceToDevice, st));
         if (physics == TH_NS) TRY((px_inv<R, 0>(gf, in, X, 3, twx, tw4, st)));
         else if (physics == TH_MHD) TRY((px_inv<R, 1>(gf, in, X, 6, twx, tw4, st)));
         else TRY((px_inv<R, 2>(gf, in, X, 4, twx, tw4, st)));
