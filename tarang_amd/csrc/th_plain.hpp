@@ -134,6 +134,9 @@ __global__ __launch_bounds__(256) void k_plain_stage(FG g, FastDiv dH, FastDiv d
         const double kx = (g.scft ? l1 : kx_four(l1, g.N1)) * g.f1, ky = ky_of(l2, g.N2) * g.f2, kz = l3 * g.f3;
         const double k2 = ksq_f(kx, ky, kz);
         const double h0 = exp(-d0 * 0.5 * dt * k2), h1 = NC > 3 ? exp(-d1 * 0.5 * dt * k2) : 0.0;
+        // the whole step's factors by themselves (not as squares: one rounding, as k_exp_ksqr's)
+        const bool whole = kind == 0 || kind == 1 || kind == 4;
+        const double w0 = whole ? exp(-d0 * dt * k2) : 0.0, w1 = NC > 3 && whole ? exp(-d1 * dt * k2) : 0.0;
         Dc q[NC];
 #pragma unroll
         for (int c = 0; c < NC; c++) q[c] = dl(r[c]);
@@ -147,7 +150,7 @@ __global__ __launch_bounds__(256) void k_plain_stage(FG g, FastDiv dH, FastDiv d
         }
 #pragma unroll
         for (int c = 0; c < NC; c++) {
-            const double eh = c < 3 ? h0 : h1, e1 = eh * eh;
+            const double eh = c < 3 ? h0 : h1, e1 = c < 3 ? w0 : w1;
             const Dc V = dl(s[c]);
             Dc o;
             if (kind == 0) o = sc(add(V, sc(q[c], dt)), e1);

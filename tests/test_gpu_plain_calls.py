@@ -38,3 +38,24 @@ def test_last_stage_may_be_the_fields_themselves(ctx, physics, scheme):
                                     last_stage=last)
     for x, y in zip(a, b):
         assert np.array_equal(x.cpu().numpy(), y.cpu().numpy())
+
+
+@pytest.mark.parametrize("scheme", (0, 1, 2))
+def test_pure_decay_has_the_factor_of_exp_ksqr(ctx, scheme):
+    """A shear flow (0, f(x), 0) has no nonlinear term, exactly (V_x = 0 and Ky = Kz = 0 on its modes): an EULER or RK4
+    step multiplies each mode by exp(-nu K^2 dt), evaluated and rounded once, as exp_ksqr does; RK2 by the half step's
+    factor twice."""
+    import torch
+    from tarang_amd import Plan, abi
+    print(scheme, flush=True)
+    nu, dt = 3e-3, 0.37
+    p = Plan(ctx, (96, 16, 16), kfactor=(0.7, 1.0, 1.0))
+    V = [torch.zeros(p.shape, dtype=p.dtype, device="cuda") for _ in range(3)]
+    for k in range(1, 32):
+        V[1][k, 0, 0] = complex(0.3 / k, 0.1)
+        V[1][-k, 0, 0] = complex(0.3 / k, -0.1)
+    ref = p.exp_ksqr(V[1].clone(), -nu * dt * (0.5 if scheme == 1 else 1.0))
+    if scheme == 1:
+        ref = p.exp_ksqr(ref, -nu * dt * 0.5)
+    got = p.step_plain(abi.TH_NS, V, dt, nu=nu, scheme=scheme)[1]
+    assert np.array_equal(got[:, 0, 0].cpu().numpy(), ref[:, 0, 0].cpu().numpy())
