@@ -191,7 +191,7 @@ th_plan::~th_plan()
     tw.release();
     rs.release();
     if (radii_dev) (void)hipFree(radii_dev);
-    plain.release();
+    plain_release(plain);
     release_fused(this);
 }
 
@@ -865,7 +865,7 @@ template <typename R> static int do_step_plain(th_plan* p, int physics, int sche
         for (int q = 0; q < o.nc; q++) F[q] = CP(R, fields[q]);
         const int r = plain_step<R>(p, physics, scheme, F, dt, nu, physics == TH_MHD ? eta : kap, nullptr, nullptr, nullptr);
         if (r != E_NOMEM) return r;
-        p->plain.release();      // no room for its workspace: the operation sequence
+        plain_release(p->plain);      // no room for its workspace: the operation sequence
     }
     for (int q = 0; q < o.nc; q++) {
         o.F[q] = CP(R, fields[q]);
@@ -896,7 +896,7 @@ template <typename R> static int do_step_plain_forced(th_plan* p, int scheme, vo
         cplx<R>* F[3] = {CP(R, V[0]), CP(R, V[1]), CP(R, V[2])};
         const int r = plain_step<R>(p, TH_NS, scheme, F, dt, ph->nu, 0.0, fb, nullptr, o.keep);
         if (r != E_NOMEM) return r;
-        p->plain.release();
+        plain_release(p->plain);
     }
     for (int q = 0; q < 3; q++) {
         o.F[q] = CP(R, V[q]);
@@ -924,7 +924,7 @@ template <typename R> static int do_step_plain_forced_mhd(th_plan* p, int scheme
         const bool u = fu->proc == 3 || fu->per_mode > 1e-15, w = fw->proc == 3 || fw->per_mode > 1e-15;
         const int r = plain_step<R>(p, TH_MHD, scheme, F, dt, ph->nu, ph->eta, u ? fu : nullptr, w ? fw : nullptr, o.keep);
         if (r != E_NOMEM) return r;
-        p->plain.release();
+        plain_release(p->plain);
     }
     for (int q = 0; q < 6; q++) {
         o.F[q] = CP(R, q < 3 ? U[q] : B[q - 3]);
@@ -1111,12 +1111,8 @@ extern "C" int th_shell_mult_single(th_plan* p, void* const A[3], void* const B[
 
 static int upload_radii(th_plan* p, const double* radii, int nr)
 {
-    if (nr > p->radii_cap) {
-        if (p->radii_dev) (void)hipFree(p->radii_dev);
-        p->radii_dev = nullptr;
-        TH_CHECK_HIP(hipMalloc(&p->radii_dev, nr * sizeof(double)));
-        p->radii_cap = nr;
-    }
+    TRY(regrow(p->radii_dev, p->radii_cap, (size_t)nr,
+               [](double** q, size_t n) { return dev_alloc((void**)q, n * sizeof(double), "shell radii"); }, dev_free));
     TH_CHECK_HIP(hipMemcpyAsync(p->radii_dev, radii, nr * sizeof(double), hipMemcpyHostToDevice, p->ctx->stream));
     TH_CHECK_HIP(hipStreamSynchronize(p->ctx->stream));
     return OK;

@@ -73,60 +73,54 @@ FG make_fg(const Geo& geo, int prec)
 
 using namespace th;
 
-// The plain steps' workspace.  Cleared and filled by kernels: a call on a stream under capture must record no memset node
-// and no copy from the host's stack.
+// The plain steps' workspace.  Its clears and the coefficients go through kernels on the context's stream, in order with
+// the step's launches (a memset or a copy would run on the null stream, which the context's stream does not wait for).
 __global__ void k_clear(double* p, size_t n)
 {
     for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) p[i] = 0.0;
 }
 __global__ void k_put_coef(StageCoef c, StageCoef* p) { *p = c; }
 
-int PlainBufs::ensure(size_t esz, size_t nX, size_t nY, size_t nC, size_t nF, hipStream_t st)
-{
-    auto grow = [&](void** q, size_t bytes, bool clear) -> int {
-        if (*q) TH_CHECK_HIP(hipFree(*q));       // (waits for the launches that still read it)
-        *q = nullptr;
-        if (hipMalloc(q, bytes) != hipSuccess) {
-            *q = nullptr;
-            (void)hipGetLastError();
-            set_error("plain step: workspace allocation of %zu bytes failed", bytes);
-            return E_NOMEM;
-        }
-        if (clear) {
-            hipLaunchKernelGGL(k_clear, dim3(2048), dim3(256), 0, st, (double*)*q, bytes / sizeof(double));
-            TH_CHECK_HIP(hipGetLastError());
-        }
-        return OK;
-    };
-    if (nX * esz > bX) { bX = 0; TRY(grow(&X, nX * esz, true)); bX = nX * esz; }
-    if (nY * esz > bY) { bY = 0; TRY(grow(&Y, nY * esz, true)); bY = nY * esz; }
-    if (nC * esz > bC) {
-        bC = 0;
-        TRY(grow(&rhs, nC * esz, true));
-        TRY(grow(&acc, nC * esz, true));
-        TRY(grow(&zero, nC * esz, true));
-        TRY(grow(&junk, nC * esz, true));
-        bC = nC * esz;
+namespace {
+struct DevMem {
+    hipStream_t st;
+    int alloc(void** p, size_t bytes, bool clear)
+    {
+        if (dev_alloc(p, bytes, "plain step: workspace")) return E_NOMEM;
+        if (!clear) return OK;
+        hipLaunchKernelGGL(k_clear, dim3(2048), dim3(256), 0, st, (double*)*p, bytes / sizeof(double));
+        if (hipGetLastError() == hipSuccess) return OK;
+        set_error("plain step: clearing the workspace failed");
+        (void)hipFree(*p);
+        return E_HIP;
     }
-    if (nF * esz > bF) { bF = 0; TRY(grow(&Fs, nF * esz, false)); bF = nF * esz; }
-    if (!coef) {
+    void release(void* p) { (void)hipFree(p); }      // waits for the launches that still read it
+};
+}  // namespace
+
+int th::plain_ensure(PlainBufs& w, size_t esz, size_t nX, size_t nY, size_t nC, size_t nF, hipStream_t st)
+{
+    DevMem m{st};
+    bool fresh = false;
+    TRY(w.ensure(m, nX * esz, nY * esz, nC * esz, nF * esz, sizeof(StageCoef), &fresh));
+    if (fresh) {
         StageCoef c;
         memset(&c, 0, sizeof c);
         c.stage = 1;
         c.dt = 2.0;
-        TRY(grow(&coef, sizeof c, false));
-        hipLaunchKernelGGL(k_put_coef, dim3(1), dim3(1), 0, st, c, (StageCoef*)coef);
-        TH_CHECK_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_put_coef, dim3(1), dim3(1), 0, st, c, (StageCoef*)w.coef);
+        if (hipGetLastError() != hipSuccess) {
+            set_error("plain step: filling the workspace failed");
+            w.release(m);
+            return E_HIP;
+        }
     }
     return OK;
 }
-void PlainBufs::release()
+void th::plain_release(PlainBufs& w)
 {
-    for (void** q : {&X, &Y, &rhs, &acc, &zero, &junk, &Fs, &coef}) {
-        if (*q) (void)hipFree(*q);
-        *q = nullptr;
-    }
-    bX = bY = bC = bF = 0;
+    DevMem m{nullptr};
+    w.release(m);
 }
 
 struct th_state {
@@ -146,7 +140,7 @@ struct th_state {
     double* partial = nullptr;
     size_t partial_cap = 0;
     double* radii = nullptr;
-    int radii_cap = 0;
+    size_t radii_cap = 0;
     StageCoef* dcoef = nullptr;  // device [4 stages][nbox]; the captured step reads it
     StageCoef* hcoef = nullptr;  // pinned staging for dcoef
     std::vector<StageCoef> cur;  // what dcoef holds once the last upload has run
@@ -864,12 +858,8 @@ static int et_shell_rows(th_state* s, const double* radii, int nsh, int ngiv, in
     cplx<R>* X2 = (cplx<R>*)s->X2;
     cplx<R>* X3 = (cplx<R>*)s->X3;
     const int nr = nsh + 1;
-    if (s->radii_cap < nr) {
-        if (s->radii) (void)hipFree(s->radii);
-        s->radii = nullptr;
-        TH_CHECK_HIP(hipMalloc(&s->radii, nr * sizeof(double)));
-        s->radii_cap = nr;
-    }
+    auto doubles = [](double** q, size_t n) { return dev_alloc((void**)q, n * sizeof(double), "energy transfer"); };
+    TRY(regrow(s->radii, s->radii_cap, (size_t)nr, doubles, dev_free));
     TH_CHECK_HIP(hipMemcpyAsync(s->radii, radii, nr * sizeof(double), hipMemcpyHostToDevice, st));
     int nblk = 0;
     TRY(d_xfwd_et<R>(g, X1, S, twx, s->radii, nr, 0, nullptr, &nblk, st));
@@ -882,27 +872,17 @@ static int et_shell_rows(th_state* s, const double* radii, int nsh, int ngiv, in
     const size_t per = (plane ? 3 * g.cA + 9 * g.cA : 3 * g.cA + 3 * g.cB + 9 * g.cB + 9 * g.cA) * sizeof(cplx<R>);
     const size_t shared = (plane ? 3 * g.cA : 3 * g.cB) * sizeof(cplx<R>);
     int G = (int)std::min<size_t>(std::min<size_t>(std::max<size_t>((128u << 20) / per, 1), 64), ngiv);
-    if (G > 1 && shared + G * per > s->et_cap) {
-        if (s->et) TH_CHECK_HIP(hipFree(s->et));
-        s->et = nullptr;
-        s->et_cap = 0;
-        if (hipMalloc(&s->et, shared + G * per) == hipSuccess) {
-            s->et_cap = shared + G * per;
-            TH_CHECK_HIP(hipMemsetAsync(s->et, 0, s->et_cap, st));   // row padding is read (never used)
-        } else {
-            (void)hipGetLastError();
-            s->et = nullptr;
-            G = 1;   // no room: one at a time in the state's own buffers
-        }
+    if (G > 1) {
+        auto bytes = [&](void** q, size_t n) -> int {
+            TRY(dev_alloc(q, n, "energy transfer"));
+            if (hipMemsetAsync(*q, 0, n, st) == hipSuccess) return OK;   // row padding is read (never used)
+            (void)hipFree(*q);
+            return E_HIP;
+        };
+        if (regrow(s->et, s->et_cap, shared + G * per, bytes, dev_free)) G = 1;   // no room: one at a time in the state's own buffers
     }
     size_t need = (size_t)G * nblk * (2 * nr) + (size_t)ngiv * nrecv * (2 * nr);
-    if (need > s->partial_cap) {
-        if (s->partial) (void)hipFree(s->partial);
-        s->partial = nullptr;
-        s->partial_cap = 0;
-        TH_CHECK_HIP(hipMalloc(&s->partial, need * sizeof(double)));
-        s->partial_cap = need;
-    }
+    TRY(regrow(s->partial, s->partial_cap, need, doubles, dev_free));
     for (int r = 0; r < nrecv; r++) {
         Yb[r].assign((size_t)(ngiv + 1) * nr, 0.0);
         Yc[r].assign((size_t)(ngiv + 1) * nr, 0.0);

@@ -49,6 +49,18 @@ void set_error(const char* fmt, ...);
         }                                                                                  \
     } while (0)
 
+// hipMalloc as regrow (th_grow.hpp) takes it: bytes -> 0 or E_HIP; the runtime's record of a failed call is taken back, so
+// that it is not reported by the next launch
+static inline int dev_alloc(void** p, size_t bytes, const char* what)
+{
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return OK;
+    (void)hipGetLastError();
+    set_error("%s: allocation of %zu bytes failed: %s", what, bytes, hipGetErrorString(e));
+    return E_HIP;
+}
+static inline void dev_free(void* p) { (void)hipFree(p); }
+
 // Geometry of one box (reference layout (N1, N2, N3/2+1) complex, C-order).
 struct Geo {
     int basis = 0;          // 0 FOUR, 1 SCFT

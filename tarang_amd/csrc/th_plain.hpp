@@ -245,9 +245,9 @@ template <typename R> int plain_step(th_plan* p, int physics, int scheme, cplx<R
     const size_t sX = (size_t)std::max(nc * gf.cA, nout * g.cB), sY = (size_t)std::max(nc * gf.cB, nout * g.cA);
     const size_t sC = (size_t)nc * g.cS, nfull = p->g.ncplx();
     PlainBufs& w = p->plain;
-    TRY(w.ensure(sizeof(cplx<R>), sX, sY, sC, nfull * nc, st));
-    cplx<R>*X = (cplx<R>*)w.X, *Y = (cplx<R>*)w.Y, *rhs = (cplx<R>*)w.rhs, *acc = (cplx<R>*)w.acc;
-    cplx<R>*zero = (cplx<R>*)w.zero, *junk = (cplx<R>*)w.junk;
+    TRY(plain_ensure(w, sizeof(cplx<R>), sX, sY, sC, nfull * nc, st));
+    cplx<R>*X = (cplx<R>*)w.X, *Y = (cplx<R>*)w.Y, *rhs = (cplx<R>*)w.rhs(), *acc = (cplx<R>*)w.acc();
+    cplx<R>*zero = (cplx<R>*)w.zero(), *junk = (cplx<R>*)w.junk();
     for (int L : {g.N1, g.N2, g.LZ, g.N3, g.scft ? 4 * g.N1 : g.N1})
         if (!p->tw.get(L, prec, st)) { set_error("twiddle table allocation failed"); return E_NOMEM; }
     const cplx<R>*twx = p->twd<R>(g.N1), *twy = p->twd<R>(g.N2), *twz = p->twd<R>(g.LZ), *twn = p->twd<R>(g.N3);

@@ -1,6 +1,7 @@
 // th_plan.hpp -- the opaque th_plan / th_state structs of the C-ABI.
 #pragma once
 #include <vector>
+#include "th_grow.hpp"
 #include "th_internal.hpp"
 
 namespace th {
@@ -24,15 +25,6 @@ enum {
     SC_FW0 = 43,     // W.Force1..3 (forced MHD) 43..45
 };
 struct Fused;        // dealias-pruned pipeline (th_fused.hip)
-
-// Workspace of the plain steppers (th_plain.hpp), kept in the plan and grown to the largest physics it has stepped
-struct PlainBufs {
-    void *X = nullptr, *Y = nullptr, *rhs = nullptr, *acc = nullptr, *zero = nullptr, *junk = nullptr, *Fs = nullptr;
-    void* coef = nullptr;
-    size_t bX = 0, bY = 0, bC = 0, bF = 0;
-    int ensure(size_t esz, size_t X, size_t Y, size_t C, size_t Fs, hipStream_t st);
-    void release();
-};
 }  // namespace th
 
 struct th_plan {
@@ -43,7 +35,7 @@ struct th_plan {
     th::RedScratch rs;
     std::vector<void*> scratch;
     double* radii_dev = nullptr;
-    int radii_cap = 0;
+    size_t radii_cap = 0;
     th::Fused* fused = nullptr;
     th::PlainBufs plain;
     int nstates = 0;                 // fused states created on this plan and not yet destroyed
@@ -55,6 +47,9 @@ struct th_plan {
 
 namespace th {
 void release_fused(th_plan* p);
+// the plain steps' workspace: sizes in elements of esz bytes
+int plain_ensure(PlainBufs& w, size_t esz, size_t X, size_t Y, size_t C, size_t Fs, hipStream_t st);
+void plain_release(PlainBufs& w);
 void plan_free(th_plan* p);           // waits for the plan's stream, frees it, uncounts it in its context
 template <typename R> int plain_forward(th_plan* p, cplx<R>* A, int parity);
 template <typename R> int plain_inverse(th_plan* p, cplx<R>* A, int parity);

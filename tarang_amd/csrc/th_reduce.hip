@@ -9,6 +9,7 @@
 // for binned sums, tree reduction for scalars); blocks are merged with Neumaier-compensated sums.
 #include <math.h>
 #include <mutex>
+#include "th_grow.hpp"
 #include "th_internal.hpp"
 
 namespace th {
@@ -606,21 +607,18 @@ __global__ __launch_bounds__(RBLK) void k_ring_mult(GeoR g, const cplx<R>* __res
 // line (energy, spectrum, helicity, ...) costs a device and a pinned allocation each.
 int RedScratch::ensure(size_t n_dev, size_t n_host)
 {
-    if (n_dev < (1u << 20)) n_dev = 1u << 20;
-    if (n_host < 4096) n_host = 4096;
-    if (n_dev > cap) {
-        if (d) (void)hipFree(d);
-        d = nullptr;
-        TH_CHECK_HIP(hipMalloc(&d, n_dev * sizeof(double)));
-        cap = n_dev;
-    }
-    if (n_host > hcap) {
-        if (h) (void)hipHostFree(h);
-        h = nullptr;
-        TH_CHECK_HIP(hipHostMalloc(&h, n_host * sizeof(double)));
-        hcap = n_host;
-    }
-    return OK;
+    auto dev = [](double** p, size_t n) { return dev_alloc((void**)p, n * sizeof(double), "reduction scratch"); };
+    auto host = [](double** p, size_t n) -> int {
+        const hipError_t e = hipHostMalloc(p, n * sizeof(double));
+        if (e == hipSuccess) return OK;
+        (void)hipGetLastError();
+        set_error("reduction scratch: %zu pinned bytes: %s", n * sizeof(double), hipGetErrorString(e));
+        return E_HIP;
+    };
+    auto host_free = [](double* p) { (void)hipHostFree(p); };
+    // where the floor finds no room, what this call needs
+    if (n_dev > cap && (n_dev >= 1u << 20 || regrow(d, cap, 1u << 20, dev, dev_free))) TRY(regrow(d, cap, n_dev, dev, dev_free));
+    return regrow(h, hcap, n_host < 4096 ? 4096 : n_host, host, host_free);
 }
 void RedScratch::release()
 {
