@@ -1102,8 +1102,9 @@ template <typename R> static int profile_impl(th_state* s, double dt, double nu,
     double b[5] = {e * (nst * cS + nin * cA), e * (nin * cA + nin * cB), e * (nin * cB + nout * cB),
                    e * (nout * cB + nout * cA), e * (nout * cA + state_rw * nst * cS + extra)};
     if (chained) {
-        // the next stage's A lines written too, and (NS, MHD) no stage field in stages 1-3
-        b[PASS_XFWD] = e * (nout * cA + (state_rw - (stage < 4 && s->physics != TH_RB ? 1 : 0)) * nst * cS + extra + nin * cA);
+        // the next stage's A lines written too, and (NS, MHD) no stage field in stages 1-3 but a kept one
+        const bool wvs = s->physics == TH_RB || (stage == 3 && g.keep3);
+        b[PASS_XFWD] = e * (nout * cA + (state_rw - (stage < 4 && !wvs ? 1 : 0)) * nst * cS + extra + nin * cA);
         b[PASS_XINV] = 0;
     }
     if (s->plane && !forced_passes(s)) {
