@@ -440,14 +440,18 @@ static int set_coefs(th_state* s, const double* dt, const double* nu, const doub
     return OK;
 }
 
-// Workgroups per x-plane of the plane pass: one per product while that is at most four small planes per CU, one per
-// rotation step up to 384 planes, and less repeated work beyond.  us per step with 1 / 2 / 3 / 6 groups (NS):
-// 32^3 FP64 139 / 116 / 104 / 99, 256 x 64 x 64 FP32 211 / 188 / 179 / 191, 512 x 48 x 48 FP32 262 / 230 / 253 / 272,
-// 512 x 64 x 64 FP64 309 / 329 / 328 / 391.
+// Workgroups per x-plane of the plane pass: one per product while that is at most four small planes per CU (NS in FP64,
+// planes of more than 2048 points: while it is not many more than one), one per rotation step up to 384 planes, and less
+// repeated work beyond.  us per step with 1 / 2 / 3 / 6 groups (NS; MHD and RB: 9 for 6):
+// 32^3 FP64 87 / 65 / 54 / 49, 64^3 FP64 146 / 107 / 89 / 88, FP32 123 / 90 / 74 / 71, 96 x 32 x 64 FP64 129 / 99 / 93 / 88,
+// 96 x 48 x 48 FP64 179 / 129 / 118 / 142, 128 x 64 x 64 FP64 172 / 134 / 130 / 136, FP32 141 / 109 / 99 / 95,
+// 64^3 MHD FP64 242 / 170 / 133 / 129, 96 x 64 x 64 MHD FP64 265 / 192 / 181 / 167, 64^3 RB FP64 219 / 162 / 125 / 124,
+// 256 x 64 x 64 FP32 211 / 188 / 179 / 191, 512 x 48 x 48 FP32 262 / 230 / 253 / 272, 512 x 64 x 64 FP64 309 / 329 / 328 / 391.
 static int plane_groups(const FG& g, int nout)
 {
     const int n = g.N1 * g.nbox, pts = g.N2 * g.N3;
-    if (n * nout <= 1024 && pts <= 4096) return nout;
+    const bool wide = g.fp64 && nout == 6 && pts > 2048;
+    if (n * nout <= (wide ? 384 : 1024) && pts <= 4096) return nout;
     return n <= 384 ? 3 : n < 1024 ? (nout == 6 ? 2 : 3) : 1;
 }
 
