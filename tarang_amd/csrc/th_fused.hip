@@ -190,7 +190,7 @@ static std::string tune_key(const th_state* s)
 // Short boxes (th_plane.hpp).
 //
 // Passes 2 to 4 as one launch, by the grid alone (a box computes the same bits alone and in an ensemble): N2 and N3 up
-// to 128 with at most 8192 points per plane (74 KB of LDS in FP64), and in FP64 planes past 4608 points only on long
+// to 128 with at most 8192 points per plane (up to 79 KB of LDS in FP64), and in FP64 planes past 4608 points only on long
 // boxes, where the three passes wait on memory rather than on launches.
 // us per step, three passes / plane pass: 32^3 FP64 160 / 98, 64^3 FP64 174 / 125, eight 64^3 FP32 306 / 187,
 // 512 x 64 x 64 FP64 465 / 309, 512 x 128 x 64 FP32 564 / 369; past the line 96^3 FP32 213 / 202 to 248,

@@ -126,7 +126,7 @@ template <typename R> int d_gather(const FG& g, const cplx<R>* ref, cplx<R>* S, 
 template <typename R> int d_scatter(const FG& g, const cplx<R>* S, cplx<R>* ref, hipStream_t st);
 
 // ---- short boxes (th_plane.hpp) ----
-// Passes 2 to 4 in one launch, A (nin lines) -> D (nout lines), for boxes with plane_ok; ngrp = 3 or nout workgroups
+// Passes 2 to 4 in one launch, A (nin lines) -> D (nout lines), for boxes with plane_ok; ngrp workgroups (1 to nout)
 // per x-plane.  D may not be A; its box stride is bD.
 struct PlaneTab;
 constexpr int PLANE_MAX = 8192;   // points of a plane

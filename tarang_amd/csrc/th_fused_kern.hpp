@@ -299,8 +299,9 @@ __global__ __launch_bounds__(TZ * P) void k_fz(FG g, const cplx<R>* __restrict__
     // The products in an order that keeps few real lines live; rolled loops, so every operand is a fixed register.
     // Holding all inputs took 256 VGPRs and the accumulation registers (one wave per SIMD, spills in FP64 MHD) on the
     // FP64 and the 3 2^a lines, and two waves in FP32 MHD; now two to five waves and no spill.  z pass, us, before /
-    // after: 192^3 FP64 NS 124 / 85, FP64 MHD 239 / 179, 256^3 FP64 MHD 427 / 287, FP32 MHD 190 / 160, FP32 RB
-    // 136 / 132, 192^3 FP32 NS 62 / 52 (the radix-12 schedules among it); 512^3 FP32 NS 0.68 / 0.69 ms.
+    // after (medians over a run on random fields): 192^3 FP64 NS 122 / 83, FP64 MHD 237 / 177, 256^3 FP64 MHD 430 / 287,
+    // FP32 MHD 193 / 165, FP32 RB 143 / 138, 192^3 FP32 NS 62 / 52 (the radix-12 schedules among it); 2^a NS lines
+    // lose 1 to 2 %: 512^3 FP32 (8 points per thread) 741 / 752, 256^3 FP32 90.4 / 92.6.
     cplx<R> xa[XE], x[E], w[E];
     auto mul = [&](cplx<R> (&o)[E], const cplx<R> (&p)[E], const cplx<R> (&q)[E]) {
 #pragma unroll
@@ -563,8 +564,9 @@ __global__ __launch_bounds__(T * P) __attribute__((amdgpu_waves_per_eu((MODE == 
         }
     };
     // The next product's loads are issued before this one's transform where that costs no wave per SIMD (XPRE): FP32
-    // MHD and FP64 NS with 8 points per thread, chained FP32 NS on the long 3 2^a lines.  us, before / after: 256^3 FP32
-    // MHD 227 / 210, 384^3 FP32 NS 470 / 443, 128^3 FP64 NS 30.2 / 27.8; RB (k_sx_fwd_rb) 256^3 FP32 207 / 165.
+    // MHD and FP64 NS with 8 points per thread, chained FP32 NS on the long 3 2^a lines.  us, before / after (medians on
+    // random fields): 256^3 FP32 MHD 231 / 217, 384^3 FP32 NS 484 / 448 (with its radix 6 lines), 128^3 FP64 NS 28.3 / 26.1;
+    // RB (k_sx_fwd_rb) 256^3 FP32 212 / 174.
     constexpr bool XPRE = sizeof(R) == 4 ? (MODE == 1 && E == 8) || (CHAIN && !FORCED && L % 3 == 0 && L >= 192) : MODE == 0 && E == 8;
     cplx<R> nv[XPRE ? E : 1];
     if constexpr (XPRE) load(0, nv);
@@ -1006,7 +1008,7 @@ __global__ __launch_bounds__(T * P) void k_sx_fwd_rb(FG g, const cplx<R>* __rest
 // (Shell_mult_all) and |K| > kmax_inside (which only Shell_mult_single counts).
 //
 // One component i per workgroup (blockIdx.z): three products each and a third of the accumulators, so that a 128^3
-// box is 1530 workgroups instead of 510 and more of them fit a CU; and the shell search reads each radius once for all
+// FP64 box is 1494 workgroups instead of 498 and more of them fit a CU; and the shell search reads each radius once for all
 // points of a thread.  128^3 FP64 35.7 -> 30.9 us; 15 givers 96^3 FP64 1769 -> 1455 us, 256^3 FP32 7.76 -> 6.89 ms.
 // ------------------------------------------------------------------------------------------
 template <typename R, int L, int P, int T>
@@ -1256,7 +1258,7 @@ static int launch_sxinv(const FG& g, const cplx<R>* S, cplx<R>* A, const cplx<R>
     return OK;
 }
 // variant 1: half-width tiles (more, smaller workgroups; full tiles are the faster ones since the next product's
-// tile is loaded ahead, 165 against 179 us at 256^3 FP32)
+// tile is loaded ahead, 174 against 192 us at 256^3 FP32)
 template <typename R, int L, int V>
 static int launch_sxfwd(const FG& g, const cplx<R>* D, cplx<R>* S, cplx<R>* Vs, cplx<R>* acc, const cplx<R>* tw,
                         const cplx<R>* tw4, const StageCoef* sc, hipStream_t st)

@@ -169,8 +169,8 @@ __global__ __launch_bounds__(L2 * (LZ / plane_EZ(LZ))) void k_plane(FG g, PlaneT
 // CHAIN: the stage outputs go back to LDS and groups 0..NA-1 transform them along x into the next stage's A lines
 // (any radix schedule: the line changes order in LDS).
 //
-// What bounds it: at 64^3 a tile loop of six dependent load-transform rounds ran in 126 one-wave workgroups for 256
-// CUs, 17 us of latency for 5 MB of data.  Here the rounds run at the same time in six times the waves, the state
+// What bounds it: at 64^3 a tile loop of six dependent load-transform rounds ran in 123 one-wave workgroups for 256
+// CUs (FP64), 17 us of latency for 5 MB of data.  Here the rounds run at the same time in six times the waves, the state
 // and accumulator loads are issued before the first transform, and nothing is written non-temporally (the next
 // pass finds its lines in the L2).
 // ------------------------------------------------------------------------------------------
